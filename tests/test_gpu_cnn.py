@@ -245,3 +245,41 @@ def test_compact_training_keeps_pointwise_layer(cuda):
     capi.check(capi.lib().pbrt_cnn_is_compact(net.h, C.byref(flag)))
     assert flag.value == 1
     net.close()
+
+
+@pytest.mark.parametrize("w,h,count", [(256, 160, 4), (250, 150, 4), (16, 16, 4), (5, 3, 2)])
+def test_batch_gradient_is_the_mean_of_its_images(cuda, w, h, count):
+    """A batch's loss and gradient are the means of its images' own.  `count` is a power of
+    two, so the batch's 1/n scales every bf16 gradient exactly and only the FP32 sums
+    differ: over 640 tiles, more than one tile per workgroup, against 160 workgroups of
+    one; down to a single partial tile.  FP32 sums of t terms differ by at most t 2^-24 of
+    their absolute terms' sum, ~1e-5 in the norm here."""
+    rng = np.random.default_rng(w)
+    inp = dict(
+        noisy=half(rng.gamma(1.0, 0.5, (count, h, w, 4))),
+        depth=rng.uniform(0.5, 20.0, (count, h, w)).astype(np.float32),
+        normal=rng.uniform(0, np.pi, (count, h, w, 2)).astype(np.float32),
+        albedo=rng.integers(0, 256, (count, h, w, 4), dtype=np.uint8),
+        spp=rng.integers(0, 40, (count, h, w), dtype=np.uint8),
+        motion=half(rng.uniform(-1, 1, (count, h, w, 2))),
+        target=rng.uniform(0.05, 1.5, (count, h, w, 4)).astype(np.float32),
+    )
+    net = Net(3, 3)
+    n = cnn.parameter_count(cnn.shape_of(3))
+
+    def gradient(sel):
+        part = {k: v[sel] for k, v in inp.items()}
+        im, t = device_images(cuda, part, True, w, h, len(part["depth"]))
+        grad = cuda.zeros(n, dtype=cuda.float32, device="cuda")
+        loss = cuda.zeros(1, dtype=cuda.float32, device="cuda")
+        capi.check(capi.lib().pbrt_cnn_gradients(net.h, C.byref(im), capi.ptr(loss), capi.ptr(grad),
+                                                 helpers.stream(cuda)))
+        cuda.cuda.synchronize()
+        return loss.item(), grad.cpu().numpy().astype(np.float64)
+
+    loss, grad = gradient(slice(0, count))
+    parts = [gradient(slice(k, k + 1)) for k in range(count)]
+    assert abs(loss - np.mean([p[0] for p in parts])) <= 1e-5 * loss
+    mean = np.mean([p[1] for p in parts], axis=0)
+    assert np.linalg.norm(grad - mean) <= 1e-5 * np.linalg.norm(mean)
+    net.close()

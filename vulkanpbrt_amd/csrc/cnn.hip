@@ -19,7 +19,7 @@
 // k_conv3x3_wgrad per tile: dZ^T (channel-major) and three x-shifted,
 //                 channel-major copies of the input halo in LDS; every tap's
 //                 32 x cin weight gradient is a GEMM over the tile's 256 pixels;
-//                 per-tile partials are summed in a fixed order by k_reduce.
+//                 per-workgroup partials are summed in a fixed order by k_reduce_partials.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -406,94 +406,181 @@ __global__ void __launch_bounds__(256) k_conv3x3(CnnGeom g, const uint16_t* __re
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient: per-tile partial dW[tap][cout][cin] and db[cout]
+// Weight gradient: partial dW[tap][cout][cin] and db[cout] per workgroup
 // ---------------------------------------------------------------------------
+// A workgroup takes tiles b, b + gridDim.x, ... and keeps its share of the 9 x 2 x
+// CIN/16 result blocks in the MFMA accumulators across them, so it writes one partial
+// however many tiles it ran.  The operands are read as 16 bytes per lane, sixteen
+// channels side by side: the channel strides are padded so that sixteen such reads
+// fall in distinct LDS banks (264 and 296 bf16; at 256 and 288 they met in one bank
+// and in four).  The bias sums take eight lanes per channel instead of one lane
+// walking 256 pixels.  With the reductions below, a batch of 8 images of 128x128 through
+// six layers (loss and gradients) went from 948 to 218 us.
+constexpr int kDzStride = kTile * kTile + 8;          // bf16 per output channel
+constexpr int kXsStride = (kTile + 2) * kTile + 8;    // bf16 per shifted input channel
+constexpr int kWgradGrid = 512;  // workgroups of the weight gradient: two per CU (74 KB of LDS each)
+
 template <int CIN>
-__global__ void __launch_bounds__(256) k_conv3x3_wgrad(CnnGeom g, const uint16_t* __restrict__ dsrc,
+__global__ void __launch_bounds__(256) k_conv3x3_wgrad(CnnGeom g, int ntiles, const uint16_t* __restrict__ dsrc,
                                                        const uint16_t* __restrict__ mask,
                                                        const uint16_t* __restrict__ in, float* __restrict__ partial) {
     constexpr int kPart = kTaps * kCh * CIN + kCh;
-    __shared__ __attribute__((aligned(16))) uint16_t dz[kCh][256];              // [cout][pixel]
-    __shared__ __attribute__((aligned(16))) uint16_t xs[3][CIN][18][kTile];     // [dx][cin][row][col]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int x0 = blockIdx.x * kTile, y0 = blockIdx.y * kTile, img = blockIdx.z;
-    const size_t plane = (size_t)g.width * g.height;
-    {
-        // upstream gradient of this tile, masked by the ReLU, transposed to channel-major
-        const int p = tid;  // one pixel per thread
-        const int gy = y0 + p / kTile, gx = x0 + p % kTile;
-        const bool inside = gx < g.width && gy < g.height;
-        const size_t off = (plane * img + (size_t)gy * g.width + gx) * kCh;
-#pragma unroll
-        for (int c = 0; c < kCh / 8; ++c) {
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (inside) {
-                v = *reinterpret_cast<const uint4*>(dsrc + off + c * 8);
-                if (mask) v = relu_mask8(v, *reinterpret_cast<const uint4*>(mask + off + c * 8));
-            }
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                dz[c * 8 + 2 * k][p] = (uint16_t)(w[k] & 0xFFFFu);
-                dz[c * 8 + 2 * k + 1][p] = (uint16_t)(w[k] >> 16);
-            }
-        }
-    }
-    for (int e = tid; e < 3 * 18 * kTile; e += 256) {
-        const int dx = e / (18 * kTile), rem = e % (18 * kTile);
-        const int row = rem / kTile, col = rem % kTile;
-        const int gy = y0 + row - 1, gx = x0 + col + dx - 1;
-        const bool inside = gx >= 0 && gy >= 0 && gx < g.width && gy < g.height;
-        const uint16_t* s = in + (plane * img + (size_t)gy * g.width + gx) * CIN;
-#pragma unroll
-        for (int c = 0; c < CIN / 8; ++c) {
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (inside) v = *reinterpret_cast<const uint4*>(s + c * 8);
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                xs[dx][c * 8 + 2 * k][row][col] = (uint16_t)(w[k] & 0xFFFFu);
-                xs[dx][c * 8 + 2 * k + 1][row][col] = (uint16_t)(w[k] >> 16);
-            }
-        }
-    }
-    __syncthreads();
-    float* part = partial + (((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * kPart;
-    const int j = lane & 15, grp = lane >> 4;
     constexpr int kCiTiles = CIN / 16;
     constexpr int kCombos = kTaps * 2 * kCiTiles;
-    for (int cb = wave; cb < kCombos; cb += 4) {
-        const int t = cb / (2 * kCiTiles), rest = cb % (2 * kCiTiles);
-        const int ct = rest / kCiTiles, it = rest % kCiTiles;
-        const int dy = t / 3, dx = t % 3;
-        float4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    constexpr int kOwn = (kCombos + 3) / 4;  // result blocks of a wave
+    __shared__ __attribute__((aligned(16))) uint16_t dz[kCh * kDzStride];       // [cout][pixel]
+    __shared__ __attribute__((aligned(16))) uint16_t xs[3 * CIN * kXsStride];   // [dx][cin][row][col]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int j = lane & 15, grp = lane >> 4;
+    const int tiles_x = (g.width + kTile - 1) / kTile, tiles_y = (g.height + kTile - 1) / kTile;
+    const size_t plane = (size_t)g.width * g.height;
+    float4v acc[kOwn];
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            const int p0 = ks * 32 + 8 * grp;  // eight pixels of one row
-            const int row = p0 / kTile, col = p0 % kTile;
-            const bf16x8 a = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&dz[ct * 16 + j][p0]));
-            const bf16x8 b =
-                __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&xs[dx][it * 16 + j][row + dy][col]));
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+    for (int k = 0; k < kOwn; ++k) acc[k] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+    float bias = 0.0f;  // lanes 8c .. 8c + 7 of the workgroup: channel c, 32 pixels each
+    for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+        const int img = t / (tiles_x * tiles_y), rem = t % (tiles_x * tiles_y);
+        const int x0 = (rem % tiles_x) * kTile, y0 = (rem / tiles_x) * kTile;
+        if (t != (int)blockIdx.x) __syncthreads();  // the previous tile has been read
+        {
+            // upstream gradient of this tile, masked by the ReLU, transposed to channel-major
+            const int p = tid;  // one pixel per thread
+            const int gy = y0 + p / kTile, gx = x0 + p % kTile;
+            const bool inside = gx < g.width && gy < g.height;
+            const size_t off = (plane * img + (size_t)gy * g.width + gx) * kCh;
+#pragma unroll
+            for (int c = 0; c < kCh / 8; ++c) {
+                uint4 v = make_uint4(0, 0, 0, 0);
+                if (inside) {
+                    v = *reinterpret_cast<const uint4*>(dsrc + off + c * 8);
+                    if (mask) v = relu_mask8(v, *reinterpret_cast<const uint4*>(mask + off + c * 8));
+                }
+                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    dz[(c * 8 + 2 * k) * kDzStride + p] = (uint16_t)(w[k] & 0xFFFFu);
+                    dz[(c * 8 + 2 * k + 1) * kDzStride + p] = (uint16_t)(w[k] >> 16);
+                }
+            }
         }
-        // D[cout][cin]: lane holds cin it*16 + j, couts ct*16 + 4*grp + i
+        for (int e = tid; e < 3 * 18 * kTile; e += 256) {
+            const int dx = e / (18 * kTile), at = e % (18 * kTile);
+            const int row = at / kTile, col = at % kTile;
+            const int gy = y0 + row - 1, gx = x0 + col + dx - 1;
+            const bool inside = gx >= 0 && gy >= 0 && gx < g.width && gy < g.height;
+            const uint16_t* s = in + (plane * img + (size_t)gy * g.width + gx) * CIN;
+            uint16_t* d = xs + dx * CIN * kXsStride + at;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) part[(t * kCh + ct * 16 + 4 * grp + i) * CIN + it * 16 + j] = acc[i];
+            for (int c = 0; c < CIN / 8; ++c) {
+                uint4 v = make_uint4(0, 0, 0, 0);
+                if (inside) v = *reinterpret_cast<const uint4*>(s + c * 8);
+                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    d[(c * 8 + 2 * k) * kXsStride] = (uint16_t)(w[k] & 0xFFFFu);
+                    d[(c * 8 + 2 * k + 1) * kXsStride] = (uint16_t)(w[k] >> 16);
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kOwn; ++k) {
+            const int cb = wave + 4 * k;
+            if (cb < kCombos) {
+                const int tp = cb / (2 * kCiTiles), rest = cb % (2 * kCiTiles);
+                const int ct = rest / kCiTiles, it = rest % kCiTiles;
+                const int dy = tp / 3, dx = tp % 3;
+                const uint16_t* da = dz + (ct * 16 + j) * kDzStride;
+                const uint16_t* xb = xs + (dx * CIN + it * 16 + j) * kXsStride + dy * kTile;
+#pragma unroll
+                for (int ks = 0; ks < 8; ++ks) {
+                    const int p0 = ks * 32 + 8 * grp;  // eight pixels of one row
+                    const bf16x8 a = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(da + p0));
+                    const bf16x8 b = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(xb + p0));
+                    acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[k], 0, 0, 0);
+                }
+            }
+        }
+        {
+            const uint4* src = reinterpret_cast<const uint4*>(dz + (tid >> 3) * kDzStride + (tid & 7) * 32);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint4 v = src[q];
+                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) bias += bf2f(w[k] & 0xFFFFu) + bf2f(w[k] >> 16);
+            }
+        }
     }
-    if (tid < kCh) {
-        float s = 0.0f;
-        for (int p = 0; p < 256; ++p) s += bf2f(dz[tid][p]);
-        part[kTaps * kCh * CIN + tid] = s;
+    float* part = partial + (size_t)blockIdx.x * kPart;
+#pragma unroll
+    for (int k = 0; k < kOwn; ++k) {
+        const int cb = wave + 4 * k;
+        if (cb < kCombos) {
+            const int tp = cb / (2 * kCiTiles), rest = cb % (2 * kCiTiles);
+            const int ct = rest / kCiTiles, it = rest % kCiTiles;
+            // D[cout][cin]: lane holds cin it*16 + j, couts ct*16 + 4*grp + i
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                part[(tp * kCh + ct * 16 + 4 * grp + i) * CIN + it * 16 + j] = acc[k][i];
+        }
     }
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1) bias += __shfl_xor(bias, off);
+    if ((tid & 7) == 0) part[kTaps * kCh * CIN + (tid >> 3)] = bias;
 }
 
-// grad[i] = sum over tiles of partial[tile][i], in tile order
-__global__ void __launch_bounds__(256) k_reduce_partials(const float* partial, int tiles, int size, float* grad) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= size) return;
-    float s = 0.0f;
-    for (int t = 0; t < tiles; ++t) s += partial[(size_t)t * size + i];
-    grad[i] = s;
+// grad[i] = sum over the partials' rows of partial[row][i], and in the last workgroup
+// the batch loss (when asked for).  Eight lanes cover 128 contiguous bytes of a row and
+// a workgroup's 32 lane groups take the rows r, r + 32, ..., folded through LDS in a
+// fixed order: 289 workgroups of independent 16-byte loads.  One thread per column
+// summing 512 rows one after the other left 37 workgroups waiting on memory (120 us a
+// layer at 512 rows of 9248 floats).
+constexpr int kReduceCols = 8, kReduceRows = 32;  // float4 columns x row groups of a workgroup
+
+__global__ void __launch_bounds__(kReduceCols* kReduceRows)
+k_reduce_partials(const float* __restrict__ partial, int rows, int size, float* __restrict__ grad,
+                  const float* __restrict__ loss_part, int loss_blocks, float loss_scale, float* loss) {
+    __shared__ float4 fold[kReduceRows][kReduceCols];
+    const int tid = threadIdx.x, c = tid % kReduceCols, r0 = tid / kReduceCols;
+    const int cols = size / 4, blocks = (cols + kReduceCols - 1) / kReduceCols;
+    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if ((int)blockIdx.x == blocks) {  // the loss: uniform over the workgroup
+        for (int b = tid; b < loss_blocks; b += kReduceCols * kReduceRows) s.x += loss_part[b];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) s.x += __shfl_xor(s.x, off);
+    } else {
+        const int col = blockIdx.x * kReduceCols + c;
+        if (col < cols) {
+            const float4* p = reinterpret_cast<const float4*>(partial) + col;
+#pragma unroll 8
+            for (int r = r0; r < rows; r += kReduceRows) {
+                const float4 v = p[(size_t)r * cols];
+                s.x += v.x;
+                s.y += v.y;
+                s.z += v.z;
+                s.w += v.w;
+            }
+        }
+    }
+    fold[r0][c] = s;
+    __syncthreads();
+    if ((int)blockIdx.x == blocks) {
+        constexpr int step = 64 / kReduceCols;  // rows of `fold` a wave wrote
+        if (tid == 0) *loss = (fold[0][0].x + fold[step][0].x + fold[2 * step][0].x + fold[3 * step][0].x) * loss_scale;
+        return;
+    }
+    // column c of each float4 component: one thread per float, rows in order
+    if (tid < 4 * kReduceCols) {
+        const int i = blockIdx.x * kReduceCols * 4 + tid;
+        if (i < size) {
+            const float* f = reinterpret_cast<const float*>(&fold[0][0]) + tid;
+            float t = 0.0f;
+#pragma unroll
+            for (int r = 0; r < kReduceRows; ++r) t += f[r * kReduceCols * 4];
+            grad[i] = t;
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -582,13 +669,6 @@ __global__ void __launch_bounds__(256) k_kpn(CnnGeom g, pbrt_cnn_images im, cons
         __syncthreads();
         if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
     }
-}
-
-__global__ void k_loss_total(const float* part, int blocks, float scale, float* loss) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    float s = 0.0f;
-    for (int b = 0; b < blocks; ++b) s += part[b];
-    *loss = s * scale;
 }
 
 // ---------------------------------------------------------------------------
@@ -1209,9 +1289,9 @@ void backward(const pbrt_cnn* net, const pbrt_cnn_images& im, const CnnWork& k, 
     const int layers = net->layers;
     hipLaunchKernelGGL(k_kpn<true>, dim3(blocks), dim3(256), 0, st, g, im, k.act[layers], k.grad_act[0],
                        k.loss_part);
-    if (loss) hipLaunchKernelGGL(k_loss_total, dim3(1), dim3(64), 0, st, k.loss_part, blocks, 1.0f / (float)(px * 3), loss);
-    const dim3 grid((im.width + kTile - 1) / kTile, (im.height + kTile - 1) / kTile, im.count);
-    const int tiles = (int)(grid.x * grid.y * grid.z);
+    const int tiles = (int)(((im.width + kTile - 1) / kTile) * ((im.height + kTile - 1) / kTile) * im.count);
+    const int rows = std::min(tiles, kWgradGrid);
+    const dim3 grid(rows);
     const uint16_t* wb = net->wb.as<uint16_t>();
     int cur = 0;  // grad_act[cur] holds dA of layer l+1 (dLogits for the last layer)
     for (int l = layers - 1; l >= 0; --l) {
@@ -1219,11 +1299,17 @@ void backward(const pbrt_cnn* net, const pbrt_cnn_images& im, const CnnWork& k, 
         const uint16_t* mask = l == layers - 1 ? nullptr : k.act[l + 1];
         const int size = layer_size(l);
         if (l == 0)
-            hipLaunchKernelGGL(k_conv3x3_wgrad<kFeatCh>, grid, dim3(256), 0, st, g, dsrc, mask, k.act[0], k.partial);
+            hipLaunchKernelGGL(k_conv3x3_wgrad<kFeatCh>, grid, dim3(256), 0, st, g, tiles, dsrc, mask, k.act[0],
+                               k.partial);
         else
-            hipLaunchKernelGGL(k_conv3x3_wgrad<kCh>, grid, dim3(256), 0, st, g, dsrc, mask, k.act[l], k.partial);
-        hipLaunchKernelGGL(k_reduce_partials, dim3((size + 255) / 256), dim3(256), 0, st, k.partial, tiles, size,
-                           k.grad + layer_offset(l));
+            hipLaunchKernelGGL(k_conv3x3_wgrad<kCh>, grid, dim3(256), 0, st, g, tiles, dsrc, mask, k.act[l],
+                               k.partial);
+        // the last layer's reduction also totals the loss, in one more workgroup
+        const int cols = size / 4, sum_blocks = (cols + kReduceCols - 1) / kReduceCols;
+        const bool with_loss = loss && l == layers - 1;
+        hipLaunchKernelGGL(k_reduce_partials, dim3(sum_blocks + (with_loss ? 1 : 0)),
+                           dim3(kReduceCols * kReduceRows), 0, st, k.partial, rows, size, k.grad + layer_offset(l),
+                           k.loss_part, blocks, 1.0f / (float)(px * 3), loss);
         if (l > 0) {
             launch_conv<kCh, kConvDgrad>(g, dsrc, mask, wb + weight_offset(l), nullptr, k.grad_act[cur ^ 1], st);
             cur ^= 1;
