@@ -11,11 +11,10 @@
 // reprojected previous output and remodulates (bfr.comp:202-308).
 //
 // The reference runs one b x b workgroup per block (up to 1024 threads) with two
-// barriers per Adam step.  Here a block is 64 (b = 8) or 256 threads holding
-// b*b/threads pixels each; a step reduces the 21 gradient sums inside each wave
-// (xor butterfly), folds the waves through a double-buffered LDS slot behind one
-// barrier, and every thread then applies the same Adam update to its own copy of
-// alpha, m and v, so no second barrier or broadcast is needed.
+// barriers per Adam step.  Here a 16- or 8-pixel block is one wave and a 32-pixel block
+// four: a step forms the 21 gradient sums of each 64-pixel group with lane swaps (two
+// sums share a register at xor 32, four at xor 16), lane j of the wave then runs
+// Adam for component j alone and the 21 new weights go to scalar registers.
 //
 // Project rules where bfr.comp depends on the hardware:
 //   * the stop test `gradient_rest >= GRADIENT_THRESH (0)` is reduced over all 7
@@ -51,11 +50,6 @@ struct BfrGeom {
     uint32_t frame;
 };
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
 __device__ __forceinline__ float wave_min(float v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v = fminf(v, __shfl_xor(v, off));
@@ -71,14 +65,61 @@ __device__ __forceinline__ float sign_of(float x) { return x > 0.0f ? 1.0f : (x 
 
 }  // namespace
 
-// kB: block edge; kThreads: 64 or 256; each thread owns kB*kB/kThreads pixels,
-// pixel r = tid + p * kThreads at local (r / kB, r % kB) (bfr.comp's ID order).
-template <int kB, int kThreads>
-__global__ void __launch_bounds__(kThreads) k_bfr(BfrGeom g, pbrt_bfr_images im) {
-    constexpr int kPix = kB * kB / kThreads;
-    constexpr int kWaves = kThreads / 64;
-    __shared__ float part[2][kWaves][kBfrSums];
-    __shared__ float red[2][kWaves];
+// The step loop is VALU-bound: per 64 pixels 21 multiply-adds of prediction, 21 of
+// gradient and the signs, and then the 21 sums.  What it spends beside them is kept off
+// the vector unit's redundant lanes:
+//   * the sums: v_permlane32_swap / v_permlane16_swap exchange half a register with
+//     another sum's, so xor 32 and 16 cost one swap and one add per two sums (plain
+//     butterflies through the LDS pipe: two operations per sum and step, 126 per wave
+//     and iteration in all), and xor 8 and 4 are row rotations (DPP);
+//   * Adam once per component in lane j instead of all 21 components in every lane (a
+//     correctly rounded square root and division each), its learning-rate factors from
+//     a table made once per block, lane t holding step t;
+//   * the new weights by v_readlane into scalar registers, which the multiply-adds read.
+// A sum is the same binary tree over the same pixels as a butterfly from xor 32 to xor 1
+// followed by the 64-pixel groups in order, so the steps' signs do not change with the
+// mapping.  One wave per 16-pixel block (four groups a lane) needs no barrier and runs
+// the sums' rows, Adam and the broadcast once instead of four times; a 32-pixel block's
+// 16 pixels per lane would leave two waves per SIMD, so it takes four waves and one
+// barrier a step.  At 1920x1080: 16-pixel blocks 2402 -> 357 us, 8-pixel 2335 -> 444 us,
+// 32-pixel 835 -> 246 us.
+constexpr int kSumSlots = 24;  // 21 gradient components, padded
+
+__device__ __forceinline__ float swap_add32(float a, float b) {
+    // lanes 0..31: a[l] + a[l ^ 32]; lanes 32..63: b[l] + b[l ^ 32]
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float swap_add16(float a, float b) {
+    // rows 0, 2: a[l] + a[l ^ 16]; rows 1, 3: b[l] + b[l ^ 16]
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+template <int kCtrl>
+__device__ __forceinline__ float dpp_add(float v) {
+    return v + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), kCtrl, 0xF, 0xF, true));
+}
+// four sums by row: row r of the result holds sum r's xor-32 and xor-16 steps
+__device__ __forceinline__ float rows_of(float s0, float s1, float s2, float s3) {
+    return swap_add16(swap_add32(s0, s2), swap_add32(s1, s3));
+}
+// the xor-8 and xor-4 steps: each lane adds its row's lane l ^ 8, then (the row being
+// 8-periodic) the one four further, which holds the value of l ^ 4
+__device__ __forceinline__ float row_steps84(float v) { return dpp_add<0x124>(dpp_add<0x128>(v)); }  // row_ror 8, 4
+__device__ __forceinline__ float quad_steps21(float v) { return dpp_add<0xB1>(dpp_add<0x4E>(v)); }  // quad_perm
+
+// kB: block edge; kW waves per block; a lane owns kP pixels of each of kV groups of 64:
+// pixel r = (wave * kV + group) * 64 + lane + p * 64 kW kV at local (r / kB, r % kB)
+// (bfr.comp's ID order).
+template <int kB, int kW, int kV, int kP>
+__global__ void __launch_bounds__(64 * kW) k_bfr(BfrGeom g, pbrt_bfr_images im) {
+    constexpr int kPix = kV * kP;
+    static_assert(64 * kW * kPix == kB * kB, "the lanes' pixels are the block's");
+    static_assert(kW == 1 || kV == 1, "a sum has four parts at most");
+    constexpr int kParts = kW * kV;  // 64-lane partial sums per component: 1 or 4
+    static_assert(kParts == 1 || kParts == 4, "parts are read as one or four floats");
+    __shared__ __attribute__((aligned(16))) float part[kW > 1 ? 2 : 1][kSumSlots * kParts];
+    __shared__ float red[3][kW];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
     vec3 color[kPix];
@@ -88,10 +129,10 @@ __global__ void __launch_bounds__(kThreads) k_bfr(BfrGeom g, pbrt_bfr_images im)
     bool inside[kPix];
     float depth[kPix];
     float dmin = 3.4e38f, dmax = -3.4e38f;
-    int l1_local = 0;
+    int l1_count = 0;
 #pragma unroll
     for (int p = 0; p < kPix; ++p) {
-        const int r = tid + p * kThreads;
+        const int r = (wave * kV + p / kP) * 64 + lane + (p % kP) * 64 * kParts;
         const int lx = r / kB, ly = r % kB;
         const int ax = blockIdx.x * kB + lx + g.offx, ay = blockIdx.y * kB + ly + g.offy;
         img_x[p] = mirror_coord(ax, g.width);
@@ -104,7 +145,7 @@ __global__ void __launch_bounds__(kThreads) k_bfr(BfrGeom g, pbrt_bfr_images im)
         const vec3 nn = decode_normal(n.x, n.y);
         const float spp = unorm8_to_float(im.spp[pix]) * 256.0f;
         l1px[p] = spp >= kSppThreshold;
-        l1_local += l1px[p] ? 1 : 0;
+        l1_count += __popcll(__ballot(l1px[p]));
         dmin = fminf(dmin, depth[p]);
         dmax = fmaxf(dmax, depth[p]);
         feat[p][0] = 1.0f;
@@ -117,24 +158,23 @@ __global__ void __launch_bounds__(kThreads) k_bfr(BfrGeom g, pbrt_bfr_images im)
     // block min / max depth and the count of pixels in the L1 regime
     dmin = wave_min(dmin);
     dmax = wave_max(dmax);
-    float l1f = wave_sum((float)l1_local);
-    if (kWaves > 1) {
+    float l1f = (float)l1_count;
+    if (kW > 1) {
         if (lane == 0) {
             red[0][wave] = dmin;
             red[1][wave] = dmax;
-            part[1][wave][0] = l1f;
+            red[2][wave] = l1f;
         }
         __syncthreads();
         dmin = red[0][0];
         dmax = red[1][0];
-        l1f = part[1][0][0];
+        l1f = red[2][0];
 #pragma unroll
-        for (int w = 1; w < kWaves; ++w) {
+        for (int w = 1; w < kW; ++w) {
             dmin = fminf(dmin, red[0][w]);
             dmax = fmaxf(dmax, red[1][w]);
-            l1f += part[1][w][0];
+            l1f += red[2][w];
         }
-        __syncthreads();
     }
 #pragma unroll
     for (int p = 0; p < kPix; ++p) {
@@ -146,69 +186,105 @@ __global__ void __launch_bounds__(kThreads) k_bfr(BfrGeom g, pbrt_bfr_images im)
     const float a_mix = l1_ratio * kAlphaL + (1.0f - l1_ratio) * kAlpha;
     const float b1_mix = l1_ratio * kBeta1L + (1.0f - l1_ratio) * kBeta1;
     const float b2_mix = l1_ratio * kBeta2L + (1.0f - l1_ratio) * kBeta2;
+    // exponential learning-rate decay and bias correction (bfr.comp:124-131) of step
+    // t = lane + 1
+    const float t_lane = (float)(lane + 1);
+    const float step_lane =
+        a_mix * expf(-kK * t_lane) * sqrtf(1.0f - powf(kBeta2, t_lane)) / (1.0f - powf(kBeta1, t_lane));
 
-    float alpha[kBfrSums], m[kBfrSums], v[kBfrSums];
+    // lane j: component j of alpha and of Adam's moments; aw: alpha on every lane
+    float alpha_lane = 0.0f, m = 0.0f, v = 0.0f;
+    float aw[kBfrSums];
 #pragma unroll
-    for (int j = 0; j < kBfrSums; ++j) alpha[j] = m[j] = v[j] = 0.0f;
+    for (int j = 0; j < kBfrSums; ++j) aw[j] = 0.0f;
 
+    const int row = lane >> 4, bank = (lane >> 2) & 3, quad = lane & 3;
     for (int it = 0; it < kBfrIterations; ++it) {
-        float grad[kBfrSums];
+        float grad[kV][kBfrSums];
 #pragma unroll
-        for (int j = 0; j < kBfrSums; ++j) grad[j] = 0.0f;
+        for (int w = 0; w < kV; ++w)
+#pragma unroll
+            for (int j = 0; j < kBfrSums; ++j) grad[w][j] = 0.0f;
 #pragma unroll
         for (int p = 0; p < kPix; ++p) {
             vec3 pred = make_vec3(0.0f);
 #pragma unroll
             for (int j = 0; j < kBfrFeatures; ++j)
-                pred += make_vec3(alpha[3 * j], alpha[3 * j + 1], alpha[3 * j + 2]) * feat[p][j];
+                pred += make_vec3(aw[3 * j], aw[3 * j + 1], aw[3 * j + 2]) * feat[p][j];
             vec3 d = color[p] - pred;
             if (l1px[p]) d = make_vec3(sign_of(d.x), sign_of(d.y), sign_of(d.z));
+            float* gw = grad[p / kP];
 #pragma unroll
             for (int j = 0; j < kBfrFeatures; ++j) {
-                grad[3 * j] += feat[p][j] * d.x;
-                grad[3 * j + 1] += feat[p][j] * d.y;
-                grad[3 * j + 2] += feat[p][j] * d.z;
+                gw[3 * j] += feat[p][j] * d.x;
+                gw[3 * j + 1] += feat[p][j] * d.y;
+                gw[3 * j + 2] += feat[p][j] * d.z;
             }
         }
+        float* slot = part[kW > 1 ? (it & 1) : 0];
+        if constexpr (kV == 4) {
+            // row r: group r's part of a component; four components by lane quartet (bank),
+            // four such registers by lane within the quartet
+            float q[kSumSlots / 4];
 #pragma unroll
-        for (int j = 0; j < kBfrSums; ++j) grad[j] = wave_sum(grad[j]);
-        if (kWaves > 1) {
-            const int buf = it & 1;
-            if (lane == 0) {
+            for (int f = 0; f < kSumSlots / 4; ++f) {
+                float s[4];
 #pragma unroll
-                for (int j = 0; j < kBfrSums; ++j) part[buf][wave][j] = grad[j];
+                for (int b = 0; b < 4; ++b) {
+                    const int j = 4 * f + b;
+                    s[b] = 0.0f;
+                    if (j < kBfrSums) s[b] = row_steps84(rows_of(grad[0][j], grad[1][j], grad[2][j], grad[3][j]));
+                }
+                const float lo = (bank & 1) ? s[1] : s[0], hi = (bank & 1) ? s[3] : s[2];
+                q[f] = quad_steps21((bank & 2) ? hi : lo);
             }
+            const float lo = (quad & 1) ? q[1] : q[0], hi = (quad & 1) ? q[3] : q[2];
+            slot[(4 * quad + bank) * 4 + row] = (quad & 2) ? hi : lo;
+            if (quad < 2) slot[(16 + 4 * quad + bank) * 4 + row] = quad ? q[5] : q[4];
+        } else {
+            // row r: component 4 k + r of register k, the lane's by its quartet
+            float q[kSumSlots / 4];
+#pragma unroll
+            for (int k = 0; k < kSumSlots / 4; ++k) {
+                float s[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[r] = 4 * k + r < kBfrSums ? grad[0][4 * k + r] : 0.0f;
+                q[k] = row_steps84(rows_of(s[0], s[1], s[2], s[3]));
+            }
+            const float lo = (bank & 1) ? q[1] : q[0], hi = (bank & 1) ? q[3] : q[2];
+            const float a = quad_steps21((bank & 2) ? hi : lo);
+            const float b = quad_steps21((bank & 1) ? q[5] : q[4]);
+            if (quad == 0) {
+                slot[(4 * bank + row) * kParts + wave] = a;
+                if (bank < 2) slot[(16 + 4 * bank + row) * kParts + wave] = b;
+            }
+        }
+        if (kW > 1)
             __syncthreads();
-#pragma unroll
-            for (int j = 0; j < kBfrSums; ++j) {
-                float s = part[buf][0][j];
-#pragma unroll
-                for (int w = 1; w < kWaves; ++w) s += part[buf][w][j];
-                grad[j] = s;
+        else
+            __builtin_amdgcn_wave_barrier();  // LDS operations of one wave complete in order
+        float gj = 0.0f;
+        if (lane < kBfrSums) {
+            if constexpr (kParts == 4) {
+                const float4 s = *reinterpret_cast<const float4*>(slot + 4 * lane);
+                gj = s.x + s.y + s.z + s.w;
+            } else {
+                gj = slot[lane];
             }
         }
-        // Adam with exponential learning-rate decay (bfr.comp:124-131), t = it + 1
-        const float t = (float)(it + 1);
-        const float step =
-            a_mix * expf(-kK * t) * sqrtf(1.0f - powf(kBeta2, t)) / (1.0f - powf(kBeta1, t));
-        float rest = 0.0f;
-#pragma unroll
-        for (int j = 0; j < kBfrSums; ++j) {
-            const float dl = grad[j];
-            m[j] = b1_mix * m[j] + (1.0f - kBeta1) * dl;
-            v[j] = b2_mix * v[j] + (1.0f - kBeta2) * (dl * dl);
-            alpha[j] += step * (m[j] / (sqrtf(v[j]) + kEps));
-            rest += fabsf(dl);
-        }
-        if (!(rest >= 0.0f)) break;  // NaN gradient (GRADIENT_THRESH = 0)
-    }
-
-    if (im.weights && tid < kBfrSums) {
-        float* out = im.weights + ((size_t)blockIdx.y * g.blocks_x + blockIdx.x) * kBfrSums;
+        __builtin_amdgcn_wave_barrier();
+        const float step = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(step_lane), it));
+        m = b1_mix * m + (1.0f - kBeta1) * gj;
+        v = b2_mix * v + (1.0f - kBeta2) * (gj * gj);
+        alpha_lane += step * (m / (sqrtf(v) + kEps));
 #pragma unroll
         for (int j = 0; j < kBfrSums; ++j)
-            if (tid == j) out[j] = alpha[j];
+            aw[j] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(alpha_lane), j));
+        if (__any(gj != gj)) break;  // NaN gradient (GRADIENT_THRESH = 0)
     }
+
+    if (im.weights && tid < kBfrSums)
+        im.weights[((size_t)blockIdx.y * g.blocks_x + blockIdx.x) * kBfrSums + tid] = alpha_lane;
 
     const size_t plane = (size_t)g.width * g.height;
 #pragma unroll
@@ -218,7 +294,7 @@ __global__ void __launch_bounds__(kThreads) k_bfr(BfrGeom g, pbrt_bfr_images im)
         vec3 den = make_vec3(0.0f);
 #pragma unroll
         for (int j = 0; j < kBfrFeatures; ++j)
-            den += make_vec3(alpha[3 * j], alpha[3 * j + 1], alpha[3 * j + 2]) * feat[p][j];
+            den += make_vec3(aw[3 * j], aw[3 * j + 1], aw[3 * j + 2]) * feat[p][j];
         den = vclamp(den, 0.0f, 10.0f);
         const ushort2 mv = reinterpret_cast<const ushort2*>(im.motion)[pix];
         const float mux = h2f(mv.x), muy = h2f(mv.y);
@@ -311,11 +387,11 @@ extern "C" int32_t pbrt_bfr(const pbrt_bfr_params* p, const pbrt_bfr_images* im,
         const dim3 grid(g.blocks_x, g.blocks_y);
         hipStream_t st = (hipStream_t)stream;
         if (g.bs == 8)
-            hipLaunchKernelGGL((k_bfr<8, 64>), grid, dim3(64), 0, st, g, *im);
+            hipLaunchKernelGGL((k_bfr<8, 1, 1, 1>), grid, dim3(64), 0, st, g, *im);
         else if (g.bs == 16)
-            hipLaunchKernelGGL((k_bfr<16, 256>), grid, dim3(256), 0, st, g, *im);
+            hipLaunchKernelGGL((k_bfr<16, 1, 4, 1>), grid, dim3(64), 0, st, g, *im);
         else
-            hipLaunchKernelGGL((k_bfr<32, 256>), grid, dim3(256), 0, st, g, *im);
+            hipLaunchKernelGGL((k_bfr<32, 4, 1, 4>), grid, dim3(256), 0, st, g, *im);
         PBRT_HIP(hipGetLastError());
     });
 }
