@@ -343,3 +343,41 @@ def test_bfr_blend_matches_oracle(cuda, oracle_lib):
         ok = (np.abs(g.astype(int) - o.astype(int)) <= 1).all(-1)
         print(f"blend radius {radius}: agreement {ok.mean():.5f}")
         assert ok.mean() > 0.999
+
+
+@pytest.mark.parametrize("bs", [8, 16, 32])
+@pytest.mark.parametrize("which", ["householder", "gram", "bfr"])
+def test_non_finite_pixels_stay_in_their_block(cuda, oracle_lib, frames, which, bs):
+    """NaN and infinite radiance, depth and normals in a few pixels change nothing further
+    than a block away: the block sums of the fits see only their own block's lanes, and a
+    NaN gradient ends only its own block's steps."""
+    inp = bmfr_inputs(oracle_lib, frames)
+    bad = {k: v.copy() for k, v in inp.items()}
+    spots = [(40, 50), (41, 50), (100, 140), (150, 200)]
+    noisy = bad["noisy"]
+    noisy[40, 50, 0], noisy[41, 50, 1] = 0x7E00, 0x7C00  # NaN, infinity
+    bad["depth"][100, 140] = np.inf
+    bad["normal"][150, 200, 0] = np.nan
+    denoised = half(np.random.default_rng(3).uniform(0, 2, (2, H, W, 4)))
+
+    def run(x):
+        if which != "bfr":
+            fit = capi.BMFR_FIT_HOUSEHOLDER if which == "householder" else capi.BMFR_FIT_GRAM_F64
+            return run_bmfr(cuda, fit, bs, 1, x, denoised)[2:]
+        t = {k: dev(cuda, v) for k, v in x.items()}
+        den, final = dev(cuda, denoised), cuda.zeros((H, W, 4), dtype=cuda.uint8, device="cuda")
+        p = capi.BfrParams(W, H, bs, 1)
+        im = capi.BfrImages(*(capi.ptr(t[k]) for k in ("depth", "normal", "albedo", "motion", "spp", "noisy")),
+                            capi.ptr(den), capi.ptr(final), None)
+        capi.check(capi.lib().pbrt_bfr(C.byref(p), C.byref(im), helpers.stream(cuda)))
+        cuda.cuda.synchronize()
+        return den.cpu().numpy().view(np.uint16), final.cpu().numpy()
+
+    clean, dirty = run(inp), run(bad)
+    ys, xs = np.mgrid[0:H, 0:W]
+    far = np.ones((H, W), bool)
+    for y, x in spots:
+        far &= (np.abs(ys - y) >= bs) | (np.abs(xs - x) >= bs)
+    assert far.mean() > 0.5
+    assert np.array_equal(clean[0][:, far], dirty[0][:, far]) and np.array_equal(clean[1][far], dirty[1][far])
+    assert not np.array_equal(clean[0][0], dirty[0][0])

@@ -26,6 +26,7 @@
 
 #include "capi_common.hpp"
 #include "image_ops.hpp"
+#include "wave_sums.hpp"
 
 namespace pbrt {
 
@@ -84,29 +85,6 @@ __device__ __forceinline__ float sign_of(float x) { return x > 0.0f ? 1.0f : (x 
 // barrier a step.  At 1920x1080: 16-pixel blocks 2402 -> 357 us, 8-pixel 2335 -> 444 us,
 // 32-pixel 835 -> 246 us.
 constexpr int kSumSlots = 24;  // 21 gradient components, padded
-
-__device__ __forceinline__ float swap_add32(float a, float b) {
-    // lanes 0..31: a[l] + a[l ^ 32]; lanes 32..63: b[l] + b[l ^ 32]
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float swap_add16(float a, float b) {
-    // rows 0, 2: a[l] + a[l ^ 16]; rows 1, 3: b[l] + b[l ^ 16]
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-template <int kCtrl>
-__device__ __forceinline__ float dpp_add(float v) {
-    return v + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), kCtrl, 0xF, 0xF, true));
-}
-// four sums by row: row r of the result holds sum r's xor-32 and xor-16 steps
-__device__ __forceinline__ float rows_of(float s0, float s1, float s2, float s3) {
-    return swap_add16(swap_add32(s0, s2), swap_add32(s1, s3));
-}
-// the xor-8 and xor-4 steps: each lane adds its row's lane l ^ 8, then (the row being
-// 8-periodic) the one four further, which holds the value of l ^ 4
-__device__ __forceinline__ float row_steps84(float v) { return dpp_add<0x124>(dpp_add<0x128>(v)); }  // row_ror 8, 4
-__device__ __forceinline__ float quad_steps21(float v) { return dpp_add<0xB1>(dpp_add<0x4E>(v)); }  // quad_perm
 
 // kB: block edge; kW waves per block; a lane owns kP pixels of each of kV groups of 64:
 // pixel r = (wave * kV + group) * 64 + lane + p * 64 kW kV at local (r / kB, r % kB)
@@ -235,11 +213,9 @@ __global__ void __launch_bounds__(64 * kW) k_bfr(BfrGeom g, pbrt_bfr_images im) 
                     s[b] = 0.0f;
                     if (j < kBfrSums) s[b] = row_steps84(rows_of(grad[0][j], grad[1][j], grad[2][j], grad[3][j]));
                 }
-                const float lo = (bank & 1) ? s[1] : s[0], hi = (bank & 1) ? s[3] : s[2];
-                q[f] = quad_steps21((bank & 2) ? hi : lo);
+                q[f] = quad_steps21(by_bank(bank, s[0], s[1], s[2], s[3]));
             }
-            const float lo = (quad & 1) ? q[1] : q[0], hi = (quad & 1) ? q[3] : q[2];
-            slot[(4 * quad + bank) * 4 + row] = (quad & 2) ? hi : lo;
+            slot[(4 * quad + bank) * 4 + row] = by_bank(quad, q[0], q[1], q[2], q[3]);
             if (quad < 2) slot[(16 + 4 * quad + bank) * 4 + row] = quad ? q[5] : q[4];
         } else {
             // row r: component 4 k + r of register k, the lane's by its quartet
@@ -251,8 +227,7 @@ __global__ void __launch_bounds__(64 * kW) k_bfr(BfrGeom g, pbrt_bfr_images im) 
                 for (int r = 0; r < 4; ++r) s[r] = 4 * k + r < kBfrSums ? grad[0][4 * k + r] : 0.0f;
                 q[k] = row_steps84(rows_of(s[0], s[1], s[2], s[3]));
             }
-            const float lo = (bank & 1) ? q[1] : q[0], hi = (bank & 1) ? q[3] : q[2];
-            const float a = quad_steps21((bank & 2) ? hi : lo);
+            const float a = quad_steps21(by_bank(bank, q[0], q[1], q[2], q[3]));
             const float b = quad_steps21((bank & 1) ? q[5] : q[4]);
             if (quad == 0) {
                 slot[(4 * bank + row) * kParts + wave] = a;

@@ -32,6 +32,7 @@
 #include "capi_common.hpp"
 #include "image_ops.hpp"
 #include "pbrt_fn.hpp"
+#include "wave_sums.hpp"
 
 namespace pbrt {
 
@@ -104,32 +105,8 @@ __global__ void __launch_bounds__(256) k_bmfr_noise(uint32_t frame, int bs, int 
 }
 
 // ---------------------------------------------------------------------------
-// Workgroup reductions (wave64 butterfly, then thread 0 folds the waves in order)
+// Wave reductions
 // ---------------------------------------------------------------------------
-template <class T, class Op>
-__device__ __forceinline__ T wave_reduce(T v, Op op) {
-    for (int off = 32; off > 0; off >>= 1) v = op(v, __shfl_xor(v, off));
-    return v;
-}
-
-template <class T, class Op>
-__device__ T block_reduce(T v, Op op, T* scratch) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int nwaves = (blockDim.x + 63) >> 6;
-    v = wave_reduce(v, op);
-    if (lane == 0) scratch[wave] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        T t = scratch[0];
-        for (int i = 1; i < nwaves; ++i) t = op(t, scratch[i]);
-        scratch[0] = t;
-    }
-    __syncthreads();
-    T r = scratch[0];
-    __syncthreads();
-    return r;
-}
-
 // Wave64 reduction without LDS: DPP swaps within each row of 16 lanes (xor 1,
 // xor 2, half-row mirror, row mirror leave every lane of a row with the row's
 // result), then the four rows combined from lanes 0, 16, 32, 48.  Every lane
@@ -177,6 +154,13 @@ struct OpAdd {
     __device__ T operator()(T a, T b) const { return a + b; }
 };
 
+// LDS written by some lanes of a wave and then read by others of the same wave.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 struct PixelIn {
     float depth;
     vec3 normal;
@@ -210,12 +194,22 @@ __device__ __forceinline__ void store_range(const BmfrGeom& g, int bx, int by, f
 // bmfrPre: 13 features of every padded pixel to the fp16 feature buffer
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(1024) k_bmfr_pre(BmfrGeom g, pbrt_bmfr_images im) {
-    __shared__ float scratch[16];
+    __shared__ float range[2][16];
     const int lx = threadIdx.x % g.bs, ly = threadIdx.x / g.bs;
     const int gx = blockIdx.x * g.bs + lx, gy = blockIdx.y * g.bs + ly;
     PixelIn p = load_pixel(g, im, gx, gy);
-    float mn = block_reduce(p.depth, OpMin(), scratch);
-    float mx = block_reduce(p.depth, OpMax(), scratch);
+    const int waves = (blockDim.x + 63) >> 6;
+    float mn = wave_reduce_dpp(p.depth, OpMin());
+    float mx = wave_reduce_dpp(p.depth, OpMax());
+    if ((threadIdx.x & 63) == 0) {
+        range[0][threadIdx.x >> 6] = mn;
+        range[1][threadIdx.x >> 6] = mx;
+    }
+    __syncthreads();
+    for (int w = 0; w < waves; ++w) {
+        mn = fminf(mn, range[0][w]);
+        mx = fmaxf(mx, range[1][w]);
+    }
     if (threadIdx.x == 0) store_range(g, blockIdx.x, blockIdx.y, mn, mx);
     float z = (p.depth - mn) / (mx - mn + 1e-6f);
     float px = (float)lx / (float)(g.bs - 1), py = (float)ly / (float)(g.bs - 1);
@@ -230,78 +224,141 @@ __global__ void __launch_bounds__(1024) k_bmfr_pre(BmfrGeom g, pbrt_bmfr_images 
 // ---------------------------------------------------------------------------
 // bmfrFit: FP32 Householder QR of the (bs^2 x 13) block, reference algorithm
 // ---------------------------------------------------------------------------
-template <int kSub>
-__global__ void __launch_bounds__(256) k_bmfr_fit_householder(BmfrGeom g) {
-    __shared__ float scratch[16];
-    __shared__ float u_length_squared;
-    __shared__ vec3 ws[kFeatures];
-    const int id = threadIdx.x;
-    const int T = blockDim.x;
+// What bounds it is the chain of block reductions: a column needs the norm of its lower
+// part, then its dot products with every later column.  Those up to twelve products are
+// summed together (wave_sums.hpp) and cost one barrier, as the norm does: two barriers a
+// column, against a wave butterfly and three barriers for each of the 85 sums.  Each sum
+// is the tree of a butterfly, then the waves in order.  The update's quotient
+// (2 u v) / |u|^2 divides by one number per column, so it is a product with its
+// reciprocal and one correction by the exact residual (the correctly rounded quotient,
+// in three operations), except where the divisor's magnitude could make the residual
+// inexact.  The back-substitution runs in the first wave: lane i holds row i, and each
+// solved weight is broadcast to the rows above it.  A 16-pixel block is one wave of four
+// rows per lane (no barrier; four waves of one row each took 226 us where this takes
+// 138).  Whole passes (pre, fit, post), 32-pixel blocks: 1279x719 246 -> 69 us, 1920x1080
+// 462 -> 130 us; 1920x1080 with 16-pixel blocks 368 -> 138 us; 1155x676 with 8-pixel
+// blocks 169 -> 112 us.
+constexpr int kFitCols = kAlphaSize - 1;  // columns a reduction sums at most
+
+template <int kSub, int kWaves>
+__global__ void __launch_bounds__(64 * kWaves) k_bmfr_fit_householder(BmfrGeom g) {
+    constexpr int T = 64 * kWaves;
+    __shared__ __attribute__((aligned(16))) float dots[2][kFitCols * kWaves];  // [parity][column][wave]
+    __shared__ float norms[2][kWaves];
+    __shared__ float pivot[2];  // |u|^2 of the current column
+    const int id = threadIdx.x, lane = id & 63, wave = id >> 6;
+    const int bank = (lane >> 2) & 3, row16 = lane >> 4;
     const int bs = g.bs;
     const uint32_t pb = (uint32_t)(bs * bs);
     const int basex = blockIdx.x * bs, basey = blockIdx.y * bs;
     const size_t plane = (size_t)g.wp * g.hp;
     float feat[kSub][kAlphaSize];
-    for (int col = 0; col < kAlphaSize; ++col)
-        for (int s = 0; s < kSub; ++s) {
-            const int index = id + s * T;
-            const int px = index / bs + basex, py = index % bs + basey;
-            float v = h2f(g.features[col * plane + (size_t)py * g.wp + px]);
+#pragma unroll
+    for (int s = 0; s < kSub; ++s) {
+        const int index = id + s * T;
+        const int px = index / bs + basex, py = index % bs + basey;
+        const uint16_t* src = g.features + (size_t)py * g.wp + px;
+#pragma unroll
+        for (int col = 0; col < kAlphaSize; ++col) {
+            float v = h2f(src[col * plane]);
             if (col < kFeatures)
                 v = add_noise(v, (uint32_t)index + (uint32_t)col * pb * pb + g.frame * (uint32_t)kAlphaSize * pb * pb);
             feat[s][col] = v;
         }
+    }
+    float uls = 0.0f;
+#pragma unroll
     for (int col = 0; col < kFeatures; ++col) {
+        const int buf = col & 1;
         float u[kSub];
         float val2 = 0.0f;
+#pragma unroll
         for (int s = 0; s < kSub; ++s) {
-            const int index = id + s * T;
             u[s] = feat[s][col];
-            if (index > col) val2 += u[s] * u[s];
+            if (id + s * T > col) val2 += u[s] * u[s];
         }
-        float vec_len_squ = block_reduce(val2, OpAdd(), scratch);
+        float len2 = wave_sum(val2);
+        if constexpr (kWaves > 1) {
+            if (lane == 0) norms[buf][wave] = len2;
+            __syncthreads();
+            len2 = norms[buf][0];
+#pragma unroll
+            for (int w = 1; w < kWaves; ++w) len2 += norms[buf][w];
+        }
         if (id < col) {
             u[0] = 0.0f;
         } else if (id == col) {
-            float vec_len = sqrtf(vec_len_squ + u[0] * u[0]);
+            const float vec_len = sqrtf(len2 + u[0] * u[0]);
             u[0] -= vec_len;
-            vec_len_squ += u[0] * u[0];
-            u_length_squared = vec_len_squ;
+            len2 += u[0] * u[0];
+            pivot[buf] = len2;
             feat[0][col] = vec_len;
         } else {
             feat[0][col] = 0.0f;
         }
-        __syncthreads();
-        const float uls = u_length_squared;
+        // dot products with the later columns (u is 0 in the rows above the pivot, which
+        // keep their values)
+        float q[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int f = col + 1 + 4 * k + r;
+                v[r] = 0.0f;
+                if (f < kAlphaSize) {
+#pragma unroll
+                    for (int s = 0; s < kSub; ++s)
+                        if (id + s * T >= col) v[r] += feat[s][f] * u[s];
+                }
+            }
+            q[k] = col + 1 + 4 * k < kAlphaSize ? row_steps84(rows_of(v[0], v[1], v[2], v[3])) : 0.0f;
+        }
+        const float part = quad_steps21(by_bank(bank, q[0], q[1], q[2], 0.0f));
+        if ((lane & 3) == 0 && bank < 3) dots[buf][(4 * bank + row16) * kWaves + wave] = part;
+        if (kWaves > 1)
+            __syncthreads();
+        else
+            wave_lds_sync();
+        uls = pivot[buf];
+        const float inv = 1.0f / uls;
+        // with |u|^2 well inside the normal range the residual below is exact
+        const bool safe = uls > 0x1p-60f && uls < 0x1p60f;
+#pragma unroll
         for (int f = col + 1; f < kAlphaSize; ++f) {
-            float v = 0.0f;
+            const float* d = &dots[buf][(f - col - 1) * kWaves];
+            float v = d[0];
+#pragma unroll
+            for (int w = 1; w < kWaves; ++w) v += d[w];
+#pragma unroll
             for (int s = 0; s < kSub; ++s) {
-                const int index = id + s * T;
-                if (index >= col) v += feat[s][f] * u[s];
-            }
-            v = block_reduce(v, OpAdd(), scratch);
-            for (int s = 0; s < kSub; ++s) {
-                const int index = id + s * T;
-                if (index >= col) feat[s][f] -= 2.0f * u[s] * v / uls;
+                const float n = 2.0f * u[s] * v;
+                float x;
+                if (safe) {
+                    x = n * inv;
+                    x = fmaf(fmaf(-x, uls, n), inv, x);
+                } else {
+                    x = n / uls;
+                }
+                if (id + s * T >= col) feat[s][f] -= x;
             }
         }
     }
+    if (wave != 0) return;
+    // lane i < 10: row i of the triangle, its right-hand sides in columns 10..12
+    vec3 w = make_vec3(feat[0][10], feat[0][11], feat[0][12]);
+#pragma unroll
     for (int i = kFeatures - 1; i >= 0; --i) {
-        if (id == i) {
-            vec3 w = make_vec3(feat[0][10], feat[0][11], feat[0][12]);
-            for (int x = i + 1; x < kFeatures; ++x) w -= ws[x] * feat[0][x];
-            w /= feat[0][i];
-            ws[i] = w;
-        }
-        __syncthreads();
+        if (lane == i) w /= feat[0][i];
+        const vec3 wi = make_vec3(read_lane(w.x, i), read_lane(w.y, i), read_lane(w.z, i));
+        if (lane < i) w -= wi * feat[0][i];
     }
-    if (id < kFeatures) {
-        vec3 w = ws[id];
-        if (u_length_squared == 0.0f) w = make_vec3(0.2f);
+    if (lane < kFeatures) {
+        if (uls == 0.0f) w = make_vec3(0.2f);
         float* out = g.weights + ((size_t)blockIdx.y * g.blocks_x + blockIdx.x) * 30;
-        out[id * 3 + 0] = w.x;
-        out[id * 3 + 1] = w.y;
-        out[id * 3 + 2] = w.z;
+        out[lane * 3 + 0] = w.x;
+        out[lane * 3 + 1] = w.y;
+        out[lane * 3 + 2] = w.z;
     }
 }
 
@@ -372,13 +429,6 @@ struct GramShared {
     float amax_part[kWaves][12];
     double G[12][12];
 };
-
-// LDS written by some lanes of a wave and then read by others of the same wave.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // kThreads: workgroup size (256, 512 or 1024); its waves split the block's rows,
 // so the thread count sets how the rows are tiled over the matrix cores
@@ -1064,11 +1114,11 @@ static void launch_bmfr(const pbrt_bmfr_params& p, const pbrt_bmfr_images& im, B
     if (p.fit == PBRT_BMFR_FIT_HOUSEHOLDER) {
         hipLaunchKernelGGL(k_bmfr_pre, grid, dim3(threads), 0, st, g, im);
         if (g.bs == 32)
-            hipLaunchKernelGGL(k_bmfr_fit_householder<4>, grid, dim3(256), 0, st, g);
+            hipLaunchKernelGGL((k_bmfr_fit_householder<4, 4>), grid, dim3(256), 0, st, g);
         else if (g.bs == 16)
-            hipLaunchKernelGGL(k_bmfr_fit_householder<1>, grid, dim3(256), 0, st, g);
+            hipLaunchKernelGGL((k_bmfr_fit_householder<4, 1>), grid, dim3(64), 0, st, g);
         else
-            hipLaunchKernelGGL(k_bmfr_fit_householder<1>, grid, dim3(64), 0, st, g);
+            hipLaunchKernelGGL((k_bmfr_fit_householder<1, 1>), grid, dim3(64), 0, st, g);
     } else {
         const int entries = kFeatures * g.bs * g.bs;
         const int threads = (int)(p.fit_threads ? p.fit_threads : kFitThreads);
