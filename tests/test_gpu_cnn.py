@@ -132,6 +132,40 @@ def test_forward_matches_oracle(cuda, layers):
     net.close()
 
 
+@pytest.mark.parametrize("layers,w,h,count", [(3, 130, 75, 1), (4, 57, 40, 2), (5, 44, 3, 1), (6, 52, 61, 1),
+                                              (6, 53, 7, 3), (6, 105, 50, 1), (6, 1, 30, 1), (6, 30, 1, 1),
+                                              (6, 700, 33, 1)])
+def test_row_pipeline_matches_oracle(cuda, layers, w, h, count):
+    """Inference of three to six layers walks strips of 64 - 2 layers columns in segments of
+    rows: whole and partial strips, several segments, images narrower or shorter than the
+    network's reach, several images; to the bars of the forward test."""
+    rng = np.random.default_rng(w + h)
+    inp = dict(
+        noisy=half(rng.gamma(1.0, 0.5, (count, h, w, 4))),
+        depth=rng.uniform(0.5, 20.0, (count, h, w)).astype(np.float32),
+        normal=rng.uniform(0, np.pi, (count, h, w, 2)).astype(np.float32),
+        albedo=rng.integers(0, 256, (count, h, w, 4), dtype=np.uint8),
+        spp=rng.integers(0, 40, (count, h, w), dtype=np.uint8),
+        motion=half(rng.uniform(-1, 1, (count, h, w, 2))),
+    )
+    net = Net(5, layers)
+    params = net.get()
+    o = cnn.parameter_count(cnn.shape_of(layers)) - 25 - 9 * 32 * 25
+    params[o:o + 9 * 32 * 25] *= 10.0
+    net.set(params)
+    im, t = device_images(cuda, inp, False, w, h, count)
+    capi.check(capi.lib().pbrt_cnn_denoise(net.h, C.byref(im), helpers.stream(cuda)))
+    cuda.cuda.synchronize()
+    g = t["denoised"].cpu().numpy()[..., :3]
+    ref, _ = oracle_forward(params.astype(np.float64), inp, layers)
+    rel = np.abs(g - ref) / np.maximum(np.abs(ref), 1e-3)
+    assert np.quantile(rel, 0.99) < 2e-2 and np.median(rel) < 2e-3
+    alb = inp["albedo"][..., :3].astype(np.float64) / 255 + 1e-6
+    expect = np.clip(np.maximum(alb * g, 0) ** 0.454545, 0, 1) * 255
+    assert np.abs(t["final"].cpu().numpy()[..., 2::-1].astype(float) - expect).max() <= 1.0
+    net.close()
+
+
 @pytest.mark.parametrize("layers", [6, 2, "c"])
 def test_gradients_match_oracle(cuda, layers):
     """Every layer's gradient against the oracle's; the compact network reports zero

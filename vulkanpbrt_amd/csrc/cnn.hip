@@ -179,9 +179,7 @@ __global__ void __launch_bounds__(256) k_features(CnnGeom g, pbrt_cnn_images im,
 // ---------------------------------------------------------------------------
 // 3x3 convolution (forward, or input gradient with flipped weights)
 // ---------------------------------------------------------------------------
-// kConvKpn: last layer of inference; the logits stay on chip (LDS) and the softmax
-// 5x5 kernel is applied to the noisy taps staged with the tile.
-enum ConvMode { kConvRelu = 0, kConvLinear = 1, kConvDgrad = 2, kConvKpn = 4 };
+enum ConvMode { kConvRelu = 0, kConvLinear = 1, kConvDgrad = 2 };
 
 // Persistent: each workgroup keeps the layer's weights in registers and walks a
 // strided sequence of 16x16 tiles inside its XCD's contiguous share of the tile
@@ -191,18 +189,12 @@ enum ConvMode { kConvRelu = 0, kConvLinear = 1, kConvDgrad = 2, kConvKpn = 4 };
 template <int CIN, int MODE>
 __global__ void __launch_bounds__(256) k_conv3x3(CnnGeom g, const uint16_t* __restrict__ in,
                                                  const uint16_t* __restrict__ mask, const uint16_t* __restrict__ wgt,
-                                                 const float* __restrict__ bias, uint16_t* __restrict__ out,
-                                                 pbrt_cnn_images im) {
+                                                 const float* __restrict__ bias, uint16_t* __restrict__ out) {
     constexpr int kStride = CIN + 8;  // bf16 per LDS pixel: conflict-free 16 / 8 byte lane reads
     constexpr int kChunks = CIN / 8;
     constexpr int kTilePix = 18 * 18;
     constexpr int kLoads = (kTilePix * kChunks + 255) / 256;
-    constexpr int kNoisyPix = 20 * 20;  // kernel-prediction taps of a tile (kConvKpn)
-    constexpr int kNoisyLoads = MODE == kConvKpn ? (kNoisyPix + 255) / 256 : 1;
     __shared__ __attribute__((aligned(16))) uint16_t tile[2][kTilePix * kStride];
-    __shared__ __attribute__((aligned(16))) uint2 ntile[MODE == kConvKpn ? 2 : 1][MODE == kConvKpn ? kNoisyPix : 1];
-    __shared__ __attribute__((aligned(16))) uint16_t logit[MODE == kConvKpn ? kTile * kTile * kCh : 8];
-    uint2 nregs[kNoisyLoads];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int j = lane & 15, grp = lane >> 4;
     const int tiles_x = (g.width + kTile - 1) / kTile, tiles_y = (g.height + kTile - 1) / kTile;
@@ -216,17 +208,6 @@ __global__ void __launch_bounds__(256) k_conv3x3(CnnGeom g, const uint16_t* __re
     auto fetch = [&](int tt, uint4 (&r)[kLoads]) {
         const int img = tt / per_image, rem = tt % per_image;
         const int x0 = (rem % tiles_x) * kTile, y0 = (rem / tiles_x) * kTile;
-        if (MODE == kConvKpn) {
-#pragma unroll
-            for (int k = 0; k < kNoisyLoads; ++k) {
-                const int p = tid + k * 256;
-                if (p < kNoisyPix) {
-                    const int yy = min(max(y0 + p / 20 - 2, 0), g.height - 1);
-                    const int xx = min(max(x0 + p % 20 - 2, 0), g.width - 1);
-                    nregs[k] = reinterpret_cast<const uint2*>(im.noisy)[plane * img + (size_t)yy * g.width + xx];
-                }
-            }
-        }
         const uint16_t* src = in + plane * img * CIN;
         const uint16_t* msk = mask ? mask + plane * img * CIN : nullptr;
 #pragma unroll
@@ -245,13 +226,6 @@ __global__ void __launch_bounds__(256) k_conv3x3(CnnGeom g, const uint16_t* __re
         }
     };
     auto stash = [&](int b, const uint4 (&r)[kLoads]) {
-        if (MODE == kConvKpn) {
-#pragma unroll
-            for (int k = 0; k < kNoisyLoads; ++k) {
-                const int p = tid + k * 256;
-                if (p < kNoisyPix) ntile[b][p] = nregs[k];
-            }
-        }
 #pragma unroll
         for (int k = 0; k < kLoads; ++k) {
             const int e = tid + k * 256;
@@ -328,59 +302,6 @@ __global__ void __launch_bounds__(256) k_conv3x3(CnnGeom g, const uint16_t* __re
         const int img = t / per_image, rem = t % per_image;
         const int x0 = (rem % tiles_x) * kTile, y0 = (rem / tiles_x) * kTile;
         const int gx = x0 + j;
-        if (MODE == kConvKpn) {
-            // bf16 logits of the tile to LDS, then one thread per pixel: softmax over the
-            // 25 logits and the 5x5 weighted sum of the staged noisy taps
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int p = (wave * 4 + r) * kTile + j;
-#pragma unroll
-                for (int ct = 0; ct < 2; ++ct) {
-                    float v[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) v[i] = acc[r][ct][i] + bv[ct][i];
-                    *reinterpret_cast<uint2*>(&logit[p * kCh + ct * 16 + 4 * grp]) =
-                        make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
-                }
-            }
-            __syncthreads();
-            const int py = tid / kTile, px = tid % kTile;
-            const int gy = y0 + py, gxp = x0 + px;
-            if (gxp < g.width && gy < g.height) {
-                float z[kKernelTaps];
-                float zmax = -3.4e38f;
-#pragma unroll
-                for (int c = 0; c < kKernelTaps; ++c) {
-                    z[c] = bf2f(logit[tid * kCh + c]);
-                    zmax = fmaxf(zmax, z[c]);
-                }
-                float sum = 0.0f;
-#pragma unroll
-                for (int c = 0; c < kKernelTaps; ++c) {
-                    z[c] = expf(z[c] - zmax);
-                    sum += z[c];
-                }
-                const float inv = 1.0f / sum;
-                vec3 o = make_vec3(0.0f);
-#pragma unroll
-                for (int c = 0; c < kKernelTaps; ++c) {
-                    // staged taps: tile-local row/col of the clamped image position
-                    const int yy = min(max(gy + c / 5 - 2, 0), g.height - 1) - (y0 - 2);
-                    const int xx = min(max(gxp + c % 5 - 2, 0), g.width - 1) - (x0 - 2);
-                    const uint2 hv = ntile[buf][yy * 20 + xx];
-                    o += make_vec3(h2f(hv.x & 0xFFFFu), h2f(hv.x >> 16), h2f(hv.y & 0xFFFFu)) * (z[c] * inv);
-                }
-                const size_t i = plane * img + (size_t)gy * g.width + gxp;
-                if (im.denoised) reinterpret_cast<float4*>(im.denoised)[i] = make_float4(o.x, o.y, o.z, 1.0f);
-                if (im.final_image) {
-                    const vec3 alb = xyz(load_rgba8(im.albedo, i)) + make_vec3(1e-6f);
-                    vec3 tm = alb * o;
-                    tm = make_vec3(fmaxf(tm.x, 0.0f), fmaxf(tm.y, 0.0f), fmaxf(tm.z, 0.0f));
-                    store_bgra8(im.final_image, i,
-                                make_vec4(fast_gamma(tm.x), fast_gamma(tm.y), fast_gamma(tm.z), 1.0f));
-                }
-            }
-        } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int gy = y0 + wave * 4 + r;
@@ -397,7 +318,6 @@ __global__ void __launch_bounds__(256) k_conv3x3(CnnGeom g, const uint16_t* __re
                 *reinterpret_cast<uint2*>(o + ct * 16 + 4 * grp) =
                     make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
             }
-        }
         }
         if (tn < end) stash(buf ^ 1, regs);
         __syncthreads();
@@ -584,10 +504,9 @@ k_reduce_partials(const float* __restrict__ partial, int rows, int size, float* 
 }
 
 // ---------------------------------------------------------------------------
-// Kernel prediction: softmax over 25 logits, 5x5 weighted sum of the noisy
-// illumination (taps clamped to the image); loss and its logit gradient.
+// Kernel prediction in training: softmax over 25 logits, 5x5 weighted sum of the noisy
+// illumination (taps clamped to the image), the loss and its logit gradient.
 // ---------------------------------------------------------------------------
-template <bool kTrain>
 __global__ void __launch_bounds__(256) k_kpn(CnnGeom g, pbrt_cnn_images im, const uint16_t* logits, uint16_t* dlogits,
                                             float* loss_part) {
     __shared__ float red[4];
@@ -623,52 +542,40 @@ __global__ void __launch_bounds__(256) k_kpn(CnnGeom g, pbrt_cnn_images im, cons
             tap[k] = xyz(load_half4(im.noisy, plane * img + (size_t)yy * g.width + xx));
             o += tap[k] * z[k];
         }
-        if (!kTrain) {
-            if (im.denoised) reinterpret_cast<float4*>(im.denoised)[i] = make_float4(o.x, o.y, o.z, 1.0f);
-            if (im.final_image) {
-                const vec3 alb = xyz(load_rgba8(im.albedo, i)) + make_vec3(1e-6f);
-                vec3 t = alb * o;
-                t = make_vec3(fmaxf(t.x, 0.0f), fmaxf(t.y, 0.0f), fmaxf(t.z, 0.0f));
-                store_bgra8(im.final_image, i, make_vec4(vclamp(vpow(t, 0.454545f), 0.0f, 1.0f), 1.0f));
-            }
-        } else {
-            // relative squared error of the remodulated radiance (albedo + 1e-6 as in bmfrPost)
-            const float4 t4 = reinterpret_cast<const float4*>(im.target)[i];
-            const vec3 alb = xyz(load_rgba8(im.albedo, i)) + make_vec3(1e-6f);
-            const float t[3] = {t4.x, t4.y, t4.z}, ov[3] = {o.x, o.y, o.z}, a[3] = {alb.x, alb.y, alb.z};
-            const float norm = 1.0f / (float)(n * 3);
-            float gch[3];
+        // relative squared error of the remodulated radiance (albedo + 1e-6 as in bmfrPost)
+        const float4 t4 = reinterpret_cast<const float4*>(im.target)[i];
+        const vec3 alb = xyz(load_rgba8(im.albedo, i)) + make_vec3(1e-6f);
+        const float t[3] = {t4.x, t4.y, t4.z}, ov[3] = {o.x, o.y, o.z}, a[3] = {alb.x, alb.y, alb.z};
+        const float norm = 1.0f / (float)(n * 3);
+        float gch[3];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const float at = a[c] * t[c];
-                const float d = a[c] * ov[c] - at, den = at * at + kRelEps;
-                lsum += d * d / den;
-                gch[c] = 2.0f * a[c] * d / den * norm;
-            }
-            float dw[kKernelTaps], wdw = 0.0f;
-#pragma unroll
-            for (int k = 0; k < kKernelTaps; ++k) {
-                dw[k] = gch[0] * tap[k].x + gch[1] * tap[k].y + gch[2] * tap[k].z;
-                wdw += z[k] * dw[k];
-            }
-            uint32_t packed[kCh / 2];
-#pragma unroll
-            for (int k = 0; k < kCh / 2; ++k) {
-                const float a = 2 * k < kKernelTaps ? z[2 * k] * (dw[2 * k] - wdw) : 0.0f;
-                const float b = 2 * k + 1 < kKernelTaps ? z[2 * k + 1] * (dw[2 * k + 1] - wdw) : 0.0f;
-                packed[k] = pack_bf16(a, b);
-            }
-            uint4* d4 = reinterpret_cast<uint4*>(dlogits + i * kCh);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) d4[q] = make_uint4(packed[4 * q], packed[4 * q + 1], packed[4 * q + 2], packed[4 * q + 3]);
+        for (int c = 0; c < 3; ++c) {
+            const float at = a[c] * t[c];
+            const float d = a[c] * ov[c] - at, den = at * at + kRelEps;
+            lsum += d * d / den;
+            gch[c] = 2.0f * a[c] * d / den * norm;
         }
+        float dw[kKernelTaps], wdw = 0.0f;
+#pragma unroll
+        for (int k = 0; k < kKernelTaps; ++k) {
+            dw[k] = gch[0] * tap[k].x + gch[1] * tap[k].y + gch[2] * tap[k].z;
+            wdw += z[k] * dw[k];
+        }
+        uint32_t packed[kCh / 2];
+#pragma unroll
+        for (int k = 0; k < kCh / 2; ++k) {
+            const float a = 2 * k < kKernelTaps ? z[2 * k] * (dw[2 * k] - wdw) : 0.0f;
+            const float b = 2 * k + 1 < kKernelTaps ? z[2 * k + 1] * (dw[2 * k + 1] - wdw) : 0.0f;
+            packed[k] = pack_bf16(a, b);
+        }
+        uint4* d4 = reinterpret_cast<uint4*>(dlogits + i * kCh);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d4[q] = make_uint4(packed[4 * q], packed[4 * q + 1], packed[4 * q + 2], packed[4 * q + 3]);
     }
-    if (kTrain) {
-        for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = lsum;
-        __syncthreads();
-        if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
-    }
+    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = lsum;
+    __syncthreads();
+    if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
 // ---------------------------------------------------------------------------
@@ -734,24 +641,21 @@ LayerTable layer_table(int layers) {
     return lt;
 }
 
-// Softmax over one output pixel's 25 bf16 logits (LDS, `logits`: 32 channels, 25
-// used) and the 5x5 weighted sum of its noisy taps; thread `tid` of the 16x16 tile at
-// (x0, y0).  `taps` is the tile's noisy halo (raw FP16 RGBA, clamped to the image)
-// with row length `halo`, offset so that tap (ky, kx) of tile pixel (py, px) sits at
-// (py + ky, px + kx).  Writes the denoised radiance and / or the final image.
-__device__ __forceinline__ void kpn_apply_pixel(const CnnGeom& g, const pbrt_cnn_images& im, const uint16_t* logits,
-                                                const uint2* ntile, int halo, size_t image_base, int x0, int y0,
-                                                int tid, const uint32_t* albedo_lds = nullptr) {
-    const int py = tid / kTile, px = tid % kTile;
-    const int gy = y0 + py, gx = x0 + px;
-    if (gx >= g.width || gy >= g.height) return;
+// Softmax weights of one output pixel from its 25 bf16 logits (LDS, `logits`: 32
+// channels, 25 used; its 16-byte chunk q at q ^ swizzle), not yet normalised.
+struct KpnWeights {
+    float e[kKernelTaps];
+    float sum;
+};
+
+__device__ __forceinline__ KpnWeights kpn_weights(const uint16_t* logits, int swizzle = 0) {
     // the 25 bf16 logits (and 7 padding channels): four 16-byte reads, twice
     // (maximum, then the weighted sum) to keep few registers live
     const uint4* lz = reinterpret_cast<const uint4*>(logits);
     float zmax = -3.4e38f;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const uint4 v = lz[q];
+        const uint4 v = lz[q ^ swizzle];
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
@@ -762,47 +666,71 @@ __device__ __forceinline__ void kpn_apply_pixel(const CnnGeom& g, const pbrt_cnn
     }
     // exp(z - max) = exp2(z log2(e) - max log2(e)); the normalisation is applied once
     const float l2e = 1.4426950408889634f, zm = zmax * l2e;
-    // the halo holds the clamped noisy pixel at every position, so tap (ky, kx) of
-    // this pixel sits at (py + ky, px + kx) also on border tiles: the 25 reads are
-    // constant offsets from one address
-    const uint2* taps = &ntile[py * halo + px];
-    float sum = 0.0f, ox = 0.0f, oy = 0.0f, oz = 0.0f;
+    KpnWeights r;
+    r.sum = 0.0f;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const uint4 v = lz[q];
+        const uint4 v = lz[q ^ swizzle];
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const int c = 8 * q + k;
             if (c < kKernelTaps) {
                 const float zc = __uint_as_float((k & 1) ? (w[k / 2] & 0xFFFF0000u) : (w[k / 2] << 16));
-                const float e = __builtin_amdgcn_exp2f(fmaf(zc, l2e, -zm));
-                // FP16 taps widen exactly inside the multiply-add (v_fma_mix_f32)
-                const uint2 nv = taps[(c / 5) * halo + c % 5];
-                const half2v rg = __builtin_bit_cast(half2v, nv.x), ba = __builtin_bit_cast(half2v, nv.y);
-                sum += e;
-                ox = fmaf((float)rg.x, e, ox);
-                oy = fmaf((float)rg.y, e, oy);
-                oz = fmaf((float)ba.x, e, oz);
+                r.e[c] = __builtin_amdgcn_exp2f(fmaf(zc, l2e, -zm));
+                r.sum += r.e[c];
             }
         }
     }
-    const float inv = __builtin_amdgcn_rcpf(sum);  // 1 ulp
+    return r;
+}
+
+// The 5x5 weighted sum of the noisy taps (`tap(k)`: raw FP16 RGBA of tap k, from the halo
+// clamped to the image).  Writes the denoised radiance and / or the final image of pixel
+// `i`; `albedo` is that pixel's RGBA8 (in a register, LDS or the image).
+template <class Tap>
+__device__ __forceinline__ void kpn_apply(const pbrt_cnn_images& im, const KpnWeights& k, Tap tap, size_t i,
+                                          const uint32_t* albedo) {
+    float ox = 0.0f, oy = 0.0f, oz = 0.0f;
+#pragma unroll
+    for (int c = 0; c < kKernelTaps; ++c) {
+        // FP16 taps widen exactly inside the multiply-add (v_fma_mix_f32)
+        const uint2 nv = tap(c);
+        const half2v rg = __builtin_bit_cast(half2v, nv.x), ba = __builtin_bit_cast(half2v, nv.y);
+        ox = fmaf((float)rg.x, k.e[c], ox);
+        oy = fmaf((float)rg.y, k.e[c], oy);
+        oz = fmaf((float)ba.x, k.e[c], oz);
+    }
+    const float inv = __builtin_amdgcn_rcpf(k.sum);  // 1 ulp
     ox *= inv;
     oy *= inv;
     oz *= inv;
-    const size_t i = image_base + (size_t)gy * g.width + gx;
     if (im.denoised) reinterpret_cast<float4*>(im.denoised)[i] = make_float4(ox, oy, oz, 1.0f);
     if (im.final_image) {
-        // remodulated, gamma 1/2.2 (the albedo from LDS when the caller staged it)
-        const uchar4 ac = albedo_lds ? __builtin_bit_cast(uchar4, *albedo_lds)
-                                     : reinterpret_cast<const uchar4*>(im.albedo)[i];
-        const float k = 1.0f / 255.0f;
-        const float tx = fmaxf(((float)ac.x * k + 1e-6f) * ox, 0.0f);
-        const float ty = fmaxf(((float)ac.y * k + 1e-6f) * oy, 0.0f);
-        const float tz = fmaxf(((float)ac.z * k + 1e-6f) * oz, 0.0f);
+        // remodulated, gamma 1/2.2
+        const uchar4 ac = __builtin_bit_cast(uchar4, *albedo);
+        const float k255 = 1.0f / 255.0f;
+        const float tx = fmaxf(((float)ac.x * k255 + 1e-6f) * ox, 0.0f);
+        const float ty = fmaxf(((float)ac.y * k255 + 1e-6f) * oy, 0.0f);
+        const float tz = fmaxf(((float)ac.z * k255 + 1e-6f) * oz, 0.0f);
         store_bgra8(im.final_image, i, make_vec4(fast_gamma(tx), fast_gamma(ty), fast_gamma(tz), 1.0f));
     }
+}
+
+// The softmax filter for thread `tid` of the 16x16 tile at (x0, y0).  `ntile` is the tile's noisy
+// halo with row length `halo`, offset so that tap (ky, kx) of tile pixel (py, px) sits at
+// (py + ky, px + kx), also on border tiles: the 25 reads are constant offsets from one
+// address.
+__device__ __forceinline__ void kpn_apply_pixel(const CnnGeom& g, const pbrt_cnn_images& im, const uint16_t* logits,
+                                                const uint2* ntile, int halo, size_t image_base, int x0, int y0,
+                                                int tid, const uint32_t* albedo_lds = nullptr) {
+    const int py = tid / kTile, px = tid % kTile;
+    const int gy = y0 + py, gx = x0 + px;
+    if (gx >= g.width || gy >= g.height) return;
+    const uint2* taps = &ntile[py * halo + px];
+    const size_t i = image_base + (size_t)gy * g.width + gx;
+    kpn_apply(im, kpn_weights(logits), [&](int c) { return taps[(c / 5) * halo + c % 5]; }, i,
+              albedo_lds ? albedo_lds : reinterpret_cast<const uint32_t*>(im.albedo) + i);
 }
 
 // ---------------------------------------------------------------------------
@@ -947,6 +875,233 @@ __global__ void __launch_bounds__(256, 3) k_two_layer(CnnGeom g, pbrt_cnn_images
         kpn_apply_pixel(g, im, buf_f + tid * kHidStride, ntile, kTwoHalo, plane * img, x0, y0, tid);
         __syncthreads();  // the next tile's features overwrite the logits and taps
     }
+}
+
+// ---------------------------------------------------------------------------
+// Three to six layers, fused (inference): a row pipeline
+// ---------------------------------------------------------------------------
+// A workgroup walks down a strip of 64 columns one row per step and every layer works on
+// the row its predecessor finished in the step before, so activations never leave LDS
+// and the only recomputed pixels are the strip's L columns and rows at each edge.  Two
+// waves per layer take 16 output channels each with that layer's weights in registers;
+// one wave computes the feature row and two the softmax filter of the finished logits, on
+// alternate rows (at 6 layers 15 waves, at most 128 registers, one workgroup per CU).
+//   A convolution wave reads each input row once, as three horizontally shifted operands
+// per 16 columns, and adds it to the three output rows it contributes to (output row r
+// receives input rows r - 1, r, r + 1 in three consecutive steps): three LDS reads per
+// nine matrix instructions.  Reading it nine times, once per tap, would need more LDS
+// bandwidth than the matrix cores leave time for.
+//   Step t, with row numbers counted from y0 - L: the features wave writes row t, layer l
+// finishes row t - 2l - 2, the filter takes row t - 1 - 2L and stores it in the step
+// after.  Rows and columns outside the image are zero after every layer (the
+// convolutions' padding); edge columns and the first rows a layer finishes hold values
+// made from unwritten neighbours, which reach only pixels the strip does not output.
+//   What bounds it: the matrix cores, 1728 cycles a row on the busiest SIMD (154 us at
+// 1920x1080, of which a third is strip and segment halo), then a step's first operands,
+// its stores and the barrier.  Two rows per step save barriers but add L rows of latency
+// (217 us).  6 layers, before (seven launches through HBM) and now: 1920x1080 377 -> 210
+// us, 1280x720 166 -> 103, 480x270 48 -> 36, 200x120 31 -> 26.
+constexpr int kPipeCols = 64;                 // columns of a strip
+constexpr int kPipeTiles = kPipeCols / 16;    // 16-pixel matrix tiles of a row
+constexpr int kPipePix = kPipeCols + 2;       // LDS pixels of a row (column c at c + 1)
+constexpr int kPipeRing = 32;                 // noisy rows kept for the filter (2L + 5 are live)
+// An LDS pixel is 32 channels in four 16-byte chunks, chunk q at q ^ pipe_swizzle(pixel).
+// A 16-byte read serves sixteen lanes at a time, eight neighbouring pixels of one chunk and
+// the same pixels of the next: so placed, they meet in distinct banks (pixels side by side
+// without it, or 80 bytes apart, spent half of the LDS cycles on conflicts).
+__device__ __forceinline__ constexpr int pipe_swizzle(int pixel) { return (pixel & 4) >> 1; }
+constexpr int kPipeStride = kCh, kPipeFeatStride = kFeatCh;
+
+constexpr int pipe_threads(int layers) { return 64 * (2 * layers + 3); }
+
+template <int L>
+struct PipeShared {
+    // double-buffered by step
+    __attribute__((aligned(16))) uint16_t feat[2][kPipePix * kPipeFeatStride];
+    __attribute__((aligned(16))) uint16_t act[L][2][kPipePix * kPipeStride];  // layer l's rows; the last: logits
+    __attribute__((aligned(16))) uint2 noisy[kPipeRing][kPipeCols];          // clamped to the image, raw FP16
+};
+
+// What every wave of a workgroup knows of its strip: image column of strip column 0,
+// image row of row number 0, its output rows and the number of steps (a multiple of 3).
+struct PipeStrip {
+    int x0, y0, rows, steps, img;
+};
+
+// One convolution wave: layer `l`, output channels 16 half ... + 15.  kFirst: 16 input
+// channels, two horizontal taps per matrix instruction (the third with a zero partner).
+template <int L, bool kFirst, bool kLast>
+__device__ __forceinline__ void pipe_conv(const CnnGeom& g, const PipeStrip& p, PipeShared<L>& S, int l, int half,
+                                          const uint16_t* __restrict__ wf, const float* __restrict__ master) {
+    constexpr int kK = kFirst ? 2 : 3;  // operands per tile and input row
+    constexpr int kStride = kFirst ? kPipeFeatStride : kPipeStride;
+    const int lane = threadIdx.x & 63, j = lane & 15, grp = lane >> 4;
+    const int woff = kFirst ? 0 : weight_offset(1) + (l - 1) * layer_weights(1);
+    const int boff = kFirst ? layer_weights(0) : layer_offset(1) + (l - 1) * layer_size(1) + layer_weights(1);
+    bf16x8 w[3][kK];
+#pragma unroll
+    for (int ky = 0; ky < 3; ++ky)
+#pragma unroll
+        for (int k = 0; k < kK; ++k) {
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (kFirst) {
+                const int kx = 2 * k + (grp >> 1);
+                if (kx < 3)
+                    v = *reinterpret_cast<const uint4*>(
+                        wf + woff + ((ky * 3 + kx) * kCh + half * 16 + j) * kFeatCh + 8 * (grp & 1));
+            } else {
+                v = *reinterpret_cast<const uint4*>(wf + woff + ((ky * 3 + k) * kCh + half * 16 + j) * kCh + 8 * grp);
+            }
+            w[ky][k] = __builtin_bit_cast(bf16x8, v);
+        }
+    float4v bias;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bias[i] = master[boff + half * 16 + 4 * grp + i];
+    // upper bound of the ReLU by column: 0 outside the image
+    float hi[kPipeTiles];
+#pragma unroll
+    for (int n = 0; n < kPipeTiles; ++n) {
+        const int x = p.x0 + 16 * n + j;
+        hi[n] = x >= 0 && x < g.width ? INFINITY : 0.0f;
+    }
+    // this lane's element of an operand: pixel j + tap of a tile, 8 channels (the zero
+    // partner of the first layer's third tap reads that tap's own pixel)
+    int at[kK];
+#pragma unroll
+    for (int k = 0; k < kK; ++k)
+        at[k] = kFirst ? (k == 0 ? j + (grp >> 1) : j + 2) * kStride + 8 * (grp & 1)
+                       : (j + k) * kStride + 8 * (grp ^ pipe_swizzle(j + k));
+    // the lane's 16 bytes of a finished tile pair (see below)
+    const int out = (1 + 16 * (grp & 1) + j) * kPipeStride + 8 * ((2 * half + (grp >> 1)) ^ pipe_swizzle(1 + j));
+    float4v acc[3][kPipeTiles];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int n = 0; n < kPipeTiles; ++n) acc[a][n] = bias;
+    for (int t3 = 0; t3 < p.steps; t3 += 3) {
+#pragma unroll
+        for (int ph = 0; ph < 3; ++ph) {  // the accumulators this step's row completes
+            const int t = t3 + ph;
+            const uint16_t* in = kFirst ? S.feat[(t & 1) ^ 1] : S.act[l - 1][(t & 1) ^ 1];
+#pragma unroll
+            for (int n = 0; n < kPipeTiles; ++n) {
+                float4v &fin = acc[ph][n], &mid = acc[(ph + 1) % 3][n], &beg = acc[(ph + 2) % 3][n];
+                beg = bias;
+#pragma unroll
+                for (int k = 0; k < kK; ++k) {
+                    const bf16x8 b =
+                        __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(in + 16 * n * kStride + at[k]));
+                    fin = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[2][k], b, fin, 0, 0, 0);
+                    mid = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[1][k], b, mid, 0, 0, 0);
+                    beg = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[0][k], b, beg, 0, 0, 0);
+                }
+            }
+            const int y = p.y0 + t - 2 * l - 2;
+            const bool row = y >= 0 && y < g.height;
+            uint16_t* o = S.act[l][t & 1] + out;
+            // a lane holds channels 4 grp .. 4 grp + 3 of a pixel; swapping odd and even
+            // 16-lane rows between two tiles leaves each lane eight channels of one pixel:
+            // the even rows of the first tile's, the odd rows of the second's
+#pragma unroll
+            for (int n = 0; n < kPipeTiles; n += 2) {
+                uint32_t q[2][2];
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    float v[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        v[i] = kLast ? acc[ph][n + m][i]
+                                     : __builtin_amdgcn_fmed3f(acc[ph][n + m][i], 0.0f, row ? hi[n + m] : 0.0f);
+                    q[m][0] = pack_bf16(v[0], v[1]);
+                    q[m][1] = pack_bf16(v[2], v[3]);
+                }
+                const auto lo = __builtin_amdgcn_permlane16_swap(q[0][0], q[1][0], false, false);
+                const auto up = __builtin_amdgcn_permlane16_swap(q[0][1], q[1][1], false, false);
+                *reinterpret_cast<uint4*>(o + 16 * n * kPipeStride) = make_uint4(lo[0], up[0], lo[1], up[1]);
+            }
+            __syncthreads();
+        }
+    }
+}
+
+template <int L>
+__device__ __forceinline__ void pipe_features(const CnnGeom& g, const PipeStrip& p, const pbrt_cnn_images& im,
+                                              PipeShared<L>& S) {
+    const int c = threadIdx.x & 63, x = p.x0 + c;
+    const size_t base = (size_t)g.width * g.height * p.img;
+    const int xc = min(max(x, 0), g.width - 1);
+    auto fetch = [&](int t) {
+        const int yc = min(max(p.y0 + t, 0), g.height - 1);
+        return load_raw_pixel(im, base + (size_t)yc * g.width + xc);
+    };
+    RawPixel raw = fetch(0);
+    for (int t = 0; t < p.steps; ++t) {
+        const RawPixel cur = raw;
+        raw = fetch(t + 1);  // in flight until the next step
+        const int y = p.y0 + t;
+        uint4 lo = make_uint4(0, 0, 0, 0), hi = lo;
+        if (x == xc && y >= 0 && y < g.height) raw_features(cur, lo, hi);
+        uint16_t* f = S.feat[t & 1] + (c + 1) * kPipeFeatStride;
+        *reinterpret_cast<uint4*>(f) = lo;
+        *reinterpret_cast<uint4*>(f + 8) = hi;
+        S.noisy[t % kPipeRing][c] = cur.noisy;
+        __syncthreads();
+    }
+}
+
+// The softmax filter of every second row, over two steps a row: the weights in the step
+// its logits arrive, the 25 taps and the stores in the next.
+template <int L>
+__device__ __forceinline__ void pipe_filter(const CnnGeom& g, const PipeStrip& p, const pbrt_cnn_images& im,
+                                            const PipeShared<L>& S, int parity) {
+    const int c = threadIdx.x & 63, x = p.x0 + c;
+    const size_t base = (size_t)g.width * g.height * p.img;
+    const bool column = c >= L && c < kPipeCols - L && x < g.width;
+    uint32_t albedo = 0;
+    KpnWeights k;
+    for (int t = 0; t < p.steps; ++t) {
+        // the row whose logits arrived in this step, or in the one before
+        const int o = t - 1 - 2 * L - ((t & 1) ^ parity);
+        if (column && o >= L && o < L + p.rows) {
+            const size_t i = base + (size_t)(p.y0 + o) * g.width + x;
+            if ((t & 1) == parity) {
+                albedo = reinterpret_cast<const uint32_t*>(im.albedo)[i];
+                k = kpn_weights(S.act[L - 1][(t & 1) ^ 1] + (c + 1) * kPipeStride, pipe_swizzle(c + 1));
+            } else {
+                const uint2* taps[5];
+#pragma unroll
+                for (int q = 0; q < 5; ++q) taps[q] = &S.noisy[(o + q - 2) % kPipeRing][c - 2];
+                kpn_apply(im, k, [&](int q) { return taps[q / 5][q % 5]; }, i, &albedo);
+            }
+        }
+        __syncthreads();
+    }
+}
+
+template <int L>
+__global__ void __launch_bounds__(pipe_threads(L)) k_pipeline(CnnGeom g, pbrt_cnn_images im,
+                                                              const uint16_t* __restrict__ wf,
+                                                              const float* __restrict__ master, int seg_rows,
+                                                              int strips_x) {
+    __shared__ PipeShared<L> S;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    PipeStrip p;
+    const int first = blockIdx.y * seg_rows;
+    p.x0 = (int)(blockIdx.x % strips_x) * (kPipeCols - 2 * L) - L;
+    p.y0 = first - L;
+    p.rows = min(seg_rows, g.height - first);
+    p.steps = (p.rows + 3 * L + 2 + 2) / 3 * 3;  // the last row is stored in step rows + 3L + 1
+    p.img = blockIdx.x / strips_x;
+    if (wave < 2)
+        pipe_conv<L, true, false>(g, p, S, 0, wave, wf, master);
+    else if (wave < 2 * L - 2)
+        pipe_conv<L, false, false>(g, p, S, wave >> 1, wave & 1, wf, master);
+    else if (wave < 2 * L)
+        pipe_conv<L, false, true>(g, p, S, L - 1, wave & 1, wf, master);
+    else if (wave < 2 * L + 2)
+        pipe_filter<L>(g, p, im, S, wave & 1);
+    else
+        pipe_features<L>(g, p, im, S);
 }
 
 // ---------------------------------------------------------------------------
@@ -1184,29 +1339,33 @@ void check_images(const pbrt_cnn_images* im, bool training, int layers, const ch
     PBRT_REQUIRE(im->workspace && im->workspace_bytes >= need, std::string(fn) + ": workspace too small");
 }
 
-// Workgroups for a persistent convolution: every CU's resident share, a multiple of
-// the 8 XCDs, no more than the tiles.
-template <class K>
-dim3 persistent_grid(K kernel, int tiles) {
+int compute_units() {
     static int cus = 0;
     if (!cus) {
         int dev = 0;
         PBRT_HIP(hipGetDevice(&dev));
         PBRT_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     }
+    return std::max(cus, 1);
+}
+
+// Workgroups for a persistent convolution: every CU's resident share, a multiple of
+// the 8 XCDs, no more than the tiles.
+template <class K>
+dim3 persistent_grid(K kernel, int tiles) {
     int per_cu = 0;
     PBRT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, 0));
-    int blocks = std::max(1, cus * std::max(per_cu, 1));
+    int blocks = std::max(1, compute_units() * std::max(per_cu, 1));
     blocks = std::min(blocks, ((tiles + 7) / 8) * 8);
     return dim3((unsigned)(((blocks + 7) / 8) * 8));
 }
 
 template <int CIN, int MODE>
 void launch_conv(const CnnGeom& g, const uint16_t* in, const uint16_t* mask, const uint16_t* w, const float* b,
-                 uint16_t* out, hipStream_t st, const pbrt_cnn_images& im = pbrt_cnn_images{}) {
+                 uint16_t* out, hipStream_t st) {
     const int tiles = ((g.width + kTile - 1) / kTile) * ((g.height + kTile - 1) / kTile) * g.count;
     const dim3 grid = persistent_grid(k_conv3x3<CIN, MODE>, tiles);
-    hipLaunchKernelGGL((k_conv3x3<CIN, MODE>), grid, dim3(256), 0, st, g, in, mask, w, b, out, im);
+    hipLaunchKernelGGL((k_conv3x3<CIN, MODE>), grid, dim3(256), 0, st, g, in, mask, w, b, out);
 }
 
 // inference of a two-layer network: one fused kernel, no workspace
@@ -1242,23 +1401,40 @@ void mask_pointwise_gradient(const pbrt_cnn* net, float* padded_grad, hipStream_
                        padded_grad + layer_offset(l), cin_pad(l));
 }
 
-// inference: kernel prediction fused into the last layer
-void forward_fused(const pbrt_cnn* net, const pbrt_cnn_images& im, const CnnWork& k, hipStream_t st) {
+// inference of three to six layers: the row pipeline, no workspace.  Strips are cut into
+// segments so that the workgroups (one per CU) fill whole rounds of the chip: of one to
+// eight rounds, the one with the fewest rows in all (a segment of r rows takes r + 3L + 2
+// steps with its halo and the pipeline's latency, an unfilled round idles CUs).
+template <int L>
+void launch_pipeline(const pbrt_cnn* net, const pbrt_cnn_images& im, hipStream_t st) {
     const CnnGeom g{(int)im.width, (int)im.height, (int)im.count};
-    const size_t px = (size_t)im.width * im.height * im.count;
-    hipLaunchKernelGGL(k_features, dim3((unsigned)((px + 255) / 256)), dim3(256), 0, st, g, im, k.feat);
-    const uint16_t* wf = net->wf.as<uint16_t>();
-    const float* master = net->master.as<float>();
-    const int layers = net->layers;
-    for (int l = 0; l < layers; ++l) {
-        const uint16_t* w = wf + weight_offset(l);
-        const float* b = master + layer_offset(l) + layer_weights(l);
-        if (l == 0)
-            launch_conv<kFeatCh, kConvRelu>(g, k.act[0], nullptr, w, b, k.act[1], st);
-        else if (l < layers - 1)
-            launch_conv<kCh, kConvRelu>(g, k.act[l], nullptr, w, b, k.act[l + 1], st);
-        else
-            launch_conv<kCh, kConvKpn>(g, k.act[l], nullptr, w, b, nullptr, st, im);
+    constexpr uint32_t out = kPipeCols - 2 * L;
+    const uint32_t strips_x = (im.width + out - 1) / out;
+    const uint64_t strips = (uint64_t)strips_x * im.count, cus = (uint64_t)compute_units();
+    PBRT_REQUIRE(strips < (1ull << 31), "pbrt_cnn_denoise: batch too large");
+    uint64_t best = ~0ull;
+    uint32_t rows = im.height;
+    for (uint64_t rounds = 1; rounds <= 8; ++rounds) {
+        const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(rounds * cus / strips, 1), im.height);
+        const uint64_t r = (im.height + want - 1) / want, n = (im.height + r - 1) / r;
+        const uint64_t cost = (strips * n + cus - 1) / cus * (r + 3 * L + 2);
+        if (cost < best) {
+            best = cost;
+            rows = (uint32_t)r;
+        }
+    }
+    rows = std::max(rows, (im.height + 65534) / 65535);
+    const dim3 grid((uint32_t)strips, (im.height + rows - 1) / rows);
+    hipLaunchKernelGGL(k_pipeline<L>, grid, dim3(pipe_threads(L)), 0, st, g, im, net->wf.as<uint16_t>(),
+                       net->master.as<float>(), (int)rows, (int)strips_x);
+}
+
+void forward_pipeline(const pbrt_cnn* net, const pbrt_cnn_images& im, hipStream_t st) {
+    switch (net->layers) {
+        case 3: launch_pipeline<3>(net, im, st); break;
+        case 4: launch_pipeline<4>(net, im, st); break;
+        case 5: launch_pipeline<5>(net, im, st); break;
+        default: launch_pipeline<6>(net, im, st); break;
     }
 }
 
@@ -1287,7 +1463,7 @@ void backward(const pbrt_cnn* net, const pbrt_cnn_images& im, const CnnWork& k, 
     const size_t px = (size_t)im.width * im.height * im.count;
     const int blocks = (int)((px + 255) / 256);
     const int layers = net->layers;
-    hipLaunchKernelGGL(k_kpn<true>, dim3(blocks), dim3(256), 0, st, g, im, k.act[layers], k.grad_act[0],
+    hipLaunchKernelGGL(k_kpn, dim3(blocks), dim3(256), 0, st, g, im, k.act[layers], k.grad_act[0],
                        k.loss_part);
     const int tiles = (int)(((im.width + kTile - 1) / kTile) * ((im.height + kTile - 1) / kTile) * im.count);
     const int rows = std::min(tiles, kWgradGrid);
@@ -1484,9 +1660,7 @@ extern "C" int32_t pbrt_cnn_denoise(const pbrt_cnn* net, const pbrt_cnn_images* 
             forward_two_layer(net, *im, st);
         } else {
             check_images(im, false, net->layers, "pbrt_cnn_denoise");
-            const CnnWork k =
-                layout(im->width, im->height, im->count, false, net->layers, static_cast<char*>(im->workspace));
-            forward_fused(net, *im, k, st);
+            forward_pipeline(net, *im, st);
         }
         PBRT_HIP(hipGetLastError());
     });
