@@ -312,6 +312,30 @@ def test_persistent_equals_megakernel(cuda, cfg1, w, h):
             assert a.tobytes() == b.tobytes(), f"{k} differs at {w}x{h} frame {frame}"
 
 
+@pytest.mark.parametrize("w,h", [(W, H), (61, 37), (1, 1), (200, 9), (9, 130), (512, 256), (520, 256), (640, 480)])
+@pytest.mark.parametrize("output", [capi.OUTPUT_DEMOD_ILLUMINATION_FLOAT, capi.OUTPUT_FINAL_IMAGE])
+def test_small_frame_tracer_equals_the_others(cuda, cfg1, w, h, output):
+    """Frames whose waves are all resident at once (512x256 is the largest on 256 CUs of 16
+    waves) are traced 32 pixels to a wave, shadow and next rays side by side; a counted
+    trace runs the tracer it names.  Both, and the persistent tracer on either side of
+    the limit, give the same bytes: every random draw and sum of a pixel is the same."""
+    gen, scene, _ = cfg1
+    for frame in (0, 5):
+        pc, _, _ = helpers.frame_push_constants(gen, w, h, frame, sample=frame)
+        images = []
+        for tracer, counted in ((capi.TRACER_MEGAKERNEL, False), (capi.TRACER_MEGAKERNEL, True),
+                                (capi.TRACER_PERSISTENT, False), (capi.TRACER_PERSISTENT, True)):
+            img = {k: cuda.full_like(v, 0.25 if v.is_floating_point() else 7)
+                   for k, v in helpers.gbuffer(cuda, w, h).items()}
+            cnt = cuda.zeros(6, dtype=cuda.int64, device="cuda") if counted else None
+            helpers.trace(cuda, scene, pc, img, w, h, max_depth=4, min_depth=1, tracer=tracer, output=output,
+                          counters=cnt)
+            images.append(helpers.to_np(img))
+        for other in images[1:]:
+            for k in images[0]:
+                assert images[0][k].tobytes() == other[k].tobytes(), f"{k} differs at {w}x{h} frame {frame}"
+
+
 def test_trace_timing_records_every_stage(cuda, cfg1):
     """pbrt_trace_timing_begin/_end: one segment per wavefront stage launch, positive times."""
     gen, scene, _ = cfg1

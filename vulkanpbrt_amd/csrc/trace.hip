@@ -156,6 +156,202 @@ pt_megakernel(DeviceScene sc, TraceConsts c, float* depth_img,
     }
 }
 
+// The images a path writes.
+struct PathImages {
+    float* depth;
+    float* normal;
+    uint8_t* material;
+    uint8_t* albedo;
+    float4* illum;
+};
+
+// A path between two walks (pt_pairs): the ray to walk next, the shadow ray of its last
+// vertex and the radiance for either outcome of it.
+struct PathState {
+    Rng re;
+    vec3 o, d;           // origin of both rays; direction of the next ray
+    vec3 ls;             // direction and tmax of the shadow ray
+    float ts;
+    bool shadow, next;   // which rays the path has
+    vec3 throughput;
+    vec3 lit, unlit;     // radiance so far if the shadow ray is unoccluded / occluded
+    vec3 albedo;         // of the primary hit
+    bool primary;        // the next ray is the camera ray
+    bool at_infinity;    // the last vertex lies at infinity (no demodulation)
+    int depth_i, trans_depth;
+};
+
+__device__ __forceinline__ void path_begin(const TraceConsts& c, uint32_t px, uint32_t py, PathState& p) {
+    const bool anti_alias = c.output == PBRT_OUTPUT_FINAL_IMAGE && c.sample_number > 0;
+    p.re = rng_init(px, py, c.frame_number);
+    create_ray(c, px, py, anti_alias, p.re, p.o, p.d);
+    p.throughput = make_vec3(1.0f);
+    p.lit = p.unlit = p.albedo = make_vec3(0.0f);
+    p.ls = make_vec3(0.0f);
+    p.ts = 0.0f;
+    p.shadow = false;
+    p.next = true;
+    p.primary = true;
+    p.depth_i = p.trans_depth = 0;
+}
+
+// One vertex of ptRaygen.rgen:24-104 at the end of the walked ray: surface, next-event
+// estimation (the shadow ray is left to the next walk, p.lit / p.unlit hold the radiance
+// for both outcomes), G-buffer on the primary hit, then the bounce loop's head
+// (indirectLighting, lighting.glsl:263-287): the next ray, or none when the path ends.
+__device__ __forceinline__ void path_vertex(const DeviceScene& sc, const TraceConsts& c, const PathImages& img,
+                                            size_t pix, const Hit& h, PathState& p) {
+    SurfaceInfo s;
+    vec3 pos;
+    uint32_t category;
+    if (h.tri != kNoHit)
+        shade_hit(sc, h, p.d, s, pos, category);
+    else
+        miss_surface(s, pos, category);
+    const bool miss = is_miss(s);
+    const vec3 out = p.primary ? -normalize(p.d) : -p.d;
+    // nextEventEsitmation (lighting.glsl:246-261); throughput is (1, 1, 1) on the primary
+    vec3 ne = make_vec3(0.0f);
+    p.shadow = false;
+    if (miss) {
+        ne = sky_color(-out) * p.throughput;
+    } else {
+        const LightSample l = sample_light(sc, c.light_sampling, pos, s.normal, p.re);
+        if (l.valid) {
+            p.shadow = true;
+            p.ls = l.l;
+            p.ts = l.tmax;
+            ne = nee_unshadowed(l, out, s, p.throughput);
+        }
+    }
+    const vec3 em = s.emissive_color * p.throughput;
+    p.unlit = p.lit + (make_vec3(0.0f) + em);
+    p.lit = p.lit + (ne + em);
+    p.at_infinity = isinf(pos.x);
+    if (p.primary) {
+        p.albedo = s.diffuse_color + s.specular_color;
+        if (c.write_gbuffer) {
+            img.depth[pix] = distance(pos, p.o);
+            img.normal[2 * pix + 0] = acosf(s.normal.z);
+            img.normal[2 * pix + 1] = atan2f(s.normal.y, s.normal.x);
+            uint8_t* mat = img.material + 4 * pix;
+            mat[0] = unorm8((float)category / 255.0f);
+            mat[1] = 0;
+            mat[2] = 0;
+            mat[3] = 0;
+            uint8_t* alb = img.albedo + 4 * pix;
+            alb[0] = unorm8(p.albedo.x);
+            alb[1] = unorm8(p.albedo.y);
+            alb[2] = unorm8(p.albedo.z);
+            alb[3] = 255;
+        }
+    } else {
+        ++p.depth_i;
+    }
+    p.primary = false;
+    p.next = false;
+    if (!miss && p.depth_i < (int)c.max_depth && p.trans_depth < 10) {
+        if (s.illumination_type == 7) {
+            --p.depth_i;
+            ++p.trans_depth;
+        }
+        const vec3 v = normalize(p.o - pos);
+        vec3 l;
+        float pdf;
+        const vec3 brdf = sample_brdf(s, p.re, v, l, pdf);
+        if (!(brdf == make_vec3(0.0f) || pdf < kEpsilon)) {
+            float tc = dot(l, s.normal);
+            if (s.illumination_type == 7) tc = 1.0f;
+            vec3 path_tp = p.throughput * (brdf * tc) / pdf;
+            p.next = true;
+            if ((uint32_t)p.depth_i > c.min_depth) {
+                if (rng_float(p.re) < kMinTermination)
+                    p.next = false;
+                else
+                    path_tp /= 1.0f - kMinTermination;
+            }
+            if (p.next) {
+                p.throughput = path_tp;
+                p.d = l;
+            }
+        }
+    }
+    p.o = pos;
+}
+
+// The finished path's pixel: clamp, then demodulated radiance or the progressive image.
+__device__ __forceinline__ void path_write(const TraceConsts& c, const PathImages& img, size_t pix,
+                                           const PathState& p) {
+    const vec3 color = vclamp(p.lit, 0.0f, kMaxRadiance);
+    if (c.output == PBRT_OUTPUT_DEMOD_ILLUMINATION_FLOAT) {
+        vec3 demod = color;
+        if (!p.at_infinity) demod = vmin(color / (p.albedo + make_vec3(kEpsilon)), 1e3f);
+        img.illum[pix] = make_float4(demod.x, demod.y, demod.z, 1.0f);
+    } else {
+        vec3 fc = color;
+        if (c.sample_number > 0) {
+            float4 prev = img.illum[pix];
+            float alpha = 1.0f / (float)(c.sample_number + 1);
+            vec3 pl = srgb_to_linear(make_vec3(prev.x, prev.y, prev.z));
+            fc = vmix(pl, fc, alpha);
+        }
+        fc = linear_to_srgb(fc);
+        fc = vclamp(fc, 0.0f, 1.0f);
+        img.illum[pix] = make_float4(fc.x, fc.y, fc.z, 1.0f);
+    }
+}
+
+constexpr uint32_t kPairX = 8, kPairY = 4;  // pixels of a wave of pt_pairs
+
+// The tracer of small frames, where the chip holds few waves and a frame takes as long as
+// its slowest wave's chain of walks: 32 pixels (8x4) per wave, lane l < 32 walking its
+// path's next ray while lane l + 32 walks the shadow ray of the vertex that ray leaves.
+// The chain is then one walk per vertex instead of two, and each waits for the longest of
+// 32 paths instead of 64.  The random draws and the radiance of a pixel are those of
+// pt_megakernel (the order of a vertex's draws does not depend on its shadow ray).
+//   At most 128 registers (four waves per SIMD, four of them spilled): with 141 the frames
+// of 110k to 131k pixels needed a second round of waves (480x270 589 us against 452).
+//   Megakernel and this, us per trace: Cornell box, 2 bounces: 96x72 280 -> 212, 256x256
+// 302 -> 226, 480x270 312 -> 257; atrium, 4 bounces: 160x90 445 -> 320, 384x216 518 -> 385;
+// city, 8 bounces: 480x270 686 -> 520.
+__global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4))) pt_pairs(DeviceScene sc, TraceConsts c, PathImages img) {
+    __shared__ int stack_mem[kTraversalStackSize * kTileThreads];
+    const uint32_t lane = threadIdx.x, l = lane & 31u;
+    const bool any = lane >= 32u;
+    int* stack = stack_mem + lane;
+    const uint32_t px = blockIdx.x * kPairX + l % kPairX, py = blockIdx.y * kPairY + l / kPairX;
+    const bool inside = px < c.width && py < c.height;
+    const size_t pix = (size_t)py * c.width + px;
+    TraversalCounters cnt{0, 0};
+    PathState p;
+    path_begin(c, inside ? px : 0u, inside ? py : 0u, p);
+    p.next = inside;
+    bool alive = inside && !any;
+    while (__any(alive)) {
+        // lane l + 32 takes the shadow ray of lane l
+        const vec3 o = make_vec3(__shfl(p.o.x, (int)l), __shfl(p.o.y, (int)l), __shfl(p.o.z, (int)l));
+        const vec3 ls = make_vec3(__shfl(p.ls.x, (int)l), __shfl(p.ls.y, (int)l), __shfl(p.ls.z, (int)l));
+        const float ts = __shfl(p.ts, (int)l);
+        const int want = __shfl(p.shadow ? 1 : 0, (int)l);
+        Hit h;
+        h.tri = kNoHit;
+        bool hit = false;
+        if (any ? want != 0 : alive && p.next)
+            hit = walk<false, 1>(sc, o, any ? ls : p.d, 0.001f, any ? ts : 10000.0f, any, h, stack, kTileThreads, cnt);
+        const unsigned long long hits = __ballot(hit);
+        if (alive) {
+            if (p.shadow && (hits >> (l + 32u) & 1ull)) p.lit = p.unlit;
+            if (p.next) {
+                path_vertex(sc, c, img, pix, h, p);
+            } else {
+                path_write(c, img, pix, p);
+                p.shadow = false;
+                alive = false;
+            }
+        }
+    }
+}
+
 // Pixel of the id-th path of a frame: the frame is cut into bands of 8 rows and
 // each band into tiles of 8 columns (narrower at the right edge, shorter in the
 // last band); ids run tile by tile, row-major inside a tile, so consecutive ids
@@ -389,25 +585,22 @@ using namespace pbrt;
 
 namespace {
 
-// Workgroups of the persistent tracer: as many as stay resident on the current
-// device at once (occupancy of the kernel variant times the compute units).
-uint32_t persistent_waves(bool counting) {
+// Workgroups of one wave of `kernel` that stay resident on the current device at once
+// (its occupancy times the compute units).
+template <class K>
+uint32_t resident_waves(K kernel) {
     int dev = 0;
     PBRT_HIP(hipGetDevice(&dev));
     static std::mutex m;
-    static std::map<std::pair<int, bool>, uint32_t> cache;
+    static std::map<std::pair<int, const void*>, uint32_t> cache;
     std::lock_guard<std::mutex> lock(m);
-    auto it = cache.find({dev, counting});
+    const std::pair<int, const void*> key{dev, reinterpret_cast<const void*>(kernel)};
+    auto it = cache.find(key);
     if (it != cache.end()) return it->second;
     int per_cu = 0, cus = 0;
-    if (counting)
-        PBRT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pt_persistent<true>, kTileThreads, 0));
-    else
-        PBRT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pt_persistent<false>, kTileThreads, 0));
+    PBRT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kTileThreads, 0));
     PBRT_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const uint32_t n = (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, cus);
-    cache[{dev, counting}] = n;
-    return n;
+    return cache[key] = (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, cus);
 }
 
 }  // namespace
@@ -444,15 +637,27 @@ extern "C" int32_t pbrt_trace(const pbrt_scene* scene, const pbrt_trace_params* 
         c.output = p->output;
         c.write_gbuffer = p->write_gbuffer;
         dim3 grid((p->width + kTileX - 1) / kTileX, (p->height + kTileY - 1) / kTileY);
+        const dim3 pair_grid((p->width + kPairX - 1) / kPairX, (p->height + kPairY - 1) / kPairY);
         hipStream_t st = (hipStream_t)stream;
         float4* illum = reinterpret_cast<float4*>(img->illumination);
         TraceTiming* tm = scene_timing(scene);
         if (p->tracer == PBRT_TRACER_WAVEFRONT) {
             wavefront_trace(sc, c, *img, counters, tm, p->block_threads, p->queue_paths, st);
+        } else if (!counters && (uint64_t)pair_grid.x * pair_grid.y <= resident_waves(pt_pairs)) {
+            // The whole frame's pairs of walks are resident at once: its time is its longest
+            // path's, which pt_pairs shortens.  Past that (131,072 pixels here) a second
+            // round of waves costs more than the pairs save: atrium 480x270 547 -> 452 us,
+            // 512x288 559 -> 606.  Counted traces keep the tracer they name, whose
+            // traversal counts they report.
+            const PathImages images{img->depth, img->normal, img->material, img->albedo, illum};
+            if (tm) tm->frame_begin(st);
+            hipLaunchKernelGGL(pt_pairs, pair_grid, dim3(kTileThreads), 0, st, sc, c, images);
+            if (tm) tm->mark(kTimeMegakernel, st);
         } else if (p->tracer == PBRT_TRACER_PERSISTENT) {
             const uint32_t pixels = p->width * p->height;
             const uint32_t waves =
-                std::min(persistent_waves(counters != nullptr), (pixels + kTileThreads - 1) / kTileThreads);
+                std::min(counters ? resident_waves(pt_persistent<true>) : resident_waves(pt_persistent<false>),
+                         (pixels + kTileThreads - 1) / kTileThreads);
             uint32_t* work = scene_work_counter(scene);
             if (tm) tm->frame_begin(st);
             if (counters)

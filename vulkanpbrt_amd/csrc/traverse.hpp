@@ -190,13 +190,13 @@ __device__ __forceinline__ int pop_node(const int* stack, int stride, int& sp) {
 //   sel_z0 and derives the other two per node (2 operations), for the persistent
 //   kernel, whose occupancy two more registers would lower.
 //   kPlanes 0: all twelve planes formed and ordered by min / max.
-//   kOrdered: closest-hit walks take the nearer child first; any-hit (shadow) walks
+//   any: closest-hit walks take the nearer child first; any-hit (shadow) walks
 //   the farther one, since an occluder tends to lie toward the light rather than
 //   next to the surface the ray leaves (atrium: 25.2 node visits per shadow ray
 //   against 26.4 nearer-first and 25.9 in stored order).
-template <int kPlanes, bool kOrdered = true>
+template <int kPlanes>
 __device__ __forceinline__ int visit_inner(const uint4* __restrict__ nodes, int node, const TraversalRay& r,
-                                           float tcur, int* stack, int stride, int& sp) {
+                                           float tcur, int* stack, int stride, int& sp, bool any) {
     // a 32-bit byte offset from the array's base (node indices stay below 2^27), so
     // the loads take the scalar-base addressing form
     const char* base = reinterpret_cast<const char*>(nodes);
@@ -246,7 +246,7 @@ __device__ __forceinline__ int visit_inner(const uint4* __restrict__ nodes, int 
     int ch0 = (int)na.w;
     int ch1 = (int)nb.w;
     if (h0 && h1) {
-        bool swap = kOrdered ? near1 < near0 : near1 > near0;
+        const bool swap = any ? near1 > near0 : near1 < near0;
         stack[sp * stride] = swap ? ch0 : ch1;
         ++sp;
         return swap ? ch1 : ch0;
@@ -268,8 +268,8 @@ __device__ __forceinline__ bool wins_tie(const float4* __restrict__ tris, uint32
 // The triangles of one leaf (Moller-Trumbore, alpha test on alpha-tested
 // instances); closest hit keeps the nearest accepted t, any-hit returns true on
 // the first accepted candidate.
-template <bool kAnyHit, bool kCount>
-__device__ __forceinline__ bool test_leaf(const DeviceScene& sc, int node, const TraversalRay& r, Hit& hit,
+template <bool kCount>
+__device__ __forceinline__ bool test_leaf(const DeviceScene& sc, int node, const TraversalRay& r, Hit& hit, bool any,
                                           TraversalCounters& cnt) {
     const float4* __restrict__ tris = sc.tris;
     const vec3 o = r.o, d = r.d;
@@ -295,7 +295,7 @@ __device__ __forceinline__ bool test_leaf(const DeviceScene& sc, int node, const
         float v = dot(d, qv) * inv;
         if (!(v >= 0.0f && u + v <= 1.0f)) continue;
         float t = dot(e2, qv) * inv;
-        if constexpr (kAnyHit) {
+        if (any) {
             if (!(t >= r.tmin && t < hit.t)) continue;
         } else {
             // at exactly the current t the lower (instance, primitive) wins, so the
@@ -312,7 +312,7 @@ __device__ __forceinline__ bool test_leaf(const DeviceScene& sc, int node, const
         hit.tri = k;
         hit.u = u;
         hit.v = v;
-        if (kAnyHit) return true;
+        if (any) return true;
     }
     return false;
 }
@@ -324,9 +324,10 @@ __device__ __forceinline__ bool test_leaf(const DeviceScene& sc, int node, const
 // instead of interleaving with node visits.  The triangles tested are those of
 // the plain nearest-child-first walk; only the order of leaves can differ, which
 // changes nothing but the choice among hits at exactly equal t.
-template <bool kAnyHit, bool kCount, int kPlanes = 1>
-__device__ bool traverse(const DeviceScene& sc, vec3 o, vec3 d, float tmin, float tmax, Hit& hit, int* stack,
-                         int stride, TraversalCounters& cnt) {
+//   `any`: any-hit walk (true on the first accepted candidate).
+template <bool kCount, int kPlanes>
+__device__ __forceinline__ bool walk(const DeviceScene& sc, vec3 o, vec3 d, float tmin, float tmax, bool any, Hit& hit,
+                                     int* stack, int stride, TraversalCounters& cnt) {
     const TraversalRay r = make_traversal_ray(o, d, tmin);
     hit.tri = kNoHit;
     hit.t = tmax;
@@ -336,7 +337,7 @@ __device__ bool traverse(const DeviceScene& sc, vec3 o, vec3 d, float tmin, floa
     while (node != kNodeDone || leaf != 0) {
         while (node >= 0) {
             if (kCount) cnt.nodes++;
-            node = visit_inner<kPlanes, !kAnyHit>(sc.nodes, node, r, hit.t, stack, stride, sp);
+            node = visit_inner<kPlanes>(sc.nodes, node, r, hit.t, stack, stride, sp, any);
             if (node < 0 && node != kNodeDone && leaf == 0) {
                 leaf = node;
                 node = pop_node(stack, stride, sp);
@@ -348,7 +349,7 @@ __device__ bool traverse(const DeviceScene& sc, vec3 o, vec3 d, float tmin, floa
         }
         const int lf = leaf != 0 ? leaf : (node != kNodeDone ? node : 0);
         if (lf != 0) {
-            if (test_leaf<kAnyHit, kCount>(sc, lf, r, hit, cnt)) return true;
+            if (test_leaf<kCount>(sc, lf, r, hit, any, cnt) && any) return true;
             if (leaf != 0)
                 leaf = 0;
             else
@@ -356,6 +357,13 @@ __device__ bool traverse(const DeviceScene& sc, vec3 o, vec3 d, float tmin, floa
         }
     }
     return hit.tri != kNoHit;
+}
+
+// The walk of one kind of ray (all lanes any-hit, or none).
+template <bool kAnyHit, bool kCount, int kPlanes = 1>
+__device__ bool traverse(const DeviceScene& sc, vec3 o, vec3 d, float tmin, float tmax, Hit& hit, int* stack,
+                         int stride, TraversalCounters& cnt) {
+    return walk<kCount, kPlanes>(sc, o, d, tmin, tmax, kAnyHit, hit, stack, stride, cnt);
 }
 
 // ---------------------------------------------------------------------------
