@@ -391,7 +391,7 @@ enum pbrt_bmfr_fit {
      * sky blocks cond(A^T A) reaches 1e10 and the fit error grows to ~1e-1. */
     PBRT_BMFR_FIT_GRAM_F16 = 1,
     /* as PBRT_BMFR_FIT_GRAM_F16 but the Gram matrix is accumulated by FP64 MFMA
-     * (v_mfma_f64_16x16x4f64) from the fp32 projected columns; fitted values
+     * (v_mfma_f64_4x4x4f64) from the fp32 projected columns; fitted values
      * stay within ~1e-5 of the FP64 least-squares solution on every block. */
     PBRT_BMFR_FIT_GRAM_F64 = 2
 };
@@ -404,7 +404,8 @@ typedef struct pbrt_bmfr_params {
     uint32_t fit;            /* enum pbrt_bmfr_fit */
     uint32_t fit_threads;    /* Gram fits: workgroup size 256, 512 or 1024 (0 = 256), i.e. how a
                                 block's rows are tiled over the waves' MFMA Gram accumulations;
-                                pbrt_autotune_bmfr picks it */
+                                pbrt_autotune_bmfr picks it.  At 0 and 256 the FP64 fit of 16- and
+                                8-pixel blocks runs one wave per block. */
     uint32_t reserved[2];
 } pbrt_bmfr_params;
 
@@ -464,8 +465,8 @@ int32_t pbrt_autotune_bmfr(const pbrt_bmfr_params* params, const pbrt_bmfr_image
  * one launch and post-processed in a second, instead of one BMFR dispatch chain
  * per frame (BMFR::add_dispatch_to_command_graph, BMFR.cpp:206-229).  All frames
  * share block_size and fit, and the fit is PBRT_BMFR_FIT_GRAM_F16 or _F64 (the
- * Householder path stages features per frame); the batch fits with 256-thread
- * workgroups whatever fit_threads says.  images.workspace of each frame
+ * Householder path stages features per frame); the batch fits with the
+ * default workgroups whatever fit_threads says.  images.workspace of each frame
  * is ignored: the batch workspace holds the frame table and every frame's
  * weights.  The frame table is staged through a pinned host buffer owned by the
  * library; a call waits only for the previous call's table upload. */

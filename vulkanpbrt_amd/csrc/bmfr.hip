@@ -12,7 +12,7 @@
 //   k_bmfr_fit_householder   the reference's FP32 Householder QR over the fp16
 //                            feature buffer, subgroup reductions on wave64
 //   k_bmfr_fit_gram<F64>     pre + fit fused, features in registers: the Gram matrix
-//                            of the raw columns on v_mfma_f64_16x16x4f64, the
+//                            of the raw columns on v_mfma_f64_4x4x4f64, the
 //                            projection against the noised constant column a0 as a
 //                            rank-1 downdate in FP64, equilibrated FP64 elimination
 //   k_bmfr_fit_gram<F16>     the columns projected against a0 in FP64 per row, scaled
@@ -116,6 +116,8 @@ __device__ __forceinline__ uint32_t dpp_u32(uint32_t v, int ctrl) {
         case 0xB1: return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, false);   // quad_perm 1,0,3,2
         case 0x4E: return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, false);   // quad_perm 2,3,0,1
         case 0x141: return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, false); // row_half_mirror
+        case 0x124: return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x124, 0xF, 0xF, false); // row_ror 4
+        case 0x128: return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, false); // row_ror 8
         default: return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x140, 0xF, 0xF, false);   // row_mirror
     }
 }
@@ -372,6 +374,14 @@ typedef double double4v __attribute__((ext_vector_type(4)));
 
 constexpr int kGramCols = 16;  // 13 columns (FP64: a0, 9 features, rgb; FP16: 9 projected features, rgb) + zeros
 constexpr int kFitThreads = 256;
+
+// Workgroup size of a Gram fit: as asked (256 by default), except that the FP64 fit of 16-
+// and 8-pixel blocks runs one wave per block by default: their 256 and 64 rows leave four
+// waves one row a lane or none, and one wave needs no barrier.  1920x1080, whole BMFR:
+// 16-pixel blocks 76 -> 61 us, 8-pixel blocks 192 -> 91 us.
+__host__ __device__ constexpr int gram_threads(bool f64, int bs, uint32_t asked) {
+    return f64 && bs < 32 && (asked == 0 || asked == 256) ? 64 : asked ? (int)asked : kFitThreads;
+}
 
 // FP16 fit: wave-private staging of 64 rows (one per lane) as column-major fp16 hi / lo
 // planes, the per-wave partial Gram matrices, and the per-wave partial sums of the
@@ -665,7 +675,7 @@ __device__ __forceinline__ void bmfr_fit_gram_f16_block(const BmfrGeom& g, const
 // reductions, solve) uncovered, and with four a block whose wave 0 is still solving
 // keeps the CU from starting the next block.
 // The FP64 fit.  The Gram matrix R of the raw columns [a0 | a1..a9 | r g b] (fp32
-// values: their products are exact in FP64) is accumulated on v_mfma_f64_16x16x4f64;
+// values: their products are exact in FP64) is accumulated on v_mfma_f64_4x4x4f64;
 // the normal equations of the features projected against the noised constant column
 // a0 follow in FP64 by the rank-1 downdate G = R[1:,1:] - R[0,1:] R[0,1:]^T / R[0,0].
 // The 9 x 9 feature block of G is equilibrated by its diagonal and solved for the three
@@ -677,12 +687,14 @@ __device__ __forceinline__ void bmfr_fit_gram_f16_block(const BmfrGeom& g, const
 // block reductions beyond the depth range.
 template <int kWaves>
 struct RawGramShared {
-    float st[kWaves][64][kGramCols + 1];  // wave-private rows (odd stride: no bank conflicts)
-    double gram[kWaves][kGramCols * kGramCols];
+    // wave-private rows, 20 floats apart: 16-byte writes of one row per lane and the
+    // operand reads (lane l: row l / 4, column l % 4 of a group) meet no bank twice
+    __attribute__((aligned(16))) float st[kWaves][64][20];
+    double gram[kWaves][kGramCols * kGramCols];  // upper triangle
     float depth_min[kWaves], depth_max[kWaves];
     float coord[32];
     double r0[kAlphaSize];  // row 0 of R: a0 . a_c
-    double G[12][12];       // projected normal equations (9 features | 3 colours)
+    double G[kFeatures - 1][12];  // projected normal equations (9 features | 3 colours)
     double eq[kFeatures - 1];  // equilibration 1 / sqrt(G_ii)
 };
 
@@ -774,51 +786,70 @@ __device__ __forceinline__ void bmfr_fit_raw_gram_block(const BmfrGeom& g, const
         }
     }
     // 3. R = A^T A on the matrix cores, 64 rows at a time through the wave's own LDS
-    //    slice (lane l stages its row of chunk s); both operands of the product hold
-    //    the same values (lane l: column l % 16 of a group of four rows)
+    //    slice (lane l stages its row of chunk s).  v_mfma_f64_4x4x4f64 forms four 4x4
+    //    products of four rows each; here all four are the same pair of column groups
+    //    over four times as many rows, so the groups [a0 a1..a3 | a4..a7 | a8 a9 r g | b]
+    //    take the nine pairs R needs (the upper triangle without b's own) where a
+    //    16x16 product forms all sixteen: 9 x 16 cycles per 16 rows against 4 x 64.
+    //    Both operands hold the same values (lane l: row l / 4, column l % 4 of a group).
+    //    1920x1080, whole BMFR: 63.5 -> 57.5 us.
     {
-        const int col = lane & 15, grp = lane >> 4;
-        // two accumulators: even and odd row groups form independent MFMA chains
-        double4v d = {0.0, 0.0, 0.0, 0.0}, d1 = {0.0, 0.0, 0.0, 0.0};
+        constexpr int kPairs = 9;
+        constexpr int gi[kPairs] = {0, 0, 0, 0, 1, 1, 1, 2, 2}, gj[kPairs] = {0, 1, 2, 3, 1, 2, 3, 2, 3};
+        double acc[kPairs];
+#pragma unroll
+        for (int k = 0; k < kPairs; ++k) acc[k] = 0.0;
 #pragma unroll
         for (int s = 0; s < kSub; ++s) {
             if (s > 0) wave_lds_sync();  // the previous chunk has been read
+            float* dst = S.st[wave][lane];
+            if (row[s] < 0) {
 #pragma unroll
-            for (int c = 0; c < kGramCols; ++c) S.st[wave][lane][c] = (c < kAlphaSize && row[s] >= 0) ? a[s][c] : 0.0f;
+                for (int c = 0; c < kAlphaSize; ++c) a[s][c] = 0.0f;
+            }
+#pragma unroll
+            for (int c = 0; c < 12; c += 4)
+                *reinterpret_cast<float4*>(dst + c) = make_float4(a[s][c], a[s][c + 1], a[s][c + 2], a[s][c + 3]);
+            dst[12] = a[s][12];  // the columns past it reach only unused entries
             wave_lds_sync();
 #pragma unroll
-            for (int ch = 0; ch < 16; ch += 2) {
-                const double x0 = (double)S.st[wave][ch * 4 + grp][col];
-                const double x1 = (double)S.st[wave][ch * 4 + 4 + grp][col];
-                d = __builtin_amdgcn_mfma_f64_16x16x4f64(x0, x0, d, 0, 0, 0);
-                d1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x1, x1, d1, 0, 0, 0);
+            for (int ch = 0; ch < 4; ++ch) {
+                const float* src = &S.st[wave][ch * 16 + (lane >> 2)][lane & 3];
+                double x[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) x[q] = (double)src[4 * q];
+#pragma unroll
+                for (int k = 0; k < kPairs; ++k)
+                    acc[k] = __builtin_amdgcn_mfma_f64_4x4x4f64(x[gi[k]], x[gj[k]], acc[k], 0, 0, 0);
             }
         }
-        d += d1;
-        // register i of v_mfma_f64_16x16x4f64's result is row grp + 4 * i, column `col`
+        // lane 16 i + 4 b + j holds entry (i, j) of product b: summed over b
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S.gram[wave][(grp + 4 * i) * kGramCols + col] = d[i];
+        for (int k = 0; k < kPairs; ++k) {
+            acc[k] += dpp_move(acc[k], 0x128);  // row_ror 8
+            acc[k] += dpp_move(acc[k], 0x124);  // row_ror 4
+            if ((lane & 12) == 0)
+                S.gram[wave][(4 * gi[k] + (lane >> 4)) * kGramCols + 4 * gj[k] + (lane & 3)] = acc[k];
+        }
     }
     __syncthreads();
-    // 4. R summed over the waves and symmetrised; G by the rank-1 downdate
+    // 4. R summed over the waves; G by the rank-1 downdate
     constexpr int pw = kGramCols * kGramCols;
     const double* gr = &S.gram[0][0];
-    auto rsum = [&](int i, int j) {
-        double a_ij = 0.0, a_ji = 0.0;
+    auto rsum = [&](int i, int j) {  // i <= j
+        double r = gr[i * kGramCols + j];
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) {
-            a_ij += gr[w * pw + i * kGramCols + j];
-            a_ji += gr[w * pw + j * kGramCols + i];
-        }
-        return 0.5 * (a_ij + a_ji);
+        for (int w = 1; w < kWaves; ++w) r += gr[w * pw + i * kGramCols + j];
+        return r;
     };
     const double r00 = rsum(0, 0), inv_r00 = 1.0 / r00;
-    for (int e = tid; e < 12 * 12 + kAlphaSize; e += kThreads) {
-        if (e < 12 * 12) {
+    constexpr int kEntries = (kFeatures - 1) * 12;  // feature rows, feature and colour columns
+    for (int e = tid; e < kEntries + kAlphaSize; e += kThreads) {
+        if (e < kEntries) {
             const int i = e / 12 + 1, j = e % 12 + 1;
-            S.G[i - 1][j - 1] = rsum(i, j) - rsum(0, i) * rsum(0, j) * inv_r00;
+            S.G[i - 1][j - 1] = rsum(min(i, j), max(i, j)) - rsum(0, i) * rsum(0, j) * inv_r00;
         } else {
-            S.r0[e - 12 * 12] = rsum(0, e - 12 * 12);
+            S.r0[e - kEntries] = rsum(0, e - kEntries);
         }
     }
     __syncthreads();
@@ -827,7 +858,7 @@ __device__ __forceinline__ void bmfr_fit_raw_gram_block(const BmfrGeom& g, const
     //    by the feature rows' factor only), solved in wave 0
     constexpr int n = kFeatures - 1;
     const int lj = lane < 12 ? lane : 0;
-    const double gjj = S.G[lj][lj];
+    const double gjj = S.G[lj < n ? lj : 0][lj];
     const double eqj = lj < n ? (gjj > 0.0 ? 1.0 / sqrt(gjj) : 0.0) : 1.0;
     if (lane < n) S.eq[lane] = eqj;
     wave_lds_sync();
@@ -875,7 +906,7 @@ __device__ __forceinline__ void grid_block(const BmfrGeom& g, int& bx, int& by) 
 }
 
 template <int kRows, bool kF64, int kThreads>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kF64 && kThreads == 256 ? 5 : 4)))
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kF64 && kThreads <= 256 ? 5 : 4)))
 k_bmfr_fit_gram(BmfrGeom g, pbrt_bmfr_images im) {
     int bx, by;
     grid_block(g, bx, by);
@@ -984,8 +1015,8 @@ __device__ __forceinline__ uint32_t batch_frame_of(const BmfrBatchFrame* frames,
     return lo;
 }
 
-template <int kRows, bool kF64>
-__global__ void __launch_bounds__(kFitThreads) __attribute__((amdgpu_waves_per_eu(kF64 ? 5 : 4)))
+template <int kRows, bool kF64, int kThreads>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kF64 ? 5 : 4)))
 k_bmfr_fit_gram_batched(const BmfrBatchFrame* frames, uint32_t n) {
     const uint32_t b = xcd_contiguous(blockIdx.x, gridDim.x);
     const uint32_t f = batch_frame_of(frames, n, b);
@@ -994,16 +1025,16 @@ k_bmfr_fit_gram_batched(const BmfrBatchFrame* frames, uint32_t n) {
     const uint32_t local = b - frames[f].first_block;
     const int bx = (int)(local % (uint32_t)g.blocks_x), by = (int)(local / (uint32_t)g.blocks_x);
     if constexpr (kF64)
-        bmfr_fit_raw_gram_block<kRows, kFitThreads>(g, im, bx, by);
+        bmfr_fit_raw_gram_block<kRows, kThreads>(g, im, bx, by);
     else
-        bmfr_fit_gram_f16_block<kRows, kFitThreads>(g, im, bx, by);
+        bmfr_fit_gram_f16_block<kRows, kThreads>(g, im, bx, by);
 }
 
 // the noise table of every frame of a batch (blockIdx.y: frame)
-__global__ void __launch_bounds__(256) k_bmfr_noise_batched(const BmfrBatchFrame* frames) {
+__global__ void __launch_bounds__(256) k_bmfr_noise_batched(const BmfrBatchFrame* frames, int threads) {
     const BmfrGeom& g = frames[blockIdx.y].g;
     const int e = blockIdx.x * 256 + threadIdx.x;
-    if (e < kFeatures * g.bs * g.bs) noise_table_entry(g.frame, g.bs, kFitThreads, e, g.noise);
+    if (e < kFeatures * g.bs * g.bs) noise_table_entry(g.frame, g.bs, threads, e, g.noise);
 }
 
 template <int kBs>  // one block size per batch
@@ -1073,7 +1104,12 @@ static void launch_gram_rows(int bs, dim3 grid, hipStream_t st, const BmfrGeom& 
 template <bool kF64>
 static void launch_gram_threads(int bs, uint32_t threads, dim3 grid, hipStream_t st, const BmfrGeom& g,
                                 const pbrt_bmfr_images& im) {
-    if (threads == 1024)
+    if (kF64 && threads == 64) {
+        if (bs == 16)
+            hipLaunchKernelGGL((k_bmfr_fit_gram<256, kF64, 64>), grid, dim3(64), 0, st, g, im);
+        else
+            hipLaunchKernelGGL((k_bmfr_fit_gram<64, kF64, 64>), grid, dim3(64), 0, st, g, im);
+    } else if (threads == 1024)
         launch_gram_rows<kF64, 1024>(bs, grid, st, g, im);
     else if (threads == 512)
         launch_gram_rows<kF64, 512>(bs, grid, st, g, im);
@@ -1121,7 +1157,7 @@ static void launch_bmfr(const pbrt_bmfr_params& p, const pbrt_bmfr_images& im, B
             hipLaunchKernelGGL((k_bmfr_fit_householder<1, 1>), grid, dim3(64), 0, st, g);
     } else {
         const int entries = kFeatures * g.bs * g.bs;
-        const int threads = (int)(p.fit_threads ? p.fit_threads : kFitThreads);
+        const int threads = gram_threads(p.fit == PBRT_BMFR_FIT_GRAM_F64, g.bs, p.fit_threads);
         hipLaunchKernelGGL(k_bmfr_noise, dim3((entries + 255) / 256), dim3(256), 0, st, g.frame, g.bs, threads,
                            g.noise);
         launch_gram_fit(p.fit == PBRT_BMFR_FIT_GRAM_F64, g.bs, (uint32_t)threads, grid, st, g, im);
@@ -1365,23 +1401,15 @@ extern "C" int32_t pbrt_bmfr_batched(const pbrt_bmfr_batch_frame* frames, uint32
         const dim3 grid(plan.blocks);
         const bool f64 = plan.fit == PBRT_BMFR_FIT_GRAM_F64;
         const int entries = kFeatures * plan.bs * plan.bs;
-        hipLaunchKernelGGL(k_bmfr_noise_batched, dim3((entries + 255) / 256, count), dim3(256), 0, st, table);
-        if (plan.bs == 32) {
-            if (f64)
-                hipLaunchKernelGGL((k_bmfr_fit_gram_batched<1024, true>), grid, dim3(kFitThreads), 0, st, table, count);
-            else
-                hipLaunchKernelGGL((k_bmfr_fit_gram_batched<1024, false>), grid, dim3(kFitThreads), 0, st, table, count);
-        } else if (plan.bs == 16) {
-            if (f64)
-                hipLaunchKernelGGL((k_bmfr_fit_gram_batched<256, true>), grid, dim3(kFitThreads), 0, st, table, count);
-            else
-                hipLaunchKernelGGL((k_bmfr_fit_gram_batched<256, false>), grid, dim3(kFitThreads), 0, st, table, count);
-        } else {
-            if (f64)
-                hipLaunchKernelGGL((k_bmfr_fit_gram_batched<64, true>), grid, dim3(kFitThreads), 0, st, table, count);
-            else
-                hipLaunchKernelGGL((k_bmfr_fit_gram_batched<64, false>), grid, dim3(kFitThreads), 0, st, table, count);
-        }
+        const int threads = gram_threads(f64, plan.bs, 0);
+        hipLaunchKernelGGL(k_bmfr_noise_batched, dim3((entries + 255) / 256, count), dim3(256), 0, st, table, threads);
+        auto fit = f64 ? (plan.bs == 32   ? k_bmfr_fit_gram_batched<1024, true, 256>
+                          : plan.bs == 16 ? k_bmfr_fit_gram_batched<256, true, 64>
+                                          : k_bmfr_fit_gram_batched<64, true, 64>)
+                       : (plan.bs == 32   ? k_bmfr_fit_gram_batched<1024, false, 256>
+                          : plan.bs == 16 ? k_bmfr_fit_gram_batched<256, false, 256>
+                                          : k_bmfr_fit_gram_batched<64, false, 256>);
+        hipLaunchKernelGGL(fit, grid, dim3(threads), 0, st, table, count);
         const int rows = post_rows(plan.bs);
         const dim3 post_grid(plan.blocks * (uint32_t)(plan.bs / rows)), post_block(plan.bs * rows);
         if (plan.bs == 32)
