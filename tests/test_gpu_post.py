@@ -381,3 +381,45 @@ def test_non_finite_pixels_stay_in_their_block(cuda, oracle_lib, frames, which, 
     assert far.mean() > 0.5
     assert np.array_equal(clean[0][:, far], dirty[0][:, far]) and np.array_equal(clean[1][far], dirty[1][far])
     assert not np.array_equal(clean[0][0], dirty[0][0])
+
+
+def test_reprojection_far_outside_the_image_wraps(cuda, oracle_lib, frames):
+    """BMFR's temporal fetch repeats the previous image wherever the motion points: just
+    inside and outside its borders (one wrap), many images away (the general remainder),
+    up to the largest fp16 value."""
+    inp = bmfr_inputs(oracle_lib, frames)
+    rng = np.random.default_rng(11)
+    uv = rng.uniform(0, 1.2, (H, W, 2))
+    uv[: H // 3] = rng.uniform(0, 30, (H // 3, W, 2))
+    uv[:, : W // 4, 1] *= -1  # only x decides whether a pixel was reprojected
+    uv[0, :8, 0] = [0, 1, 0.5 / W, 1 - 0.5 / W, 1 + 0.5 / W, 2, 65504, -1]
+    uv[1, :8, 1] = [0, 1, 0.5 / H, 1 - 0.5 / H, -0.5 / H, -1, -65504, 65504]
+    inp["motion"] = half(uv)
+    denoised = half(rng.uniform(0, 2, (2, H, W, 4)))
+    _, weights, den, final = run_bmfr(cuda, capi.BMFR_FIT_HOUSEHOLDER, 32, 1, inp, denoised)
+    oden, ofinal = oracle_lib.bmfr_post(W, H, 32, 1, inp["depth"], inp["normal"], inp["albedo"], inp["motion"],
+                                        inp["spp"], inp["noisy"], weights, denoised)
+    d_ok = np.isclose(unhalf(den[0]), unhalf(oden[0]), rtol=2e-3, atol=1e-3).all(-1)
+    f_ok = (np.abs(final.astype(int) - ofinal.astype(int)) <= 1).all(-1)
+    assert d_ok.mean() > 0.999 and f_ok.mean() > 0.999
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (1, 40), (16, 2), (17, 33), (50, 16)])
+def test_taa_at_image_borders(cuda, oracle_lib, w, h):
+    """The neighbourhood of border pixels holds only the image's pixels (tiles of 16 with a
+    one-pixel halo): frames narrower than a tile, one past it, single pixels."""
+    rng = np.random.default_rng(w * 100 + h)
+    motion = half(rng.uniform(-0.1, 1.1, (h, w, 2)))
+    den = rng.integers(0, 256, (h, w, 4), dtype=np.uint8)
+    hist = np.clip(den.astype(int) + rng.integers(-30, 31, den.shape), 0, 255).astype(np.uint8)[..., [2, 1, 0, 3]]
+    hist = np.ascontiguousarray(hist)
+    m, d, hh = dev(cuda, motion), dev(cuda, den), dev(cuda, hist)
+    out = cuda.zeros((h, w, 4), dtype=cuda.uint8, device="cuda")
+    capi.check(capi.lib().pbrt_taa(w, h, 1, C.byref(capi.TaaImages(*(capi.ptr(x) for x in (m, d, hh, out)))),
+                                   helpers.stream(cuda)))
+    cuda.cuda.synchronize()
+    ref = oracle_lib.taa(w, h, 1, motion, den, hist)
+    ref = ref[0] if isinstance(ref, tuple) else ref
+    # a neighbourhood test at exactly its bound may fall either way on a rounding
+    assert (np.abs(out.cpu().numpy().astype(int) - ref.astype(int)) <= 1).all(-1).mean() >= 0.99
+    assert np.array_equal(hh.cpu().numpy(), out.cpu().numpy())

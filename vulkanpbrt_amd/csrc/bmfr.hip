@@ -692,7 +692,6 @@ struct RawGramShared {
     __attribute__((aligned(16))) float st[kWaves][64][20];
     double gram[kWaves][kGramCols * kGramCols];  // upper triangle
     float depth_min[kWaves], depth_max[kWaves];
-    float coord[32];
     double r0[kAlphaSize];  // row 0 of R: a0 . a_c
     double G[kFeatures - 1][12];  // projected normal equations (9 features | 3 colours)
     double eq[kFeatures - 1];  // equilibration 1 / sqrt(G_ii)
@@ -705,22 +704,22 @@ __device__ __forceinline__ void bmfr_fit_raw_gram_block(const BmfrGeom& g, const
     constexpr int kWaves = kThreads / 64;
     __shared__ RawGramShared<kWaves> S;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int bs = g.bs;
+    // the block size follows from the rows, so a pixel's place in its block is a shift and
+    // a mask (by the run-time size they were an integer division and a remainder per pixel;
+    // with the bilinear fetch's, 1920x1080 BMFR 57.5 -> 54.1 us)
+    constexpr int bs = kRows == 1024 ? 32 : kRows == 256 ? 16 : 8;
     const int basex = bx * bs, basey = by * bs;
 
     // 1. load pixels; block min/max of depth
     float a[kSub][kAlphaSize];
     float depth[kSub];
-    int row[kSub];
     float dmin = 3.4e38f, dmax = -3.4e38f;
 #pragma unroll
     for (int s = 0; s < kSub; ++s) {
         const int q = tid + s * kThreads;
-        row[s] = -1;
+        depth[s] = 0.0f;
         if (q < kRows) {
-            const int qx = q % bs, qy = q / bs;
-            row[s] = qx * bs + qy;
-            const PixelIn p = load_pixel(g, im, basex + qx, basey + qy);
+            const PixelIn p = load_pixel(g, im, basex + q % bs, basey + q / bs);
             depth[s] = p.depth;
             a[s][1] = p.normal.x;
             a[s][2] = p.normal.y;
@@ -738,7 +737,6 @@ __device__ __forceinline__ void bmfr_fit_raw_gram_block(const BmfrGeom& g, const
         S.depth_min[wave] = dmin;
         S.depth_max[wave] = dmax;
     }
-    if (tid < bs) S.coord[tid] = (float)tid / (float)(bs - 1);  // bmfrPre.comp:36-43
     __syncthreads();
     float mn = S.depth_min[0], mx = S.depth_max[0];
 #pragma unroll
@@ -749,11 +747,12 @@ __device__ __forceinline__ void bmfr_fit_raw_gram_block(const BmfrGeom& g, const
     if (tid == 0) store_range(g, bx, by, mn, mx);
     // 2. features, fp16-quantised (the reference's R16F feature buffer), + noise; the
     //    noise of feature c for this thread's pixels is one vector load
+    //    the block coordinates are i / (bs - 1) (bmfrPre.comp:36-43)
 #pragma unroll
     for (int s = 0; s < kSub; ++s) {
-        const int r = row[s] < 0 ? 0 : row[s];
+        const int q = tid + s * kThreads;
         const float z = (depth[s] - mn) / (mx - mn + 1e-6f);
-        const float fx = S.coord[r / bs], fy = S.coord[r % bs];
+        const float fx = div_small<bs - 1>((float)(q % bs)), fy = div_small<bs - 1>((float)(q / bs % bs));
         a[s][0] = 1.0f;
         a[s][4] = fx;
         a[s][5] = fy;
@@ -803,7 +802,7 @@ __device__ __forceinline__ void bmfr_fit_raw_gram_block(const BmfrGeom& g, const
         for (int s = 0; s < kSub; ++s) {
             if (s > 0) wave_lds_sync();  // the previous chunk has been read
             float* dst = S.st[wave][lane];
-            if (row[s] < 0) {
+            if (tid + s * kThreads >= kRows) {
 #pragma unroll
                 for (int c = 0; c < kAlphaSize; ++c) a[s][c] = 0.0f;
             }

@@ -51,6 +51,20 @@ __device__ __forceinline__ int wrap_coord(int i, int n) {
     return r < 0 ? r + n : r;
 }
 
+// The two texels i and i + 1 of a bilinear fetch along an axis of n texels, with REPEAT
+// addressing.  Within one image of the origin (reprojected positions are) they wrap by one
+// addition and one compare; the integer remainders of the general case are some twenty
+// instructions each, four to a fetch.
+__device__ __forceinline__ void wrap_pair(int i, int n, int& i0, int& i1) {
+    if ((uint32_t)i + (uint32_t)n < 2u * (uint32_t)n) {  // -n <= i < n
+        i0 = i < 0 ? i + n : i;
+        i1 = i0 + 1 == n ? 0 : i0 + 1;
+    } else {
+        i0 = wrap_coord(i, n);
+        i1 = wrap_coord(i + 1, n);
+    }
+}
+
 // Bilinear fetch with REPEAT addressing at normalized (u, v); fetch(x, y) returns vec4.
 template <class F>
 __device__ __forceinline__ vec4 sample_bilinear(F fetch, int w, int h, float u, float v) {
@@ -58,8 +72,9 @@ __device__ __forceinline__ vec4 sample_bilinear(F fetch, int w, int h, float u, 
     float y = v * (float)h - 0.5f;
     float x0f = floorf(x), y0f = floorf(y);
     float fx = x - x0f, fy = y - y0f;
-    int x0 = wrap_coord((int)x0f, w), x1 = wrap_coord((int)x0f + 1, w);
-    int y0 = wrap_coord((int)y0f, h), y1 = wrap_coord((int)y0f + 1, h);
+    int x0, x1, y0, y1;
+    wrap_pair((int)x0f, w, x0, x1);
+    wrap_pair((int)y0f, h, y0, y1);
     vec4 a = fetch(x0, y0), b = fetch(x1, y0), c = fetch(x0, y1), d = fetch(x1, y1);
     float gx = 1.0f - fx, gy = 1.0f - fy;
     vec4 top = make_vec4(a.x * gx + b.x * fx, a.y * gx + b.y * fx, a.z * gx + b.z * fx, a.w * gx + b.w * fx);
