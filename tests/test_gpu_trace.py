@@ -336,6 +336,26 @@ def test_small_frame_tracer_equals_the_others(cuda, cfg1, w, h, output):
                 assert images[0][k].tobytes() == other[k].tobytes(), f"{k} differs at {w}x{h} frame {frame}"
 
 
+@pytest.mark.parametrize("block,queue", [(0, 0), (64, 3000), (128, 0), (256, 7777)])
+@pytest.mark.parametrize("w,h,depth", [(W, H, 0), (61, 37, 1), (1, 1, 4), (200, 9, 4), (W, H, 4)])
+def test_wavefront_joined_walks_equal_the_stages(cuda, cfg1, block, queue, w, h, depth):
+    """An uncounted wavefront trace walks a bounce's shadow rays and the next bounce's rays in
+    one launch, a counted one stage by stage: the same bytes, whatever the launch shape, one
+    vertex per path (no bounce to join with) to five, frames below one tile included."""
+    gen, scene, _ = cfg1
+    pc, _, _ = helpers.frame_push_constants(gen, w, h, 2)
+    staged = helpers.gbuffer(cuda, w, h)
+    cnt = cuda.zeros(6, dtype=cuda.int64, device="cuda")
+    helpers.trace(cuda, scene, pc, staged, w, h, max_depth=depth, tracer=capi.TRACER_WAVEFRONT, counters=cnt)
+    for _ in range(2):
+        img = helpers.gbuffer(cuda, w, h)
+        helpers.trace(cuda, scene, pc, img, w, h, max_depth=depth, tracer=capi.TRACER_WAVEFRONT, block_threads=block,
+                      queue_paths=queue)
+        cuda.cuda.synchronize()
+        for k in staged:
+            assert cuda.equal(staged[k], img[k]), k
+
+
 def test_trace_timing_records_every_stage(cuda, cfg1):
     """pbrt_trace_timing_begin/_end: one segment per wavefront stage launch, positive times."""
     gen, scene, _ = cfg1

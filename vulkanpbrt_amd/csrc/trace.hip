@@ -642,7 +642,7 @@ extern "C" int32_t pbrt_trace(const pbrt_scene* scene, const pbrt_trace_params* 
         float4* illum = reinterpret_cast<float4*>(img->illumination);
         TraceTiming* tm = scene_timing(scene);
         if (p->tracer == PBRT_TRACER_WAVEFRONT) {
-            wavefront_trace(sc, c, *img, counters, tm, p->block_threads, p->queue_paths, st);
+            wavefront_trace(sc, scene_bvh_depth(scene), c, *img, counters, tm, p->block_threads, p->queue_paths, st);
         } else if (!counters && (uint64_t)pair_grid.x * pair_grid.y <= resident_waves(pt_pairs)) {
             // The whole frame's pairs of walks are resident at once: its time is its longest
             // path's, which pt_pairs shortens.  Past that (131,072 pixels here) a second
