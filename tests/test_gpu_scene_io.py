@@ -156,3 +156,35 @@ def test_wavefront_equals_megakernel_with_glass(cuda, pbrt_lib, tmp_path):
     rel = np.abs(out[0] - out[1]) / np.maximum(np.abs(out[0]), 1e-3)
     print(f"megakernel vs wavefront: identical pixels {same:.5f}, within 1e-5 {(rel.max(-1) <= 1e-5).mean():.5f}")
     assert (rel.max(-1) <= 1e-5).mean() >= 0.999
+
+
+@pytest.mark.parametrize("tw,th", [(1, 5), (2, 1), (2, 2), (3, 7), (17, 5)])
+def test_texture_taps_wrap_at_every_width(cuda, pbrt_lib, oracle_lib, tmp_path, tw, th):
+    """Bilinear taps that are neighbours in a row come in one load, those across the wrap in
+    two: textures of one, two and odd numbers of texels a row, tiled on both sides of zero."""
+    _box_scene(tmp_path)
+    rng = np.random.default_rng(tw * 10 + th)
+    tex = rng.integers(0, 256, (th, tw, 4), dtype=np.uint8)
+    tex[..., 3] = 255
+    Image.fromarray(tex, "RGBA").save(tmp_path / "checker.png")
+    obj = (tmp_path / "box.obj").read_text()
+    for old, new in (("vt 0 0", "vt -2.3 -1.7"), ("vt 1 0", "vt 3.4 -1.7"), ("vt 1 1", "vt 3.4 2.6"),
+                     ("vt 0 1", "vt -2.3 2.6")):
+        obj = obj.replace(old + "\n", new + "\n")
+    (tmp_path / "box.obj").write_text(obj)
+    loaded = capi.LoadedScene(tmp_path / "box.obj")
+    scene = capi.Scene(loaded.desc, keepalive=loaded)
+    osc = oracle_lib.OracleScene(loaded.desc)
+    view, proj = camera.pose_matrices(_pose([0.6, -1.6, 0.7], [0.6, 0.6, 0.6]), N, N)
+    pc = camera.push_constants(view, proj, view, 1)
+    img = helpers.gbuffer(cuda, N, N)
+    helpers.trace(cuda, scene, pc, img, N, N, max_depth=2)
+    cuda.cuda.synchronize()
+    gpu = helpers.to_np(img)
+    ref = osc.trace(N, N, np.array(pc.view_inverse[:], np.float32), np.array(pc.proj_inverse[:], np.float32), frame=1,
+                    precision=32)
+    glass = np.all(gpu["albedo"][..., :3] == 255, axis=-1)
+    keys = ("depth", "albedo", "illumination")
+    frac = _compare_frame({k: gpu[k][~glass] for k in keys}, {k: ref[k][~glass] for k in keys}, f"texture {tw}x{th}")
+    _assert_mirror_exact(frac)
+    assert len(np.unique(gpu["albedo"].reshape(-1, 4), axis=0)) > (20 if tw * th > 2 else 2)

