@@ -201,10 +201,14 @@ enum pbrt_illumination_output {
 
 enum pbrt_tracer_kind {
     PBRT_TRACER_MEGAKERNEL = 0, /* one thread per path, whole path in one launch */
-    PBRT_TRACER_WAVEFRONT = 1,  /* ray queues: extend / shade / shadow launches per bounce */
+    PBRT_TRACER_WAVEFRONT = 1,  /* ray queues: extend / shade / shadow launches per bounce (a
+                                   bounce's shadow rays go with the next one's extend, unless the
+                                   trace is counted or its stages timed) */
     PBRT_TRACER_PERSISTENT = 2  /* megakernel with path regeneration: resident waves draw pixels
                                    from a frame counter, a lane whose path ends starts the next
                                    pixel (same per-pixel results as the megakernel) */
+    /* Uncounted traces of small frames (at most 131,072 pixels on 256 CUs) run one kernel of
+     * 32 pixels per wave for both megakernels, with the same per-pixel results. */
 };
 
 typedef struct pbrt_trace_params {
