@@ -99,8 +99,7 @@ def outer_taps(layers):
 
 @pytest.mark.parametrize("layers", [6, 2, "c"])
 def test_forward_matches_oracle(cuda, layers):
-    """Six layers: the layer-by-layer path with kernel prediction fused into the last
-    layer; two layers: the single fused kernel (features to filtered radiance in LDS);
+    """Six layers: the row pipeline; two layers: the single fused kernel (features to filtered radiance in LDS);
     the compact network ("c": the second layer pointwise, its outer taps zero): its own
     fused kernel (both layers in registers per 16-pixel row).  The oracle runs the
     two-layer shape with the same parameters."""
@@ -163,6 +162,44 @@ def test_row_pipeline_matches_oracle(cuda, layers, w, h, count):
     alb = inp["albedo"][..., :3].astype(np.float64) / 255 + 1e-6
     expect = np.clip(np.maximum(alb * g, 0) ** 0.454545, 0, 1) * 255
     assert np.abs(t["final"].cpu().numpy()[..., 2::-1].astype(float) - expect).max() <= 1.0
+    net.close()
+
+
+@pytest.mark.parametrize("layers,w,h,count", [(6, 200, 120, 1), (5, 57, 40, 2), (4, 130, 33, 1), (3, 16, 9, 3),
+                                              (6, 1, 1, 1)])
+def test_inference_takes_the_training_roundings(cuda, layers, w, h, count):
+    """Inference gives the image that the training pass scores, bit for bit: the same bf16
+    roundings of every activation and the same softmax.  Its output as the loss's target
+    leaves a residual a o - a t of the two products' roundings alone, at most 2^-24 of a t,
+    so the loss is at most 2^-48; one bf16 activation rounded the other way (2^-9 of it)
+    moves some outputs by 1e-5 and more."""
+    rng = np.random.default_rng(w * h)
+    inp = dict(
+        noisy=half(rng.gamma(1.0, 0.5, (count, h, w, 4))),
+        depth=rng.uniform(0.5, 20.0, (count, h, w)).astype(np.float32),
+        normal=rng.uniform(0, np.pi, (count, h, w, 2)).astype(np.float32),
+        albedo=rng.integers(128, 256, (count, h, w, 4), dtype=np.uint8),
+        spp=rng.integers(0, 40, (count, h, w), dtype=np.uint8),
+        motion=half(rng.uniform(-1, 1, (count, h, w, 2))),
+        target=np.zeros((count, h, w, 4), np.float32),
+    )
+    net = Net(11, layers)
+    params = net.get()
+    n = cnn.parameter_count(cnn.shape_of(layers))
+    params[n - 25 - 9 * 32 * 25:n - 25] *= 10.0
+    params += rng.normal(0, 0.01, n).astype(np.float32)  # biases, zero at first, among them
+    net.set(params)
+    im, t = device_images(cuda, inp, True, w, h, count)
+    st = helpers.stream(cuda)
+    capi.check(capi.lib().pbrt_cnn_denoise(net.h, C.byref(im), st))
+    t["target"].copy_(t["denoised"])
+    loss = cuda.zeros(1, dtype=cuda.float32, device="cuda")
+    grad = cuda.zeros(n, dtype=cuda.float32, device="cuda")
+    capi.check(capi.lib().pbrt_cnn_gradients(net.h, C.byref(im), capi.ptr(loss), capi.ptr(grad), st))
+    cuda.cuda.synchronize()
+    assert t["denoised"][..., :3].abs().mean() > 0.1
+    print(f"{layers} layers {w}x{h}x{count}: loss against its own output {loss.item():.3e}")
+    assert loss.item() <= 2.0 ** -48
     net.close()
 
 

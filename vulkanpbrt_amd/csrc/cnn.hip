@@ -641,21 +641,21 @@ LayerTable layer_table(int layers) {
     return lt;
 }
 
-// Softmax weights of one output pixel from its 25 bf16 logits (LDS, `logits`: 32
-// channels, 25 used; its 16-byte chunk q at q ^ swizzle), not yet normalised.
+// Softmax weights of one output pixel, not yet normalised.
 struct KpnWeights {
     float e[kKernelTaps];
     float sum;
 };
 
-__device__ __forceinline__ KpnWeights kpn_weights(const uint16_t* logits, int swizzle = 0) {
+// From its 25 bf16 logits (LDS, `logits`: 32 channels, 25 used).
+__device__ __forceinline__ KpnWeights kpn_weights(const uint16_t* logits) {
     // the 25 bf16 logits (and 7 padding channels): four 16-byte reads, twice
     // (maximum, then the weighted sum) to keep few registers live
     const uint4* lz = reinterpret_cast<const uint4*>(logits);
     float zmax = -3.4e38f;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const uint4 v = lz[q ^ swizzle];
+        const uint4 v = lz[q];
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
@@ -670,7 +670,7 @@ __device__ __forceinline__ KpnWeights kpn_weights(const uint16_t* logits, int sw
     r.sum = 0.0f;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const uint4 v = lz[q ^ swizzle];
+        const uint4 v = lz[q];
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
@@ -884,40 +884,42 @@ __global__ void __launch_bounds__(256, 3) k_two_layer(CnnGeom g, pbrt_cnn_images
 // the row its predecessor finished in the step before, so activations never leave LDS
 // and the only recomputed pixels are the strip's L columns and rows at each edge.  Two
 // waves per layer take 16 output channels each with that layer's weights in registers;
-// one wave computes the feature row and two the softmax filter of the finished logits, on
-// alternate rows (at 6 layers 15 waves, at most 128 registers, one workgroup per CU).
+// four waves take turns at the feature row and the softmax filter of the finished logits
+// (at 6 layers 16 waves, at most 128 registers, one workgroup per CU).
 //   A convolution wave reads each input row once, as three horizontally shifted operands
 // per 16 columns, and adds it to the three output rows it contributes to (output row r
 // receives input rows r - 1, r, r + 1 in three consecutive steps): three LDS reads per
 // nine matrix instructions.  Reading it nine times, once per tap, would need more LDS
 // bandwidth than the matrix cores leave time for.
-//   Step t, with row numbers counted from y0 - L: the features wave writes row t, layer l
-// finishes row t - 2l - 2, the filter takes row t - 1 - 2L and stores it in the step
-// after.  Rows and columns outside the image are zero after every layer (the
+//   Step t, with row numbers counted from y0 - L: the features of row t are written, layer l
+// finishes row t - 2l - 2, the filter takes row t - 1 - 2L and stores it two steps later.  Rows and columns outside the image are zero after every layer (the
 // convolutions' padding); edge columns and the first rows a layer finishes hold values
 // made from unwritten neighbours, which reach only pixels the strip does not output.
-//   What bounds it: the matrix cores, 1728 cycles a row on the busiest SIMD (154 us at
-// 1920x1080, of which a third is strip and segment halo), then a step's first operands,
-// its stores and the barrier.  Two rows per step save barriers but add L rows of latency
-// (217 us).  6 layers, before (seven launches through HBM) and now: 1920x1080 377 -> 210
-// us, 1280x720 166 -> 103, 480x270 48 -> 36, 200x120 31 -> 26.
+//   Every rounding is that of the layer-by-layer kernels (k_conv3x3, and k_kpn's softmax), so
+// inference gives, bit for bit, the image that training scores.
+//   What bounds it: the matrix cores, 1728 of a step's some 2,900 cycles (154 us at
+// 1920x1080, of which a third is strip and segment halo), then what a step cannot hide
+// behind them: its first operands, the bias, ReLU and rounding after its last product, the
+// filter's vector work and the barrier.  Two rows per step save barriers but add L rows of
+// latency.  6 layers, before (seven launches through HBM) and now: 1920x1080 369 -> 238
+// us, 1280x720 166 -> 116, 480x270 48 -> 39, 200x120 31 -> 28.
 constexpr int kPipeCols = 64;                 // columns of a strip
 constexpr int kPipeTiles = kPipeCols / 16;    // 16-pixel matrix tiles of a row
 constexpr int kPipePix = kPipeCols + 2;       // LDS pixels of a row (column c at c + 1)
-constexpr int kPipeRing = 32;                 // noisy rows kept for the filter (2L + 5 are live)
+constexpr int kPipeRing = 32;                 // noisy rows kept for the filter (2L + 6 are live)
 // An LDS pixel is 32 channels in four 16-byte chunks, chunk q at q ^ pipe_swizzle(pixel).
 // A 16-byte read serves sixteen lanes at a time, eight neighbouring pixels of one chunk and
 // the same pixels of the next: so placed, they meet in distinct banks (pixels side by side
 // without it, or 80 bytes apart, spent half of the LDS cycles on conflicts).
 __device__ __forceinline__ constexpr int pipe_swizzle(int pixel) { return (pixel & 4) >> 1; }
-constexpr int kPipeStride = kCh, kPipeFeatStride = kFeatCh;
+constexpr int kPipeStride = kCh;
 
-constexpr int pipe_threads(int layers) { return 64 * (2 * layers + 3); }
+constexpr int pipe_threads(int layers) { return 64 * (2 * layers + 4); }
 
 template <int L>
 struct PipeShared {
     // double-buffered by step
-    __attribute__((aligned(16))) uint16_t feat[2][kPipePix * kPipeFeatStride];
+    __attribute__((aligned(16))) uint16_t feat[2][kPipePix * kPipeStride];    // 16 features, 16 zeros
     __attribute__((aligned(16))) uint16_t act[L][2][kPipePix * kPipeStride];  // layer l's rows; the last: logits
     __attribute__((aligned(16))) uint2 noisy[kPipeRing][kPipeCols];          // clamped to the image, raw FP16
 };
@@ -928,32 +930,26 @@ struct PipeStrip {
     int x0, y0, rows, steps, img;
 };
 
-// One convolution wave: layer `l`, output channels 16 half ... + 15.  kFirst: 16 input
-// channels, two horizontal taps per matrix instruction (the third with a zero partner).
+// One convolution wave: layer `l`, output channels 16 half ... + 15.  A pixel's sum is
+// k_conv3x3's, rounding for rounding: nine products from zero in the taps' row-major order,
+// then the bias; so inference sees the activations that training does.  kFirst: the 16
+// features in a 32-deep product with 16 zeros, which gives the bits of the 16-deep one and
+// issues faster.
 template <int L, bool kFirst, bool kLast>
 __device__ __forceinline__ void pipe_conv(const CnnGeom& g, const PipeStrip& p, PipeShared<L>& S, int l, int half,
                                           const uint16_t* __restrict__ wf, const float* __restrict__ master) {
-    constexpr int kK = kFirst ? 2 : 3;  // operands per tile and input row
-    constexpr int kStride = kFirst ? kPipeFeatStride : kPipeStride;
+    constexpr int kCin = kFirst ? kFeatCh : kCh;
     const int lane = threadIdx.x & 63, j = lane & 15, grp = lane >> 4;
     const int woff = kFirst ? 0 : weight_offset(1) + (l - 1) * layer_weights(1);
     const int boff = kFirst ? layer_weights(0) : layer_offset(1) + (l - 1) * layer_size(1) + layer_weights(1);
-    bf16x8 w[3][kK];
+    bf16x8 w[3][3];
 #pragma unroll
-    for (int ky = 0; ky < 3; ++ky)
-#pragma unroll
-        for (int k = 0; k < kK; ++k) {
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (kFirst) {
-                const int kx = 2 * k + (grp >> 1);
-                if (kx < 3)
-                    v = *reinterpret_cast<const uint4*>(
-                        wf + woff + ((ky * 3 + kx) * kCh + half * 16 + j) * kFeatCh + 8 * (grp & 1));
-            } else {
-                v = *reinterpret_cast<const uint4*>(wf + woff + ((ky * 3 + k) * kCh + half * 16 + j) * kCh + 8 * grp);
-            }
-            w[ky][k] = __builtin_bit_cast(bf16x8, v);
-        }
+    for (int tp = 0; tp < kTaps; ++tp) {
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (!kFirst || grp < 2)
+            v = *reinterpret_cast<const uint4*>(wf + woff + (tp * kCh + half * 16 + j) * kCin + 8 * grp);
+        w[tp / 3][tp % 3] = __builtin_bit_cast(bf16x8, v);
+    }
     float4v bias;
 #pragma unroll
     for (int i = 0; i < 4; ++i) bias[i] = master[boff + half * 16 + 4 * grp + i];
@@ -964,20 +960,18 @@ __device__ __forceinline__ void pipe_conv(const CnnGeom& g, const PipeStrip& p, 
         const int x = p.x0 + 16 * n + j;
         hi[n] = x >= 0 && x < g.width ? INFINITY : 0.0f;
     }
-    // this lane's element of an operand: pixel j + tap of a tile, 8 channels (the zero
-    // partner of the first layer's third tap reads that tap's own pixel)
-    int at[kK];
+    // this lane's element of an operand: pixel j + tap of a tile, 8 channels
+    int at[3];
 #pragma unroll
-    for (int k = 0; k < kK; ++k)
-        at[k] = kFirst ? (k == 0 ? j + (grp >> 1) : j + 2) * kStride + 8 * (grp & 1)
-                       : (j + k) * kStride + 8 * (grp ^ pipe_swizzle(j + k));
+    for (int k = 0; k < 3; ++k)
+        at[k] = (j + k) * kPipeStride + 8 * (grp ^ pipe_swizzle(j + k));
     // the lane's 16 bytes of a finished tile pair (see below)
     const int out = (1 + 16 * (grp & 1) + j) * kPipeStride + 8 * ((2 * half + (grp >> 1)) ^ pipe_swizzle(1 + j));
     float4v acc[3][kPipeTiles];
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
-        for (int n = 0; n < kPipeTiles; ++n) acc[a][n] = bias;
+        for (int n = 0; n < kPipeTiles; ++n) acc[a][n] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
     for (int t3 = 0; t3 < p.steps; t3 += 3) {
 #pragma unroll
         for (int ph = 0; ph < 3; ++ph) {  // the accumulators this step's row completes
@@ -986,11 +980,11 @@ __device__ __forceinline__ void pipe_conv(const CnnGeom& g, const PipeStrip& p, 
 #pragma unroll
             for (int n = 0; n < kPipeTiles; ++n) {
                 float4v &fin = acc[ph][n], &mid = acc[(ph + 1) % 3][n], &beg = acc[(ph + 2) % 3][n];
-                beg = bias;
+                beg = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int k = 0; k < kK; ++k) {
+                for (int k = 0; k < 3; ++k) {
                     const bf16x8 b =
-                        __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(in + 16 * n * kStride + at[k]));
+                        __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(in + 16 * n * kPipeStride + at[k]));
                     fin = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[2][k], b, fin, 0, 0, 0);
                     mid = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[1][k], b, mid, 0, 0, 0);
                     beg = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[0][k], b, beg, 0, 0, 0);
@@ -1009,9 +1003,10 @@ __device__ __forceinline__ void pipe_conv(const CnnGeom& g, const PipeStrip& p, 
                 for (int m = 0; m < 2; ++m) {
                     float v[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        v[i] = kLast ? acc[ph][n + m][i]
-                                     : __builtin_amdgcn_fmed3f(acc[ph][n + m][i], 0.0f, row ? hi[n + m] : 0.0f);
+                    for (int i = 0; i < 4; ++i) {
+                        v[i] = acc[ph][n + m][i] + bias[i];
+                        if (!kLast) v[i] = __builtin_amdgcn_fmed3f(v[i], 0.0f, row ? hi[n + m] : 0.0f);
+                    }
                     q[m][0] = pack_bf16(v[0], v[1]);
                     q[m][1] = pack_bf16(v[2], v[3]);
                 }
@@ -1024,57 +1019,131 @@ __device__ __forceinline__ void pipe_conv(const CnnGeom& g, const PipeStrip& p, 
     }
 }
 
+// The softmax filter in the arithmetic of the training pass (k_kpn), so that a network gives
+// what it was trained to give: exponentials by expf, one division, normalised weights.
+// One pixel's bf16 logits (16-byte chunk q at q ^ swizzle), less their maximum:
+__device__ __forceinline__ void pipe_logits(const uint16_t* logits, int swizzle, KpnWeights& k) {
+    const uint4* lz = reinterpret_cast<const uint4*>(logits);
+    float zmax = -3.4e38f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint4 v = lz[q ^ swizzle];
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int c = 8 * q + i;
+            if (c < kKernelTaps) {
+                k.e[c] = __uint_as_float((i & 1) ? (w[i / 2] & 0xFFFF0000u) : (w[i / 2] << 16));
+                zmax = fmaxf(zmax, k.e[c]);
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < kKernelTaps; ++c) k.e[c] -= zmax;
+    k.sum = 0.0f;
+}
+
+// The exponentials of taps kFrom .. kTo - 1 and their share of the sum:
+template <int kFrom, int kTo>
+__device__ __forceinline__ void pipe_exponentials(KpnWeights& k) {
+#pragma unroll
+    for (int c = kFrom; c < kTo; ++c) {
+        k.e[c] = expf(k.e[c]);
+        k.sum += k.e[c];
+    }
+}
+
+__device__ __forceinline__ void pipe_normalise(KpnWeights& k) {
+    const float inv = 1.0f / k.sum;
+#pragma unroll
+    for (int c = 0; c < kKernelTaps; ++c) k.e[c] *= inv;
+}
+
+// The weighted sum of the taps, stored as denoised radiance and / or final image:
+template <class Tap>
+__device__ __forceinline__ void pipe_apply(const pbrt_cnn_images& im, const KpnWeights& k, Tap tap, size_t i,
+                                           uint32_t albedo) {
+    vec3 o = make_vec3(0.0f);
+#pragma unroll
+    for (int c = 0; c < kKernelTaps; ++c) {
+        const uint2 nv = tap(c);
+        const half2v rg = __builtin_bit_cast(half2v, nv.x), ba = __builtin_bit_cast(half2v, nv.y);
+        o += make_vec3((float)rg.x, (float)rg.y, (float)ba.x) * k.e[c];
+    }
+    if (im.denoised) reinterpret_cast<float4*>(im.denoised)[i] = make_float4(o.x, o.y, o.z, 1.0f);
+    if (im.final_image) {
+        const uchar4 ac = __builtin_bit_cast(uchar4, albedo);
+        const vec3 alb = make_vec3(unorm8_to_float(ac.x), unorm8_to_float(ac.y), unorm8_to_float(ac.z));
+        const vec3 tm = (alb + make_vec3(1e-6f)) * o;
+        store_bgra8(im.final_image, i,
+                    make_vec4(fast_gamma(fmaxf(tm.x, 0.0f)), fast_gamma(fmaxf(tm.y, 0.0f)),
+                              fast_gamma(fmaxf(tm.z, 0.0f)), 1.0f));
+    }
+}
+
+// The four other waves, one per SIMD: each takes every fourth row, one step for its
+// features and three for its filter, so that no step is longer than a convolution wave's
+// and the SIMDs carry equal shares.  Turn t: the features of row t in step t; then, of the
+// output row whose logits arrive in step t + 1, the logits and some exponentials, the other
+// exponentials and the division, the 25 taps and the stores.
 template <int L>
-__device__ __forceinline__ void pipe_features(const CnnGeom& g, const PipeStrip& p, const pbrt_cnn_images& im,
-                                              PipeShared<L>& S) {
+__device__ __forceinline__ void pipe_pixels(const CnnGeom& g, const PipeStrip& p, const pbrt_cnn_images& im,
+                                            PipeShared<L>& S, int phase) {
     const int c = threadIdx.x & 63, x = p.x0 + c;
     const size_t base = (size_t)g.width * g.height * p.img;
     const int xc = min(max(x, 0), g.width - 1);
+    const bool column = c >= L && c < kPipeCols - L && x < g.width;
     auto fetch = [&](int t) {
         const int yc = min(max(p.y0 + t, 0), g.height - 1);
         return load_raw_pixel(im, base + (size_t)yc * g.width + xc);
     };
-    RawPixel raw = fetch(0);
-    for (int t = 0; t < p.steps; ++t) {
-        const RawPixel cur = raw;
-        raw = fetch(t + 1);  // in flight until the next step
-        const int y = p.y0 + t;
-        uint4 lo = make_uint4(0, 0, 0, 0), hi = lo;
-        if (x == xc && y >= 0 && y < g.height) raw_features(cur, lo, hi);
-        uint16_t* f = S.feat[t & 1] + (c + 1) * kPipeFeatStride;
-        *reinterpret_cast<uint4*>(f) = lo;
-        *reinterpret_cast<uint4*>(f + 8) = hi;
-        S.noisy[t % kPipeRing][c] = cur.noisy;
-        __syncthreads();
-    }
-}
-
-// The softmax filter of every second row, over two steps a row: the weights in the step
-// its logits arrive, the 25 taps and the stores in the next.
-template <int L>
-__device__ __forceinline__ void pipe_filter(const CnnGeom& g, const PipeStrip& p, const pbrt_cnn_images& im,
-                                            const PipeShared<L>& S, int parity) {
-    const int c = threadIdx.x & 63, x = p.x0 + c;
-    const size_t base = (size_t)g.width * g.height * p.img;
-    const bool column = c >= L && c < kPipeCols - L && x < g.width;
+    RawPixel raw = fetch(phase);
     uint32_t albedo = 0;
     KpnWeights k;
-    for (int t = 0; t < p.steps; ++t) {
-        // the row whose logits arrived in this step, or in the one before
-        const int o = t - 1 - 2 * L - ((t & 1) ^ parity);
-        if (column && o >= L && o < L + p.rows) {
-            const size_t i = base + (size_t)(p.y0 + o) * g.width + x;
-            if ((t & 1) == parity) {
-                albedo = reinterpret_cast<const uint32_t*>(im.albedo)[i];
-                k = kpn_weights(S.act[L - 1][(t & 1) ^ 1] + (c + 1) * kPipeStride, pipe_swizzle(c + 1));
-            } else {
+    // before the convolution waves of the same SIMD, whose matrix instructions fill the rest
+    // (three layers at 1920x1080: 148 -> 141 us)
+    __builtin_amdgcn_s_setprio(3);
+    for (int t = phase - 4; t < p.steps; t += 4) {  // the first and last turns are partial
+        const int o = t - 2 * L;
+        const bool active = column && o >= L && o < L + p.rows;
+        const size_t i = base + (size_t)(p.y0 + o) * g.width + x;
+        if (t >= 0) {
+            const RawPixel cur = raw;
+            raw = fetch(t + 4);  // in flight until the next turn
+            if (active) albedo = reinterpret_cast<const uint32_t*>(im.albedo)[i];
+            const int y = p.y0 + t;
+            uint4 lo = make_uint4(0, 0, 0, 0), hi = lo;
+            if (x == xc && y >= 0 && y < g.height) raw_features(cur, lo, hi);
+            uint4* f = reinterpret_cast<uint4*>(S.feat[t & 1] + (c + 1) * kPipeStride);
+            f[pipe_swizzle(c + 1)] = lo;
+            f[1 ^ pipe_swizzle(c + 1)] = hi;
+            if (t < 2) f[2 ^ pipe_swizzle(c + 1)] = f[3 ^ pipe_swizzle(c + 1)] = make_uint4(0, 0, 0, 0);
+            S.noisy[t % kPipeRing][c] = cur.noisy;
+            __syncthreads();
+        }
+        if (t + 1 >= 0 && t + 1 < p.steps) {
+            if (active) {
+                pipe_logits(S.act[L - 1][t & 1] + (c + 1) * kPipeStride, pipe_swizzle(c + 1), k);
+                pipe_exponentials<0, 10>(k);
+            }
+            __syncthreads();
+        }
+        if (t + 2 >= 0 && t + 2 < p.steps) {
+            if (active) {
+                pipe_exponentials<10, kKernelTaps>(k);
+                pipe_normalise(k);
+            }
+            __syncthreads();
+        }
+        if (t + 3 >= 0 && t + 3 < p.steps) {
+            if (active) {
                 const uint2* taps[5];
 #pragma unroll
                 for (int q = 0; q < 5; ++q) taps[q] = &S.noisy[(o + q - 2) % kPipeRing][c - 2];
-                kpn_apply(im, k, [&](int q) { return taps[q / 5][q % 5]; }, i, &albedo);
+                pipe_apply(im, k, [&](int q) { return taps[q / 5][q % 5]; }, i, albedo);
             }
+            __syncthreads();
         }
-        __syncthreads();
     }
 }
 
@@ -1090,7 +1159,7 @@ __global__ void __launch_bounds__(pipe_threads(L)) k_pipeline(CnnGeom g, pbrt_cn
     p.x0 = (int)(blockIdx.x % strips_x) * (kPipeCols - 2 * L) - L;
     p.y0 = first - L;
     p.rows = min(seg_rows, g.height - first);
-    p.steps = (p.rows + 3 * L + 2 + 2) / 3 * 3;  // the last row is stored in step rows + 3L + 1
+    p.steps = (p.rows + 3 * L + 3 + 2) / 3 * 3;  // the last row is stored in step rows + 3L + 2
     p.img = blockIdx.x / strips_x;
     if (wave < 2)
         pipe_conv<L, true, false>(g, p, S, 0, wave, wf, master);
@@ -1098,10 +1167,8 @@ __global__ void __launch_bounds__(pipe_threads(L)) k_pipeline(CnnGeom g, pbrt_cn
         pipe_conv<L, false, false>(g, p, S, wave >> 1, wave & 1, wf, master);
     else if (wave < 2 * L)
         pipe_conv<L, false, true>(g, p, S, L - 1, wave & 1, wf, master);
-    else if (wave < 2 * L + 2)
-        pipe_filter<L>(g, p, im, S, wave & 1);
     else
-        pipe_features<L>(g, p, im, S);
+        pipe_pixels<L>(g, p, im, S, wave - 2 * L);
 }
 
 // ---------------------------------------------------------------------------
@@ -1403,7 +1470,7 @@ void mask_pointwise_gradient(const pbrt_cnn* net, float* padded_grad, hipStream_
 
 // inference of three to six layers: the row pipeline, no workspace.  Strips are cut into
 // segments so that the workgroups (one per CU) fill whole rounds of the chip: of one to
-// eight rounds, the one with the fewest rows in all (a segment of r rows takes r + 3L + 2
+// eight rounds, the one with the fewest rows in all (a segment of r rows takes r + 3L + 3
 // steps with its halo and the pipeline's latency, an unfilled round idles CUs).
 template <int L>
 void launch_pipeline(const pbrt_cnn* net, const pbrt_cnn_images& im, hipStream_t st) {
@@ -1417,7 +1484,7 @@ void launch_pipeline(const pbrt_cnn* net, const pbrt_cnn_images& im, hipStream_t
     for (uint64_t rounds = 1; rounds <= 8; ++rounds) {
         const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(rounds * cus / strips, 1), im.height);
         const uint64_t r = (im.height + want - 1) / want, n = (im.height + r - 1) / r;
-        const uint64_t cost = (strips * n + cus - 1) / cus * (r + 3 * L + 2);
+        const uint64_t cost = (strips * n + cus - 1) / cus * (r + 3 * L + 3);
         if (cost < best) {
             best = cost;
             rows = (uint32_t)r;
