@@ -592,7 +592,10 @@ int32_t pbrt_cnn_get_parameters(const pbrt_cnn* net, float* host_params);
 int32_t pbrt_cnn_set_parameters(pbrt_cnn* net, const float* host_params); /* also resets the optimiser */
 int32_t pbrt_cnn_workspace_size(uint32_t width, uint32_t height, uint32_t count, uint32_t training,
                                 size_t* out_bytes);
-/* Inference: denoised and/or final_image of every image. */
+/* Inference: denoised and/or final_image of every image.  Networks of three to six layers
+ * run as one kernel, or layer by layer through images.workspace where that is faster
+ * (batches of small images) and where an output image shares memory with an input; the
+ * result is the same bits.  Their workspace is required either way. */
 int32_t pbrt_cnn_denoise(const pbrt_cnn* net, const pbrt_cnn_images* images, void* stream);
 /* Loss and its gradient (device pointers: 1 float, parameter_count floats in
  * canonical order) without changing the network. */

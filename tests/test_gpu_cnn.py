@@ -162,6 +162,47 @@ def test_row_pipeline_matches_oracle(cuda, layers, w, h, count):
     alb = inp["albedo"][..., :3].astype(np.float64) / 255 + 1e-6
     expect = np.clip(np.maximum(alb * g, 0) ** 0.454545, 0, 1) * 255
     assert np.abs(t["final"].cpu().numpy()[..., 2::-1].astype(float) - expect).max() <= 1.0
+    # the layer-by-layer route would have left its features and activations there
+    assert not t["ws"].any()
+    net.close()
+
+
+def random_inputs(rng, w, h, count):
+    return dict(
+        noisy=half(rng.gamma(1.0, 0.5, (count, h, w, 4))),
+        depth=rng.uniform(0.5, 20.0, (count, h, w)).astype(np.float32),
+        normal=rng.uniform(0, np.pi, (count, h, w, 2)).astype(np.float32),
+        albedo=rng.integers(0, 256, (count, h, w, 4), dtype=np.uint8),
+        spp=rng.integers(0, 40, (count, h, w), dtype=np.uint8),
+        motion=half(rng.uniform(-1, 1, (count, h, w, 2))),
+    )
+
+
+@pytest.mark.parametrize("layers", [3, 4, 5, 6])
+@pytest.mark.parametrize("w,h,count,by_layers", [(16, 16, 2048, True), (8, 9, 4096, True), (33, 21, 1024, True),
+                                                (1, 300, 600, True), (130, 75, 1, False), (101, 99, 40, False)])
+def test_both_routes_give_the_same_bytes(cuda, layers, w, h, count, by_layers):
+    """Batches of small images run layer by layer, larger ones as the row pipeline.  Of every
+    batch the first and last image are denoised again on the other route: alone (one small
+    image is a pipeline) or with the output in the memory of an input (layer by layer)."""
+    inp = random_inputs(np.random.default_rng(w * h), w, h, count)
+    net = Net(5, layers)
+    params = net.get()
+    net.set(params + np.random.default_rng(layers).normal(0, 0.02, len(params)).astype(np.float32))
+    st = helpers.stream(cuda)
+    im, t = device_images(cuda, inp, False, w, h, count)
+    capi.check(capi.lib().pbrt_cnn_denoise(net.h, C.byref(im), st))
+    cuda.cuda.synchronize()
+    assert bool(t["ws"].any()) == by_layers
+    for i in (0, count - 1):
+        im1, t1 = device_images(cuda, {k: v[i:i + 1] for k, v in inp.items()}, False, w, h, 1)
+        if not by_layers:
+            im1.final_image = im1.albedo
+        capi.check(capi.lib().pbrt_cnn_denoise(net.h, C.byref(im1), st))
+        cuda.cuda.synchronize()
+        assert bool(t1["ws"].any()) != by_layers
+        assert cuda.equal(t1["denoised"][0].view(cuda.int32), t["denoised"][i].view(cuda.int32))
+        assert cuda.equal((t1["final"] if by_layers else t1["albedo"])[0], t["final"][i])
     net.close()
 
 

@@ -177,9 +177,82 @@ __global__ void __launch_bounds__(256) k_features(CnnGeom g, pbrt_cnn_images im,
 }
 
 // ---------------------------------------------------------------------------
+// The softmax filter of inference with three to six layers
+// ---------------------------------------------------------------------------
+// Softmax weights of one output pixel and their sum.
+struct KpnWeights {
+    float e[kKernelTaps];
+    float sum;
+};
+
+// The softmax filter in the arithmetic of the training pass (k_kpn), so that a network gives
+// what it was trained to give: exponentials by expf, one division, normalised weights.
+// One pixel's bf16 logits (16-byte chunk q at q ^ swizzle), less their maximum:
+__device__ __forceinline__ void exact_logits(const uint16_t* logits, int swizzle, KpnWeights& k) {
+    const uint4* lz = reinterpret_cast<const uint4*>(logits);
+    float zmax = -3.4e38f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint4 v = lz[q ^ swizzle];
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int c = 8 * q + i;
+            if (c < kKernelTaps) {
+                k.e[c] = __uint_as_float((i & 1) ? (w[i / 2] & 0xFFFF0000u) : (w[i / 2] << 16));
+                zmax = fmaxf(zmax, k.e[c]);
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < kKernelTaps; ++c) k.e[c] -= zmax;
+    k.sum = 0.0f;
+}
+
+// The exponentials of taps kFrom .. kTo - 1 and their share of the sum:
+template <int kFrom, int kTo>
+__device__ __forceinline__ void exact_exponentials(KpnWeights& k) {
+#pragma unroll
+    for (int c = kFrom; c < kTo; ++c) {
+        k.e[c] = expf(k.e[c]);
+        k.sum += k.e[c];
+    }
+}
+
+__device__ __forceinline__ void exact_normalise(KpnWeights& k) {
+    const float inv = 1.0f / k.sum;
+#pragma unroll
+    for (int c = 0; c < kKernelTaps; ++c) k.e[c] *= inv;
+}
+
+// The weighted sum of the taps, stored as denoised radiance and / or final image:
+template <class Tap>
+__device__ __forceinline__ void exact_apply(const pbrt_cnn_images& im, const KpnWeights& k, Tap tap, size_t i,
+                                           uint32_t albedo) {
+    vec3 o = make_vec3(0.0f);
+#pragma unroll
+    for (int c = 0; c < kKernelTaps; ++c) {
+        const uint2 nv = tap(c);
+        const half2v rg = __builtin_bit_cast(half2v, nv.x), ba = __builtin_bit_cast(half2v, nv.y);
+        o += make_vec3((float)rg.x, (float)rg.y, (float)ba.x) * k.e[c];
+    }
+    if (im.denoised) reinterpret_cast<float4*>(im.denoised)[i] = make_float4(o.x, o.y, o.z, 1.0f);
+    if (im.final_image) {
+        const uchar4 ac = __builtin_bit_cast(uchar4, albedo);
+        const vec3 alb = make_vec3(unorm8_to_float(ac.x), unorm8_to_float(ac.y), unorm8_to_float(ac.z));
+        const vec3 tm = (alb + make_vec3(1e-6f)) * o;
+        store_bgra8(im.final_image, i,
+                    make_vec4(fast_gamma(fmaxf(tm.x, 0.0f)), fast_gamma(fmaxf(tm.y, 0.0f)),
+                              fast_gamma(fmaxf(tm.z, 0.0f)), 1.0f));
+    }
+}
+
+// ---------------------------------------------------------------------------
 // 3x3 convolution (forward, or input gradient with flipped weights)
 // ---------------------------------------------------------------------------
-enum ConvMode { kConvRelu = 0, kConvLinear = 1, kConvDgrad = 2 };
+// kConvKpn: last layer of inference; the logits stay on chip (LDS) and the softmax
+// 5x5 kernel is applied to the noisy taps staged with the tile.
+enum ConvMode { kConvRelu = 0, kConvLinear = 1, kConvDgrad = 2, kConvKpn = 4 };
 
 // Persistent: each workgroup keeps the layer's weights in registers and walks a
 // strided sequence of 16x16 tiles inside its XCD's contiguous share of the tile
@@ -189,12 +262,18 @@ enum ConvMode { kConvRelu = 0, kConvLinear = 1, kConvDgrad = 2 };
 template <int CIN, int MODE>
 __global__ void __launch_bounds__(256) k_conv3x3(CnnGeom g, const uint16_t* __restrict__ in,
                                                  const uint16_t* __restrict__ mask, const uint16_t* __restrict__ wgt,
-                                                 const float* __restrict__ bias, uint16_t* __restrict__ out) {
+                                                 const float* __restrict__ bias, uint16_t* __restrict__ out,
+                                                 pbrt_cnn_images im) {
     constexpr int kStride = CIN + 8;  // bf16 per LDS pixel: conflict-free 16 / 8 byte lane reads
     constexpr int kChunks = CIN / 8;
     constexpr int kTilePix = 18 * 18;
     constexpr int kLoads = (kTilePix * kChunks + 255) / 256;
+    constexpr int kNoisyRow = kTile + 4, kNoisyPix = kNoisyRow * kNoisyRow;  // kernel-prediction taps of a tile
+    constexpr int kNoisyLoads = MODE == kConvKpn ? (kNoisyPix + 255) / 256 : 1;
     __shared__ __attribute__((aligned(16))) uint16_t tile[2][kTilePix * kStride];
+    __shared__ __attribute__((aligned(16))) uint2 ntile[MODE == kConvKpn ? 2 : 1][MODE == kConvKpn ? kNoisyPix : 1];
+    __shared__ __attribute__((aligned(16))) uint16_t logit[MODE == kConvKpn ? kTile * kTile * kCh : 8];
+    uint2 nregs[kNoisyLoads];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int j = lane & 15, grp = lane >> 4;
     const int tiles_x = (g.width + kTile - 1) / kTile, tiles_y = (g.height + kTile - 1) / kTile;
@@ -208,6 +287,17 @@ __global__ void __launch_bounds__(256) k_conv3x3(CnnGeom g, const uint16_t* __re
     auto fetch = [&](int tt, uint4 (&r)[kLoads]) {
         const int img = tt / per_image, rem = tt % per_image;
         const int x0 = (rem % tiles_x) * kTile, y0 = (rem / tiles_x) * kTile;
+        if (MODE == kConvKpn) {
+#pragma unroll
+            for (int k = 0; k < kNoisyLoads; ++k) {
+                const int p = tid + k * 256;
+                if (p < kNoisyPix) {
+                    const int yy = min(max(y0 + p / kNoisyRow - 2, 0), g.height - 1);
+                    const int xx = min(max(x0 + p % kNoisyRow - 2, 0), g.width - 1);
+                    nregs[k] = reinterpret_cast<const uint2*>(im.noisy)[plane * img + (size_t)yy * g.width + xx];
+                }
+            }
+        }
         const uint16_t* src = in + plane * img * CIN;
         const uint16_t* msk = mask ? mask + plane * img * CIN : nullptr;
 #pragma unroll
@@ -226,6 +316,13 @@ __global__ void __launch_bounds__(256) k_conv3x3(CnnGeom g, const uint16_t* __re
         }
     };
     auto stash = [&](int b, const uint4 (&r)[kLoads]) {
+        if (MODE == kConvKpn) {
+#pragma unroll
+            for (int k = 0; k < kNoisyLoads; ++k) {
+                const int p = tid + k * 256;
+                if (p < kNoisyPix) ntile[b][p] = nregs[k];
+            }
+        }
 #pragma unroll
         for (int k = 0; k < kLoads; ++k) {
             const int e = tid + k * 256;
@@ -302,21 +399,50 @@ __global__ void __launch_bounds__(256) k_conv3x3(CnnGeom g, const uint16_t* __re
         const int img = t / per_image, rem = t % per_image;
         const int x0 = (rem % tiles_x) * kTile, y0 = (rem / tiles_x) * kTile;
         const int gx = x0 + j;
+        if (MODE == kConvKpn) {
+            // bf16 logits of the tile to LDS, then one thread per pixel filters the staged
+            // taps: the halo holds the clamped pixel at every position
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int gy = y0 + wave * 4 + r;
-            if (gx >= g.width || gy >= g.height) continue;
-            uint16_t* o = out + (plane * img + (size_t)gy * g.width + gx) * kCh;
+            for (int r = 0; r < 4; ++r) {
+                const int p = (wave * 4 + r) * kTile + j;
 #pragma unroll
-            for (int ct = 0; ct < 2; ++ct) {
-                float v[4];
+                for (int ct = 0; ct < 2; ++ct) {
+                    float v[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    v[i] = acc[r][ct][i] + bv[ct][i];
-                    if (MODE == kConvRelu) v[i] = fmaxf(v[i], 0.0f);
+                    for (int i = 0; i < 4; ++i) v[i] = acc[r][ct][i] + bv[ct][i];
+                    *reinterpret_cast<uint2*>(&logit[p * kCh + ct * 16 + 4 * grp]) =
+                        make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
                 }
-                *reinterpret_cast<uint2*>(o + ct * 16 + 4 * grp) =
-                    make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+            }
+            __syncthreads();
+            const int py = tid / kTile, px = tid % kTile;
+            if (x0 + px < g.width && y0 + py < g.height) {
+                KpnWeights k;
+                exact_logits(logit + tid * kCh, 0, k);
+                exact_exponentials<0, kKernelTaps>(k);
+                exact_normalise(k);
+                const uint2* taps = &ntile[buf][py * kNoisyRow + px];
+                const size_t i = plane * img + (size_t)(y0 + py) * g.width + x0 + px;
+                exact_apply(im, k, [&](int c) { return taps[(c / 5) * kNoisyRow + c % 5]; }, i,
+                            reinterpret_cast<const uint32_t*>(im.albedo)[i]);
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int gy = y0 + wave * 4 + r;
+                if (gx >= g.width || gy >= g.height) continue;
+                uint16_t* o = out + (plane * img + (size_t)gy * g.width + gx) * kCh;
+#pragma unroll
+                for (int ct = 0; ct < 2; ++ct) {
+                    float v[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        v[i] = acc[r][ct][i] + bv[ct][i];
+                        if (MODE == kConvRelu) v[i] = fmaxf(v[i], 0.0f);
+                    }
+                    *reinterpret_cast<uint2*>(o + ct * 16 + 4 * grp) =
+                        make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+                }
             }
         }
         if (tn < end) stash(buf ^ 1, regs);
@@ -641,13 +767,8 @@ LayerTable layer_table(int layers) {
     return lt;
 }
 
-// Softmax weights of one output pixel, not yet normalised.
-struct KpnWeights {
-    float e[kKernelTaps];
-    float sum;
-};
-
-// From its 25 bf16 logits (LDS, `logits`: 32 channels, 25 used).
+// Softmax weights from the 25 bf16 logits (LDS, `logits`: 32 channels, 25 used), by fast
+// exponentials.
 __device__ __forceinline__ KpnWeights kpn_weights(const uint16_t* logits) {
     // the 25 bf16 logits (and 7 padding channels): four 16-byte reads, twice
     // (maximum, then the weighted sum) to keep few registers live
@@ -1019,68 +1140,6 @@ __device__ __forceinline__ void pipe_conv(const CnnGeom& g, const PipeStrip& p, 
     }
 }
 
-// The softmax filter in the arithmetic of the training pass (k_kpn), so that a network gives
-// what it was trained to give: exponentials by expf, one division, normalised weights.
-// One pixel's bf16 logits (16-byte chunk q at q ^ swizzle), less their maximum:
-__device__ __forceinline__ void pipe_logits(const uint16_t* logits, int swizzle, KpnWeights& k) {
-    const uint4* lz = reinterpret_cast<const uint4*>(logits);
-    float zmax = -3.4e38f;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const uint4 v = lz[q ^ swizzle];
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int c = 8 * q + i;
-            if (c < kKernelTaps) {
-                k.e[c] = __uint_as_float((i & 1) ? (w[i / 2] & 0xFFFF0000u) : (w[i / 2] << 16));
-                zmax = fmaxf(zmax, k.e[c]);
-            }
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < kKernelTaps; ++c) k.e[c] -= zmax;
-    k.sum = 0.0f;
-}
-
-// The exponentials of taps kFrom .. kTo - 1 and their share of the sum:
-template <int kFrom, int kTo>
-__device__ __forceinline__ void pipe_exponentials(KpnWeights& k) {
-#pragma unroll
-    for (int c = kFrom; c < kTo; ++c) {
-        k.e[c] = expf(k.e[c]);
-        k.sum += k.e[c];
-    }
-}
-
-__device__ __forceinline__ void pipe_normalise(KpnWeights& k) {
-    const float inv = 1.0f / k.sum;
-#pragma unroll
-    for (int c = 0; c < kKernelTaps; ++c) k.e[c] *= inv;
-}
-
-// The weighted sum of the taps, stored as denoised radiance and / or final image:
-template <class Tap>
-__device__ __forceinline__ void pipe_apply(const pbrt_cnn_images& im, const KpnWeights& k, Tap tap, size_t i,
-                                           uint32_t albedo) {
-    vec3 o = make_vec3(0.0f);
-#pragma unroll
-    for (int c = 0; c < kKernelTaps; ++c) {
-        const uint2 nv = tap(c);
-        const half2v rg = __builtin_bit_cast(half2v, nv.x), ba = __builtin_bit_cast(half2v, nv.y);
-        o += make_vec3((float)rg.x, (float)rg.y, (float)ba.x) * k.e[c];
-    }
-    if (im.denoised) reinterpret_cast<float4*>(im.denoised)[i] = make_float4(o.x, o.y, o.z, 1.0f);
-    if (im.final_image) {
-        const uchar4 ac = __builtin_bit_cast(uchar4, albedo);
-        const vec3 alb = make_vec3(unorm8_to_float(ac.x), unorm8_to_float(ac.y), unorm8_to_float(ac.z));
-        const vec3 tm = (alb + make_vec3(1e-6f)) * o;
-        store_bgra8(im.final_image, i,
-                    make_vec4(fast_gamma(fmaxf(tm.x, 0.0f)), fast_gamma(fmaxf(tm.y, 0.0f)),
-                              fast_gamma(fmaxf(tm.z, 0.0f)), 1.0f));
-    }
-}
-
 // The four other waves, one per SIMD: each takes every fourth row, one step for its
 // features and three for its filter, so that no step is longer than a convolution wave's
 // and the SIMDs carry equal shares.  Turn t: the features of row t in step t; then, of the
@@ -1123,15 +1182,15 @@ __device__ __forceinline__ void pipe_pixels(const CnnGeom& g, const PipeStrip& p
         }
         if (t + 1 >= 0 && t + 1 < p.steps) {
             if (active) {
-                pipe_logits(S.act[L - 1][t & 1] + (c + 1) * kPipeStride, pipe_swizzle(c + 1), k);
-                pipe_exponentials<0, 10>(k);
+                exact_logits(S.act[L - 1][t & 1] + (c + 1) * kPipeStride, pipe_swizzle(c + 1), k);
+                exact_exponentials<0, 10>(k);
             }
             __syncthreads();
         }
         if (t + 2 >= 0 && t + 2 < p.steps) {
             if (active) {
-                pipe_exponentials<10, kKernelTaps>(k);
-                pipe_normalise(k);
+                exact_exponentials<10, kKernelTaps>(k);
+                exact_normalise(k);
             }
             __syncthreads();
         }
@@ -1140,7 +1199,7 @@ __device__ __forceinline__ void pipe_pixels(const CnnGeom& g, const PipeStrip& p
                 const uint2* taps[5];
 #pragma unroll
                 for (int q = 0; q < 5; ++q) taps[q] = &S.noisy[(o + q - 2) % kPipeRing][c - 2];
-                pipe_apply(im, k, [&](int q) { return taps[q / 5][q % 5]; }, i, albedo);
+                exact_apply(im, k, [&](int q) { return taps[q / 5][q % 5]; }, i, albedo);
             }
             __syncthreads();
         }
@@ -1429,10 +1488,10 @@ dim3 persistent_grid(K kernel, int tiles) {
 
 template <int CIN, int MODE>
 void launch_conv(const CnnGeom& g, const uint16_t* in, const uint16_t* mask, const uint16_t* w, const float* b,
-                 uint16_t* out, hipStream_t st) {
+                 uint16_t* out, hipStream_t st, const pbrt_cnn_images& im = pbrt_cnn_images{}) {
     const int tiles = ((g.width + kTile - 1) / kTile) * ((g.height + kTile - 1) / kTile) * g.count;
     const dim3 grid = persistent_grid(k_conv3x3<CIN, MODE>, tiles);
-    hipLaunchKernelGGL((k_conv3x3<CIN, MODE>), grid, dim3(256), 0, st, g, in, mask, w, b, out);
+    hipLaunchKernelGGL((k_conv3x3<CIN, MODE>), grid, dim3(256), 0, st, g, in, mask, w, b, out, im);
 }
 
 // inference of a two-layer network: one fused kernel, no workspace
@@ -1468,40 +1527,118 @@ void mask_pointwise_gradient(const pbrt_cnn* net, float* padded_grad, hipStream_
                        padded_grad + layer_offset(l), cin_pad(l));
 }
 
-// inference of three to six layers: the row pipeline, no workspace.  Strips are cut into
-// segments so that the workgroups (one per CU) fill whole rounds of the chip: of one to
-// eight rounds, the one with the fewest rows in all (a segment of r rows takes r + 3L + 3
-// steps with its halo and the pipeline's latency, an unfilled round idles CUs).
-template <int L>
-void launch_pipeline(const pbrt_cnn* net, const pbrt_cnn_images& im, hipStream_t st) {
-    const CnnGeom g{(int)im.width, (int)im.height, (int)im.count};
-    constexpr uint32_t out = kPipeCols - 2 * L;
-    const uint32_t strips_x = (im.width + out - 1) / out;
-    const uint64_t strips = (uint64_t)strips_x * im.count, cus = (uint64_t)compute_units();
-    PBRT_REQUIRE(strips < (1ull << 31), "pbrt_cnn_denoise: batch too large");
-    uint64_t best = ~0ull;
-    uint32_t rows = im.height;
+// The row pipeline's cut of a batch: strips of 64 - 2L columns in segments of `rows` rows, so
+// that the workgroups (one per CU) fill whole rounds of the chip: of one to eight rounds, the
+// one with the fewest rows in all (a segment of r rows takes r + 3L + 3 steps with its halo
+// and the pipeline's latency, an unfilled round idles CUs).
+struct PipePlan {
+    uint32_t strips_x, rows;
+    uint64_t strips, steps;
+};
+
+PipePlan plan_pipeline(int layers, const pbrt_cnn_images& im) {
+    const uint32_t out = (uint32_t)(kPipeCols - 2 * layers);
+    PipePlan p;
+    p.strips_x = (im.width + out - 1) / out;
+    p.strips = (uint64_t)p.strips_x * im.count;
+    p.steps = ~0ull;
+    p.rows = im.height;
+    const uint64_t cus = (uint64_t)compute_units();
     for (uint64_t rounds = 1; rounds <= 8; ++rounds) {
-        const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(rounds * cus / strips, 1), im.height);
+        const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(rounds * cus / p.strips, 1), im.height);
         const uint64_t r = (im.height + want - 1) / want, n = (im.height + r - 1) / r;
-        const uint64_t cost = (strips * n + cus - 1) / cus * (r + 3 * L + 3);
-        if (cost < best) {
-            best = cost;
-            rows = (uint32_t)r;
+        const uint64_t steps = (p.strips * n + cus - 1) / cus * (r + 3 * (uint64_t)layers + 3);
+        if (steps < p.steps) {
+            p.steps = steps;
+            p.rows = (uint32_t)r;
         }
     }
-    rows = std::max(rows, (im.height + 65534) / 65535);
-    const dim3 grid((uint32_t)strips, (im.height + rows - 1) / rows);
-    hipLaunchKernelGGL(k_pipeline<L>, grid, dim3(pipe_threads(L)), 0, st, g, im, net->wf.as<uint16_t>(),
-                       net->master.as<float>(), (int)rows, (int)strips_x);
+    p.rows = std::max(p.rows, (im.height + 65534) / 65535);
+    return p;
 }
 
-void forward_pipeline(const pbrt_cnn* net, const pbrt_cnn_images& im, hipStream_t st) {
+// Whether an image of the call's outputs shares bytes with one of its inputs.
+bool outputs_overlap_inputs(const pbrt_cnn_images& im) {
+    const size_t px = (size_t)im.width * im.height * im.count;
+    struct Range {
+        const void* p;
+        size_t bytes;
+    };
+    const Range in[] = {{im.noisy, px * 8}, {im.depth, px * 4},  {im.normal, px * 8},
+                        {im.albedo, px * 4}, {im.spp, px},       {im.motion, px * 4}};
+    const Range out[] = {{im.denoised, px * 16}, {im.final_image, px * 4}};
+    for (const Range& o : out)
+        for (const Range& i : in) {
+            const uintptr_t a = (uintptr_t)o.p, b = (uintptr_t)i.p;
+            if (o.p && a < b + i.bytes && b < a + o.bytes) return true;
+        }
+    return false;
+}
+
+// Inference of three to six layers is the same bits layer by layer or as the row pipeline.
+// The pipeline is the faster one except where its strips are mostly padding (images narrower
+// or much lower than a strip) or hold too few rows for its latency; estimated from what both
+// take on 256 CUs, within 12 % of the better one over 160 sizes of 3 to 6 layers: 16x16
+// images x 4096, 6 layers: 181 us by layers, 698 as a pipeline; 32x32 x 1024: 182 and 247;
+// 64x64 x 256: 185 and 199; 128x128 x 64: 185 and 174; 1920x1080: 369 and 238.
+//   The pipeline reads an image's borders while other workgroups already write their part of
+// it, so an output that shares memory with an input goes layer by layer, where every layer has
+// read what it needs before the last one writes.
+bool pipeline_suits(const PipePlan& p, int layers, const pbrt_cnn_images& im) {
+    const uint64_t cus = (uint64_t)compute_units();
+    const uint64_t tiles =
+        (uint64_t)((im.width + kTile - 1) / kTile) * ((im.height + kTile - 1) / kTile) * im.count;
+    const uint64_t px = (uint64_t)im.width * im.height * im.count;
+    const uint64_t n = (uint64_t)layers;
+    // a tile costs its share of the matrix products (whole tiles) and of the traffic (pixels)
+    const uint64_t by_layers_ns =
+        4500 * n + 1500 + (1350 * n + 1400) * (tiles + px / (kTile * kTile)) / (2 * cus);
+    const uint64_t pipeline_ns = 1300 + (120 * n + 470) * p.steps;
+    // a launch holds fewer than 2^32 work items on an axis
+    if (p.strips * (uint64_t)pipe_threads(layers) >= (1ull << 32)) return false;
+    return pipeline_ns <= by_layers_ns && !outputs_overlap_inputs(im);
+}
+
+template <int L>
+void launch_pipeline(const pbrt_cnn* net, const pbrt_cnn_images& im, const PipePlan& p, hipStream_t st) {
+    const CnnGeom g{(int)im.width, (int)im.height, (int)im.count};
+    const dim3 grid((uint32_t)p.strips, (im.height + p.rows - 1) / p.rows);
+    hipLaunchKernelGGL(k_pipeline<L>, grid, dim3(pipe_threads(L)), 0, st, g, im, net->wf.as<uint16_t>(),
+                       net->master.as<float>(), (int)p.rows, (int)p.strips_x);
+}
+
+// layer by layer, kernel prediction fused into the last one
+void forward_layers(const pbrt_cnn* net, const pbrt_cnn_images& im, const CnnWork& k, hipStream_t st) {
+    const CnnGeom g{(int)im.width, (int)im.height, (int)im.count};
+    const size_t px = (size_t)im.width * im.height * im.count;
+    hipLaunchKernelGGL(k_features, dim3((unsigned)((px + 255) / 256)), dim3(256), 0, st, g, im, k.feat);
+    const uint16_t* wf = net->wf.as<uint16_t>();
+    const float* master = net->master.as<float>();
+    const int layers = net->layers;
+    for (int l = 0; l < layers; ++l) {
+        const uint16_t* w = wf + weight_offset(l);
+        const float* b = master + layer_offset(l) + layer_weights(l);
+        if (l == 0)
+            launch_conv<kFeatCh, kConvRelu>(g, k.act[0], nullptr, w, b, k.act[1], st);
+        else if (l < layers - 1)
+            launch_conv<kCh, kConvRelu>(g, k.act[l], nullptr, w, b, k.act[l + 1], st);
+        else
+            launch_conv<kCh, kConvKpn>(g, k.act[l], nullptr, w, b, nullptr, st, im);
+    }
+}
+
+void forward_inference(const pbrt_cnn* net, const pbrt_cnn_images& im, hipStream_t st) {
+    const PipePlan p = plan_pipeline(net->layers, im);
+    if (!pipeline_suits(p, net->layers, im)) {
+        forward_layers(net, im,
+                       layout(im.width, im.height, im.count, false, net->layers, static_cast<char*>(im.workspace)), st);
+        return;
+    }
     switch (net->layers) {
-        case 3: launch_pipeline<3>(net, im, st); break;
-        case 4: launch_pipeline<4>(net, im, st); break;
-        case 5: launch_pipeline<5>(net, im, st); break;
-        default: launch_pipeline<6>(net, im, st); break;
+        case 3: launch_pipeline<3>(net, im, p, st); break;
+        case 4: launch_pipeline<4>(net, im, p, st); break;
+        case 5: launch_pipeline<5>(net, im, p, st); break;
+        default: launch_pipeline<6>(net, im, p, st); break;
     }
 }
 
@@ -1727,7 +1864,7 @@ extern "C" int32_t pbrt_cnn_denoise(const pbrt_cnn* net, const pbrt_cnn_images* 
             forward_two_layer(net, *im, st);
         } else {
             check_images(im, false, net->layers, "pbrt_cnn_denoise");
-            forward_pipeline(net, *im, st);
+            forward_inference(net, *im, st);
         }
         PBRT_HIP(hipGetLastError());
     });
