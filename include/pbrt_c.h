@@ -207,8 +207,9 @@ enum pbrt_tracer_kind {
     PBRT_TRACER_PERSISTENT = 2  /* megakernel with path regeneration: resident waves draw pixels
                                    from a frame counter, a lane whose path ends starts the next
                                    pixel (same per-pixel results as the megakernel) */
-    /* Uncounted traces of small frames (at most 131,072 pixels on 256 CUs) run one kernel of
-     * 32 pixels per wave for both megakernels, with the same per-pixel results. */
+    /* Uncounted traces of small frames (at most 65,536 pixels on 256 CUs) run one kernel of
+     * 32 pixels per wave for both megakernels, with the same per-pixel results (so
+     * pbrt_autotune_trace times that kernel twice, and either name runs it). */
 };
 
 typedef struct pbrt_trace_params {

@@ -312,10 +312,10 @@ def test_persistent_equals_megakernel(cuda, cfg1, w, h):
             assert a.tobytes() == b.tobytes(), f"{k} differs at {w}x{h} frame {frame}"
 
 
-@pytest.mark.parametrize("w,h", [(W, H), (61, 37), (1, 1), (200, 9), (9, 130), (512, 256), (520, 256), (640, 480)])
+@pytest.mark.parametrize("w,h", [(W, H), (61, 37), (1, 1), (200, 9), (9, 130), (264, 256), (512, 256), (520, 256), (640, 480)])
 @pytest.mark.parametrize("output", [capi.OUTPUT_DEMOD_ILLUMINATION_FLOAT, capi.OUTPUT_FINAL_IMAGE])
 def test_small_frame_tracer_equals_the_others(cuda, cfg1, w, h, output):
-    """Frames whose waves are all resident at once (512x256 is the largest on 256 CUs of 16
+    """Frames whose waves fill at most half of the chip (256x256 is the largest on 256 CUs of 16
     waves) are traced 32 pixels to a wave, shadow and next rays side by side; a counted
     trace runs the tracer it names.  Both, and the persistent tracer on either side of
     the limit, give the same bytes: every random draw and sum of a pixel is the same."""

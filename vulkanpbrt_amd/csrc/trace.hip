@@ -309,11 +309,10 @@ constexpr uint32_t kPairX = 8, kPairY = 4;  // pixels of a wave of pt_pairs
 // The chain is then one walk per vertex instead of two, and each waits for the longest of
 // 32 paths instead of 64.  The random draws and the radiance of a pixel are those of
 // pt_megakernel (the order of a vertex's draws does not depend on its shadow ray).
-//   At most 128 registers (four waves per SIMD, four of them spilled): with 141 the frames
-// of 110k to 131k pixels needed a second round of waves (480x270 589 us against 452).
-//   Megakernel and this, us per trace: Cornell box, 2 bounces: 96x72 280 -> 212, 256x256
-// 302 -> 226, 480x270 312 -> 257; atrium, 4 bounces: 160x90 445 -> 320, 384x216 518 -> 385;
-// city, 8 bounces: 480x270 686 -> 520.
+//   At most 128 registers (four waves per SIMD, four of them spilled): with 141 three fit, and
+// frames of more waves than those took a second round (480x270 589 us against 452).
+//   Megakernel and this, us per trace: Cornell box, 2 bounces: 96x72 278 -> 212, 256x256
+// 297 -> 219; atrium, 4 bounces: 96x72 388 -> 282, 160x90 445 -> 322, 256x256 476 -> 343.
 __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4))) pt_pairs(DeviceScene sc, TraceConsts c, PathImages img) {
     __shared__ int stack_mem[kTraversalStackSize * kTileThreads];
     const uint32_t lane = threadIdx.x, l = lane & 31u;
@@ -643,12 +642,16 @@ extern "C" int32_t pbrt_trace(const pbrt_scene* scene, const pbrt_trace_params* 
         TraceTiming* tm = scene_timing(scene);
         if (p->tracer == PBRT_TRACER_WAVEFRONT) {
             wavefront_trace(sc, scene_bvh_depth(scene), c, *img, counters, tm, p->block_threads, p->queue_paths, st);
-        } else if (!counters && (uint64_t)pair_grid.x * pair_grid.y <= resident_waves(pt_pairs)) {
-            // The whole frame's pairs of walks are resident at once: its time is its longest
-            // path's, which pt_pairs shortens.  Past that (131,072 pixels here) a second
-            // round of waves costs more than the pairs save: atrium 480x270 547 -> 452 us,
-            // 512x288 559 -> 606.  Counted traces keep the tracer they name, whose
-            // traversal counts they report.
+        } else if (!counters && (uint64_t)pair_grid.x * pair_grid.y <= resident_waves(pt_pairs) / 2) {
+            // The frame's pairs of walks fill at most half of the chip (65,536 pixels here): its
+            // time is its longest path's, which pt_pairs shortens, also when other streams
+            // trace at the same time.  Larger frames gain alone while their waves are all
+            // resident (atrium 480x270 545 -> 447 us), but on four streams at once the
+            // chip is full and the pairs' idle lanes cost more than they save.  us per
+            // frame with four streams, megakernel and pairs: atrium 200x150 0.74 of the
+            // megakernel's time, 320x180 0.93, 256x256 1.05, 320x240 1.11, 480x270 1.41;
+            // city 256x256 0.81, 480x270 1.24; Cornell box 256x256 0.95.  Counted traces
+            // keep the tracer they name, whose traversal counts they report.
             const PathImages images{img->depth, img->normal, img->material, img->albedo, illum};
             if (tm) tm->frame_begin(st);
             hipLaunchKernelGGL(pt_pairs, pair_grid, dim3(kTileThreads), 0, st, sc, c, images);
