@@ -155,11 +155,12 @@ def test_bmfr_householder_matches_oracle(cuda, oracle_lib, frames, bs):
     bad = np.argwhere(~feat_eq)
     for li, yy, xx in bad[:: max(1, len(bad) // 6)][:6]:
         print(f"  layer {li} padded ({yy},{xx}): gpu {feats[li, yy, xx]:04x} oracle {ofeats[li, yy, xx]:04x}")
-    # sin/cos (normal decode) differ by an ulp between the GPU and libm: fp16 stores may
-    # round the other way; every feature stays within 1 fp16 ulp.  Normals (0, 0, -1)
+    # sin/cos (normal decode) may differ by an ulp between the GPU and libm, and an fp16 store
+    # then round the other way; every feature stays within 1 fp16 ulp and all but a few are
+    # equal: the store rounds the FP32 value, as the oracle's does.  Normals (0, 0, -1)
     # decode to normal.y = sin(0) * sin(pi) = -0 on the CPU and +0 on the GPU; the sign of
     # a zero feature does not reach the fit (noise is added before it), so +-0 count equal.
-    assert (ulps == 0).mean() > 0.99 and ulps.max() <= 1
+    assert (ulps == 0).mean() > 0.9999 and ulps.max() <= 1
     # fit on the oracle's features (isolates the fit from sin/cos ulp differences)
     W32 = oracle_lib.bmfr_fit(W, H, bs, frame, feats, subgroup=64)
     W64 = oracle_lib.bmfr_lsq64(W, H, bs, frame, feats)
@@ -184,13 +185,14 @@ def test_bmfr_householder_matches_oracle(cuda, oracle_lib, frames, bs):
     assert d_ok.mean() > 0.999 and f_ok.mean() > 0.999
 
 
-@pytest.mark.parametrize("threads", [256, 512, 1024])
-@pytest.mark.parametrize("fit", ["f64", "f16"])
-def test_bmfr_gram_mfma_vs_fp64_lsq(cuda, oracle_lib, frames, fit, threads):
-    """Every Gram tile shape (workgroup size: the waves sharing a block's row chunks)
-    meets the same bound against FP64 least squares."""
+@pytest.mark.parametrize("fit,threads,bs", [(fit, threads, 32) for fit in ("f64", "f16") for threads in (256, 512, 1024)]
+                         + [("f64", threads, bs) for bs in (16, 8) for threads in (0, 256, 512, 1024)])
+def test_bmfr_gram_mfma_vs_fp64_lsq(cuda, oracle_lib, frames, fit, threads, bs):
+    """Every Gram tile shape (workgroup size: the waves sharing a block's row chunks; 0, the
+    default, is one wave for the FP64 fit of 16- and 8-pixel blocks) meets the same bound
+    against FP64 least squares."""
     inp = bmfr_inputs(oracle_lib, frames)
-    bs, frame = 32, 1
+    frame = 1
     denoised = np.zeros((2, H, W, 4), np.uint16)
     mode = capi.BMFR_FIT_GRAM_F64 if fit == "f64" else capi.BMFR_FIT_GRAM_F16
     _, weights, _, final = run_bmfr(cuda, mode, bs, frame, inp, denoised, threads)
@@ -211,8 +213,22 @@ def test_bmfr_gram_mfma_vs_fp64_lsq(cuda, oracle_lib, frames, fit, threads):
           f"under 1e-3 {np.mean(errs < 1e-3):.4f}; "
           f"weights rel error max {werrs.max():.3e} median {np.median(werrs):.3e}")
     if fit == "f64":
-        # tighter than the reference's own FP32 Householder on these blocks (~5e-5)
-        assert errs.max() < 5e-5
+        bar = 5e-5  # tighter than the reference's own FP32 Householder on these blocks (~5e-5)
+        if bs < 32:
+            # blocks of 256 and 64 rows are near-singular more often (the solve drops a feature
+            # whose pivot falls below 1e-15 of the largest): a quarter of that fit's error there.
+            # A feature rounded differently from the oracle's fails this (1.3e-3 at 16).
+            W32 = oracle_lib.bmfr_fit(W, H, bs, frame, feats, subgroup=64)
+            ref = 0.0
+            for by in range(nby):
+                for bx in range(nbx):
+                    A = oracle_lib.bmfr_block_matrix(W, H, bs, frame, feats, bx, by).astype(np.float64)[:, :10]
+                    f64 = A @ W64[by, bx].reshape(10, 3)
+                    r = A @ W32[by, bx].reshape(10, 3).astype(np.float64)
+                    ref = max(ref, np.abs(r - f64).max() / max(1e-2, np.abs(f64).max()))
+            print(f"bs {bs}: oracle fp32 householder {ref:.3e}")
+            bar = max(bar, ref / 4)
+        assert errs.max() < bar
     else:
         # FP32-accumulated Gram: accurate on well-conditioned blocks (75 of these 80 within
         # 1e-3, median 2.2e-6), a stated error on the planar / sky blocks where

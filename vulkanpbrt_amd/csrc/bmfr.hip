@@ -60,6 +60,15 @@ __device__ __forceinline__ vec3 bmfr_decode_normal(float theta, float phi) {
     return make_vec3(cp * st, sp * st, ct);
 }
 
+// `x` as the FP32 value that the reference stores to its fp16 feature image.  Without this the
+// compiler folds the product that gives a feature into the conversion (v_fma_mixlo_f16: one
+// rounding instead of two), in some kernels and not in others, and near-singular blocks show the
+// difference: 1e-3 of the fitted values on the worst 16-pixel block of a Cornell-box frame.
+__device__ __forceinline__ float as_float(float x) {
+    asm("" : "+v"(x));
+    return x;
+}
+
 // random(uint) of bmfrGeneral.comp:83-93 (Jenkins' 6-step integer hash)
 __device__ __forceinline__ float bmfr_random(uint32_t a) {
     a = (a + 0x7ed55d16u) + (a << 12);
@@ -220,7 +229,7 @@ __global__ void __launch_bounds__(1024) k_bmfr_pre(BmfrGeom g, pbrt_bmfr_images 
     const size_t plane = (size_t)g.wp * g.hp;
     const size_t at = (size_t)gy * g.wp + gx;
 #pragma unroll
-    for (int i = 0; i < kAlphaSize; ++i) g.features[i * plane + at] = f2h(f[i]);
+    for (int i = 0; i < kAlphaSize; ++i) g.features[i * plane + at] = f2h(as_float(f[i]));
 }
 
 // ---------------------------------------------------------------------------
@@ -779,7 +788,7 @@ __device__ __forceinline__ void bmfr_fit_raw_gram_block(const BmfrGeom& g, const
         }
 #pragma unroll
         for (int s = 0; s < kSub; ++s) {
-            float v = h2f(f2h(a[s][c]));
+            float v = h2f(f2h(c < kFeatures ? as_float(a[s][c]) : a[s][c]));
             if (c < kFeatures) v = __fadd_rn(v, nz[s]);
             a[s][c] = v;
         }
