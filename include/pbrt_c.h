@@ -407,10 +407,11 @@ typedef struct pbrt_bmfr_params {
     uint32_t block_size;     /* 8, 16 or 32 (DenoisingBlockSize X8 / X16 / X32) */
     uint32_t frame_number;   /* push constant frameNumber */
     uint32_t fit;            /* enum pbrt_bmfr_fit */
-    uint32_t fit_threads;    /* Gram fits: workgroup size 256, 512 or 1024 (0 = 256), i.e. how a
-                                block's rows are tiled over the waves' MFMA Gram accumulations;
-                                pbrt_autotune_bmfr picks it.  At 0 and 256 the FP64 fit of 16- and
-                                8-pixel blocks runs one wave per block. */
+    uint32_t fit_threads;    /* Gram fits: how a block's rows are tiled over the waves' MFMA Gram
+                                accumulations: workgroups of 512 or 1024 threads, or at 0 and 256
+                                the default, 256 threads, or for the FP64 fit of 8-pixel blocks, and
+                                of 16-pixel ones where a frame has many, one wave;
+                                pbrt_autotune_bmfr picks it. */
     uint32_t reserved[2];
 } pbrt_bmfr_params;
 
@@ -452,7 +453,7 @@ int32_t pbrt_bmfr(const pbrt_bmfr_params* params, const pbrt_bmfr_images* images
 int32_t pbrt_bmfr_noalloc(const pbrt_bmfr_params* params, const pbrt_bmfr_images* images, void* stream);
 
 /* Autotuner of the Gram fits' tile shape: runs pbrt_bmfr once per workgroup size
- * (256, 512, 1024 threads), `repeats` timed runs each after a warm-up, on `stream`,
+ * (256: the default, 512, 1024 threads), `repeats` timed runs each after a warm-up, on `stream`,
  * and returns the fastest as `best` (a copy of `params` with fit_threads set).  The
  * fit must be PBRT_BMFR_FIT_GRAM_F16 or _F64.  No counterpart in the reference
  * (BMFR.cpp:155-170 fixes fitting_kernel = 256).  Writes the images pbrt_bmfr writes;

@@ -1,4 +1,4 @@
-"""Batched BMFR (pbrt_bmfr_batched): every 32x32 block of many frames at uneven
+"""Batched BMFR (pbrt_bmfr_batched): every 32x32, 16x16 or 8x8 block of many frames at uneven
 resolutions fitted in one launch.  Each frame's weights, denoised and final images
 must equal, bit for bit, what pbrt_bmfr gives for that frame alone (the same
 per-block code runs in both); the per-block fit itself is checked against the FP64
@@ -58,10 +58,10 @@ def bmfr_images(f, ws=None, ws_bytes=0):
                                                       "denoised", "final")), capi.ptr(ws), ws_bytes)
 
 
-def run_batched(torch, frames, fit):
+def run_batched(torch, frames, fit, bs=32):
     arr = (capi.BmfrBatchFrame * len(frames))()
     for i, f in enumerate(frames):
-        arr[i].params = capi.BmfrParams(f["w"], f["h"], 32, f["frame"], fit)
+        arr[i].params = capi.BmfrParams(f["w"], f["h"], bs, f["frame"], fit)
         arr[i].images = bmfr_images(f)
     n = C.c_size_t()
     capi.check(capi.lib().pbrt_bmfr_batched_workspace_size(arr, len(frames), C.byref(n)))
@@ -73,8 +73,8 @@ def run_batched(torch, frames, fit):
     return ws, time.perf_counter() - t0
 
 
-def run_single(torch, f, fit):
-    p = capi.BmfrParams(f["w"], f["h"], 32, f["frame"], fit)
+def run_single(torch, f, fit, bs=32):
+    p = capi.BmfrParams(f["w"], f["h"], bs, f["frame"], fit)
     n = C.c_size_t()
     capi.check(capi.lib().pbrt_bmfr_workspace_size(C.byref(p), C.byref(n)))
     ws = torch.zeros(n.value, dtype=torch.uint8, device="cuda")
@@ -82,28 +82,28 @@ def run_single(torch, f, fit):
     return ws
 
 
-def check_batch(torch, frames, fit):
+def check_batch(torch, frames, fit, bs=32):
     snap = [(f["denoised"].clone(), f["final"].clone()) for f in frames]
-    ws, t_batch = run_batched(torch, frames, fit)
+    ws, t_batch = run_batched(torch, frames, fit, bs)
     batched = [(f["denoised"].clone(), f["final"].clone()) for f in frames]
     for f, (d, fi) in zip(frames, snap):  # restore the inputs of the single-frame runs
         f["denoised"].copy_(d)
         f["final"].copy_(fi)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
-    singles = [run_single(torch, f, fit) for f in frames]
+    singles = [run_single(torch, f, fit, bs) for f in frames]
     torch.cuda.synchronize()
     t_single = time.perf_counter() - t0
     a256 = lambda x: (x + 255) // 256 * 256
-    nbs = [(f["w"] // 32 + 2) * (f["h"] // 32 + 2) * 30 for f in frames]
-    noise = a256(4 * 10 * 32 * 32)  # the frame's noise table [10][32 * 32]
+    nbs = [(f["w"] // bs + 2) * (f["h"] // bs + 2) * 30 for f in frames]
+    noise = a256(4 * 10 * bs * bs)  # the frame's noise table [10][bs * bs]
     ranges = [a256(8 * (nb // 30)) for nb in nbs]  # each block's depth min and max
     # workspace: frame table, then per frame its weights, its noise table and its
     # blocks' depth ranges, each in its own 256-byte aligned region
     off = ws.numel() - sum(a256(4 * nb) + noise + r for nb, r in zip(nbs, ranges))
     for i, f in enumerate(frames):
         wb = ws[off:off + 4 * nbs[i]].view(torch.float32)
-        fb = a256(13 * (f["w"] // 32 + 2) * 32 * (f["h"] // 32 + 2) * 32 * 2)
+        fb = a256(13 * (f["w"] // bs + 2) * bs * (f["h"] // bs + 2) * bs * 2)
         w1 = singles[i][fb:fb + 4 * nbs[i]].view(torch.float32)
         assert torch.equal(wb, w1), f"frame {i} weights"
         assert torch.equal(batched[i][0], f["denoised"]), f"frame {i} denoised"
@@ -112,14 +112,18 @@ def check_batch(torch, frames, fit):
     return t_batch, t_single
 
 
+@pytest.mark.parametrize("bs", [32, 16, 8])
 @pytest.mark.parametrize("fit", ["f64", "f16"])
-def test_batched_equals_per_frame(cuda, scene1, fit):
+def test_batched_equals_per_frame(cuda, scene1, fit, bs):
+    """The batch and the single frame choose their workgroup size and lay their noise table
+    out for it separately: a table of another layout permutes the noise, so the weights
+    differ."""
     gen, scene = scene1
     rng = np.random.default_rng(7)
     sizes = [(int(rng.integers(64, 400)), int(rng.integers(64, 300))) for _ in range(6)]
     frames = [make_frame(cuda, gen, scene, w, h, k) for k, (w, h) in enumerate(sizes)]
     mode = capi.BMFR_FIT_GRAM_F64 if fit == "f64" else capi.BMFR_FIT_GRAM_F16
-    check_batch(cuda, frames, mode)
+    check_batch(cuda, frames, mode, bs)
 
 
 def test_batched_rejects_mixed_block_sizes(cuda, scene1):

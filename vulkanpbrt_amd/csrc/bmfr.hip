@@ -384,12 +384,19 @@ typedef double double4v __attribute__((ext_vector_type(4)));
 constexpr int kGramCols = 16;  // 13 columns (FP64: a0, 9 features, rgb; FP16: 9 projected features, rgb) + zeros
 constexpr int kFitThreads = 256;
 
-// Workgroup size of a Gram fit: as asked (256 by default), except that the FP64 fit of 16-
-// and 8-pixel blocks runs one wave per block by default: their 256 and 64 rows leave four
-// waves one row a lane or none, and one wave needs no barrier.  1920x1080, whole BMFR:
-// 16-pixel blocks 76 -> 61 us, 8-pixel blocks 192 -> 91 us.
-__host__ __device__ constexpr int gram_threads(bool f64, int bs, uint32_t asked) {
-    return f64 && bs < 32 && (asked == 0 || asked == 256) ? 64 : asked ? (int)asked : kFitThreads;
+// Workgroup size of a Gram fit of `blocks` blocks: as asked, and at 0 and 256 the default.
+// That is 256, except that the FP64 fit of 16- and 8-pixel blocks runs one wave per block:
+// their 256 and 64 rows leave four waves one row a lane or none, and one wave needs no
+// barrier.  1920x1080, whole BMFR: 16-pixel blocks 74 -> 59 us, 8-pixel blocks 187 -> 89 us.
+//   While there is no more than one 16-pixel block per SIMD, the fit takes as long as one block
+// does alone, and four waves load and convert its rows in a quarter of the steps (one wave
+// and four: 96x72 15.0 -> 14.2 us, 480x270 16.3 -> 15.6, 640x360 (1,008 blocks) 17.3 and
+// 17.2; 800x450 (1,560 blocks) 20.2 and 21.7).  Both give the same bits, so a batch (whose
+// blocks count together) equals its frames alone.
+__host__ constexpr int gram_threads(bool f64, int bs, uint32_t asked, uint32_t blocks, uint32_t cus) {
+    if (asked != 0 && asked != 256) return (int)asked;
+    if (!f64 || bs == 32) return kFitThreads;
+    return bs == 16 && blocks <= 4 * cus ? kFitThreads : 64;
 }
 
 // FP16 fit: wave-private staging of 64 rows (one per lane) as column-major fp16 hi / lo
@@ -802,6 +809,11 @@ __device__ __forceinline__ void bmfr_fit_raw_gram_block(const BmfrGeom& g, const
     //    Both operands hold the same values (lane l: row l / 4, column l % 4 of a group).
     //    1920x1080, whole BMFR: 63.5 -> 57.5 us.
     {
+        //    Four waves with one chunk of a 16-pixel block each exchange the staged rows and
+        //    divide the nine pairs instead, so that each sum runs over the block's rows in
+        //    order, as in one wave with four chunks.
+        constexpr bool kDividePairs = kRows == 256 && kThreads == 256;
+        const int part = __builtin_amdgcn_readfirstlane(wave);  // scalar: MFMA ignores the lane mask
         constexpr int kPairs = 9;
         constexpr int gi[kPairs] = {0, 0, 0, 0, 1, 1, 1, 2, 2}, gj[kPairs] = {0, 1, 2, 3, 1, 2, 3, 2, 3};
         double acc[kPairs];
@@ -819,35 +831,42 @@ __device__ __forceinline__ void bmfr_fit_raw_gram_block(const BmfrGeom& g, const
             for (int c = 0; c < 12; c += 4)
                 *reinterpret_cast<float4*>(dst + c) = make_float4(a[s][c], a[s][c + 1], a[s][c + 2], a[s][c + 3]);
             dst[12] = a[s][12];  // the columns past it reach only unused entries
-            wave_lds_sync();
+            if (kDividePairs)
+                __syncthreads();
+            else
+                wave_lds_sync();
+            constexpr int kChunks = kDividePairs ? 4 : 1;
 #pragma unroll
-            for (int ch = 0; ch < 4; ++ch) {
-                const float* src = &S.st[wave][ch * 16 + (lane >> 2)][lane & 3];
+            for (int ch = 0; ch < 4 * kChunks; ++ch) {
+                const float* src = &S.st[kDividePairs ? ch / 4 : wave][ch % 4 * 16 + (lane >> 2)][lane & 3];
                 double x[4];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) x[q] = (double)src[4 * q];
 #pragma unroll
                 for (int k = 0; k < kPairs; ++k)
-                    acc[k] = __builtin_amdgcn_mfma_f64_4x4x4f64(x[gi[k]], x[gj[k]], acc[k], 0, 0, 0);
+                    if (!kDividePairs || k % 4 == part)
+                        acc[k] = __builtin_amdgcn_mfma_f64_4x4x4f64(x[gi[k]], x[gj[k]], acc[k], 0, 0, 0);
             }
         }
         // lane 16 i + 4 b + j holds entry (i, j) of product b: summed over b
 #pragma unroll
         for (int k = 0; k < kPairs; ++k) {
+            if (kDividePairs && k % 4 != part) continue;
             acc[k] += dpp_move(acc[k], 0x128);  // row_ror 8
             acc[k] += dpp_move(acc[k], 0x124);  // row_ror 4
             if ((lane & 12) == 0)
-                S.gram[wave][(4 * gi[k] + (lane >> 4)) * kGramCols + 4 * gj[k] + (lane & 3)] = acc[k];
+                S.gram[kDividePairs ? 0 : wave][(4 * gi[k] + (lane >> 4)) * kGramCols + 4 * gj[k] + (lane & 3)] = acc[k];
         }
     }
     __syncthreads();
-    // 4. R summed over the waves; G by the rank-1 downdate
+    // 4. R summed over the waves' partial sums; G by the rank-1 downdate
+    constexpr int kParts = kRows == 256 && kThreads == 256 ? 1 : kWaves;
     constexpr int pw = kGramCols * kGramCols;
     const double* gr = &S.gram[0][0];
     auto rsum = [&](int i, int j) {  // i <= j
         double r = gr[i * kGramCols + j];
 #pragma unroll
-        for (int w = 1; w < kWaves; ++w) r += gr[w * pw + i * kGramCols + j];
+        for (int w = 1; w < kParts; ++w) r += gr[w * pw + i * kGramCols + j];
         return r;
     };
     const double r00 = rsum(0, 0), inv_r00 = 1.0 / r00;
@@ -1101,12 +1120,13 @@ static BmfrGeom make_geom(const pbrt_bmfr_params& p) {
 // The Gram fit for a block size and workgroup size (256, 512 or 1024 threads).
 template <bool kF64, int kThreads>
 static void launch_gram_rows(int bs, dim3 grid, hipStream_t st, const BmfrGeom& g, const pbrt_bmfr_images& im) {
-    if (bs == 32)
+    if (bs == 32) {
         hipLaunchKernelGGL((k_bmfr_fit_gram<1024, kF64, kThreads>), grid, dim3(kThreads), 0, st, g, im);
-    else if (bs == 16)
+    } else if (bs == 16) {
         hipLaunchKernelGGL((k_bmfr_fit_gram<256, kF64, kThreads>), grid, dim3(kThreads), 0, st, g, im);
-    else
+    } else if constexpr (!(kF64 && kThreads == kFitThreads)) {  // gram_threads gives 64 there
         hipLaunchKernelGGL((k_bmfr_fit_gram<64, kF64, kThreads>), grid, dim3(kThreads), 0, st, g, im);
+    }
 }
 
 template <bool kF64>
@@ -1165,7 +1185,8 @@ static void launch_bmfr(const pbrt_bmfr_params& p, const pbrt_bmfr_images& im, B
             hipLaunchKernelGGL((k_bmfr_fit_householder<1, 1>), grid, dim3(64), 0, st, g);
     } else {
         const int entries = kFeatures * g.bs * g.bs;
-        const int threads = gram_threads(p.fit == PBRT_BMFR_FIT_GRAM_F64, g.bs, p.fit_threads);
+        const int threads = gram_threads(p.fit == PBRT_BMFR_FIT_GRAM_F64, g.bs, p.fit_threads,
+                                         (uint32_t)(g.blocks_x * g.blocks_y), compute_units());
         hipLaunchKernelGGL(k_bmfr_noise, dim3((entries + 255) / 256), dim3(256), 0, st, g.frame, g.bs, threads,
                            g.noise);
         launch_gram_fit(p.fit == PBRT_BMFR_FIT_GRAM_F64, g.bs, (uint32_t)threads, grid, st, g, im);
@@ -1409,10 +1430,11 @@ extern "C" int32_t pbrt_bmfr_batched(const pbrt_bmfr_batch_frame* frames, uint32
         const dim3 grid(plan.blocks);
         const bool f64 = plan.fit == PBRT_BMFR_FIT_GRAM_F64;
         const int entries = kFeatures * plan.bs * plan.bs;
-        const int threads = gram_threads(f64, plan.bs, 0);
+        const int threads = gram_threads(f64, plan.bs, 0, plan.blocks, compute_units());
         hipLaunchKernelGGL(k_bmfr_noise_batched, dim3((entries + 255) / 256, count), dim3(256), 0, st, table, threads);
         auto fit = f64 ? (plan.bs == 32   ? k_bmfr_fit_gram_batched<1024, true, 256>
-                          : plan.bs == 16 ? k_bmfr_fit_gram_batched<256, true, 64>
+                          : plan.bs == 16 ? (threads == 64 ? k_bmfr_fit_gram_batched<256, true, 64>
+                                                           : k_bmfr_fit_gram_batched<256, true, 256>)
                                           : k_bmfr_fit_gram_batched<64, true, 64>)
                        : (plan.bs == 32   ? k_bmfr_fit_gram_batched<1024, false, 256>
                           : plan.bs == 16 ? k_bmfr_fit_gram_batched<256, false, 256>

@@ -59,6 +59,17 @@ int32_t guard(F&& body) {
     }
 }
 
+// Compute units of the GPU current at the first call (every GPU of a node is the same).
+inline uint32_t compute_units() {
+    static const uint32_t n = [] {
+        int dev = 0, cus = 0;
+        PBRT_HIP(hipGetDevice(&dev));
+        PBRT_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        return (uint32_t)(cus > 0 ? cus : 1);
+    }();
+    return n;
+}
+
 // Device buffer owned by a C ABI object.
 struct DeviceBuffer {
     void* ptr = nullptr;

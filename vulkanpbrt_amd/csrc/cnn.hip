@@ -1465,23 +1465,13 @@ void check_images(const pbrt_cnn_images* im, bool training, int layers, const ch
     PBRT_REQUIRE(im->workspace && im->workspace_bytes >= need, std::string(fn) + ": workspace too small");
 }
 
-int compute_units() {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        PBRT_HIP(hipGetDevice(&dev));
-        PBRT_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    }
-    return std::max(cus, 1);
-}
-
 // Workgroups for a persistent convolution: every CU's resident share, a multiple of
 // the 8 XCDs, no more than the tiles.
 template <class K>
 dim3 persistent_grid(K kernel, int tiles) {
     int per_cu = 0;
     PBRT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, 0));
-    int blocks = std::max(1, compute_units() * std::max(per_cu, 1));
+    int blocks = (int)compute_units() * std::max(per_cu, 1);
     blocks = std::min(blocks, ((tiles + 7) / 8) * 8);
     return dim3((unsigned)(((blocks + 7) / 8) * 8));
 }
@@ -1543,7 +1533,7 @@ PipePlan plan_pipeline(int layers, const pbrt_cnn_images& im) {
     p.strips = (uint64_t)p.strips_x * im.count;
     p.steps = ~0ull;
     p.rows = im.height;
-    const uint64_t cus = (uint64_t)compute_units();
+    const uint64_t cus = compute_units();
     for (uint64_t rounds = 1; rounds <= 8; ++rounds) {
         const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(rounds * cus / p.strips, 1), im.height);
         const uint64_t r = (im.height + want - 1) / want, n = (im.height + r - 1) / r;
@@ -1585,7 +1575,7 @@ bool outputs_overlap_inputs(const pbrt_cnn_images& im) {
 // it, so an output that shares memory with an input goes layer by layer, where every layer has
 // read what it needs before the last one writes.
 bool pipeline_suits(const PipePlan& p, int layers, const pbrt_cnn_images& im) {
-    const uint64_t cus = (uint64_t)compute_units();
+    const uint64_t cus = compute_units();
     const uint64_t tiles =
         (uint64_t)((im.width + kTile - 1) / kTile) * ((im.height + kTile - 1) / kTile) * im.count;
     const uint64_t px = (uint64_t)im.width * im.height * im.count;
