@@ -88,7 +88,7 @@ def test_lbvh_queries_match_sah(cuda, pbrt_lib, config, builder):
     assert l.triangle_count == s.triangle_count and 1 < l.bvh_depth <= 40  # the traversal stack
     if builder in ("lbvh", "ploc"):
         assert l.bvh_node_count == l.triangle_count - 1
-    rays, pc = scene_rays(gen, 320, 180, 40000, config)
+    rays, _ = scene_rays(gen, 320, 180, 40000, config)
     hs, os_ = intersect(cuda, sah, rays)
     hl, ol = intersect(cuda, lb, rays)
     ts, tl = hs[:, 0].view(np.float32), hl[:, 0].view(np.float32)
@@ -104,17 +104,20 @@ def test_lbvh_queries_match_sah(cuda, pbrt_lib, config, builder):
     # (the atrium's PLOC and LBVH trees) the 40-entry build, so config 2 compares the two
     print(f"megakernel stacks: SAH tree {32 if s.bvh_depth <= 32 else 40} entries, "
           f"{builder} tree {32 if l.bvh_depth <= 32 else 40} entries")
-    imgs = []
-    for sc in (sah, lb):
-        img = helpers.gbuffer(cuda, 320, 180)
-        helpers.trace(cuda, sc, pc, img, 320, 180)
-        cuda.cuda.synchronize()
-        imgs.append(img["illumination"].cpu().numpy())
-    eq = np.all(imgs[0] == imgs[1], axis=-1).mean()
-    # pixels whose path meets an equal-t tie (coplanar instanced boxes and walls in the
-    # atrium) shade the other surface; every other pixel is bit-identical
-    print(f"traced frame: identical pixels {eq:.5f}")
-    assert eq > 0.995
+    # (frames of up to 65,536 pixels run the small-frame kernel over either tree)
+    for w, h in ((320, 180), (640, 360)):
+        pc, _, _ = helpers.frame_push_constants(gen, w, h, 0)
+        imgs = []
+        for sc in (sah, lb):
+            img = helpers.gbuffer(cuda, w, h)
+            helpers.trace(cuda, sc, pc, img, w, h)
+            cuda.cuda.synchronize()
+            imgs.append(img["illumination"].cpu().numpy())
+        eq = np.all(imgs[0] == imgs[1], axis=-1).mean()
+        # pixels whose path meets an equal-t tie (coplanar instanced boxes and walls in the
+        # atrium) shade the other surface; every other pixel is bit-identical
+        print(f"traced frame {w}x{h}: identical pixels {eq:.5f}")
+        assert eq > 0.995
     sah.close()
     lb.close()
 

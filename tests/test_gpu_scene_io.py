@@ -21,6 +21,8 @@ from vulkanpbrt_amd import camera, capi, scene_export
 pytestmark = pytest.mark.gpu
 
 N = 96
+# Frames of at most 65,536 pixels run the small-frame kernel for the megakernel; this one is past it.
+LARGE_N = 365
 
 
 def _box_scene(d):
@@ -58,9 +60,10 @@ def _pose(eye, center, fovy=50.0):
     return p
 
 
-@pytest.mark.parametrize("tracer", ["megakernel", "wavefront"])
+@pytest.mark.parametrize("tracer,size", [("megakernel", N), ("wavefront", N), ("megakernel", LARGE_N),
+                                         ("persistent", LARGE_N)])
 @pytest.mark.parametrize("instanced", [False, True])
-def test_loaded_scene_matches_the_oracle(cuda, pbrt_lib, oracle_lib, tmp_path, tracer, instanced):
+def test_loaded_scene_matches_the_oracle(cuda, pbrt_lib, oracle_lib, tmp_path, tracer, size, instanced):
     _box_scene(tmp_path)
     xf = None
     if instanced:
@@ -75,17 +78,17 @@ def test_loaded_scene_matches_the_oracle(cuda, pbrt_lib, oracle_lib, tmp_path, t
     assert st.triangle_count == 18 and info.triangle_count == 18 * (2 if instanced else 1)
     osc = oracle_lib.OracleScene(loaded.desc)
     assert info.light_count == osc.light_count
-    kind = capi.TRACER_WAVEFRONT if tracer == "wavefront" else capi.TRACER_MEGAKERNEL
-    view, proj = camera.pose_matrices(_pose([0.0, -3.2, 1.0], [0.0, 0.0, 0.9]), N, N)
+    kind = helpers.tracer_kind(tracer)
+    view, proj = camera.pose_matrices(_pose([0.0, -3.2, 1.0], [0.0, 0.0, 0.9]), size, size)
     glass_sum = np.zeros((2, 3))
     glass_px = 0
     for frame in range(8):
         pc = camera.push_constants(view, proj, view, frame)
-        img = helpers.gbuffer(cuda, N, N)
-        helpers.trace(cuda, scene, pc, img, N, N, max_depth=2, tracer=kind)
+        img = helpers.gbuffer(cuda, size, size)
+        helpers.trace(cuda, scene, pc, img, size, size, max_depth=2, tracer=kind)
         cuda.cuda.synchronize()
         gpu = helpers.to_np(img)
-        ref = osc.trace(N, N, np.array(pc.view_inverse[:], np.float32), np.array(pc.proj_inverse[:], np.float32),
+        ref = osc.trace(size, size, np.array(pc.view_inverse[:], np.float32), np.array(pc.proj_inverse[:], np.float32),
                         frame=frame, precision=32)
         # primary hits on the glass (albedo Kd + Ks saturates): paths that refract
         # through the tetrahedron, bounce inside it (transmissive hits do not count
@@ -158,8 +161,11 @@ def test_wavefront_equals_megakernel_with_glass(cuda, pbrt_lib, tmp_path):
     assert (rel.max(-1) <= 1e-5).mean() >= 0.999
 
 
-@pytest.mark.parametrize("tw,th", [(1, 5), (2, 1), (2, 2), (3, 7), (17, 5)])
-def test_texture_taps_wrap_at_every_width(cuda, pbrt_lib, oracle_lib, tmp_path, tw, th):
+@pytest.mark.parametrize("tw,th,size,tracer", [(1, 5, N, "megakernel"), (2, 1, N, "megakernel"), (2, 2, N, "megakernel"),
+                                               (3, 7, N, "megakernel"), (17, 5, N, "megakernel"),
+                                               (1, 5, LARGE_N, "megakernel"), (3, 7, LARGE_N, "megakernel"),
+                                               (1, 5, LARGE_N, "persistent"), (3, 7, LARGE_N, "persistent")])
+def test_texture_taps_wrap_at_every_width(cuda, pbrt_lib, oracle_lib, tmp_path, tw, th, size, tracer):
     """Bilinear taps that are neighbours in a row come in one load, those across the wrap in
     two: textures of one, two and odd numbers of texels a row, tiled on both sides of zero."""
     _box_scene(tmp_path)
@@ -175,16 +181,16 @@ def test_texture_taps_wrap_at_every_width(cuda, pbrt_lib, oracle_lib, tmp_path, 
     loaded = capi.LoadedScene(tmp_path / "box.obj")
     scene = capi.Scene(loaded.desc, keepalive=loaded)
     osc = oracle_lib.OracleScene(loaded.desc)
-    view, proj = camera.pose_matrices(_pose([0.6, -1.6, 0.7], [0.6, 0.6, 0.6]), N, N)
+    view, proj = camera.pose_matrices(_pose([0.6, -1.6, 0.7], [0.6, 0.6, 0.6]), size, size)
     pc = camera.push_constants(view, proj, view, 1)
-    img = helpers.gbuffer(cuda, N, N)
-    helpers.trace(cuda, scene, pc, img, N, N, max_depth=2)
+    img = helpers.gbuffer(cuda, size, size)
+    helpers.trace(cuda, scene, pc, img, size, size, max_depth=2, tracer=helpers.tracer_kind(tracer))
     cuda.cuda.synchronize()
     gpu = helpers.to_np(img)
-    ref = osc.trace(N, N, np.array(pc.view_inverse[:], np.float32), np.array(pc.proj_inverse[:], np.float32), frame=1,
+    ref = osc.trace(size, size, np.array(pc.view_inverse[:], np.float32), np.array(pc.proj_inverse[:], np.float32), frame=1,
                     precision=32)
     glass = np.all(gpu["albedo"][..., :3] == 255, axis=-1)
     keys = ("depth", "albedo", "illumination")
-    frac = _compare_frame({k: gpu[k][~glass] for k in keys}, {k: ref[k][~glass] for k in keys}, f"texture {tw}x{th}")
+    frac = _compare_frame({k: gpu[k][~glass] for k in keys}, {k: ref[k][~glass] for k in keys}, f"texture {tw}x{th} {tracer}")
     _assert_mirror_exact(frac)
     assert len(np.unique(gpu["albedo"].reshape(-1, 4), axis=0)) > (20 if tw * th > 2 else 2)

@@ -20,6 +20,15 @@ from tests import helpers
 pytestmark = pytest.mark.gpu
 
 W = H = 256
+# A frame past the 65,536 pixels up to which uncounted traces of either megakernel run the
+# small-frame kernel: here the tracer named is the one that runs.  No round size.
+LARGE = (523, 257)
+
+
+def assert_past_small_frames(torch, w, h):
+    """No device keeps more than 16 waves of the small-frame kernel (8x4 pixels each) per CU."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert ((w + 7) // 8) * ((h + 3) // 4) > 16 * cus
 
 
 @pytest.fixture(scope="module")
@@ -157,15 +166,18 @@ def _assert_mirror_exact(frac):
 
 @pytest.mark.parametrize("tracer", helpers.TRACERS)
 @pytest.mark.parametrize("frame", [0, 5])
-def test_tracer_matches_fp32_mirror(cuda, cfg1, frame, tracer):
+@pytest.mark.parametrize("w,h", [(W, H), LARGE])
+def test_tracer_matches_fp32_mirror(cuda, cfg1, frame, tracer, w, h):
+    """Cornell box, 2 bounces.  At 256x256 both megakernels run the small-frame kernel, past
+    its limit the tracer named."""
     gen, scene, osc = cfg1
-    pc, _, _ = helpers.frame_push_constants(gen, W, H, frame)
-    img = helpers.gbuffer(cuda, W, H)
+    pc, _, _ = helpers.frame_push_constants(gen, w, h, frame)
+    img = helpers.gbuffer(cuda, w, h)
     kind = helpers.tracer_kind(tracer)
-    helpers.trace(cuda, scene, pc, img, W, H, tracer=kind)
+    helpers.trace(cuda, scene, pc, img, w, h, tracer=kind)
     cuda.cuda.synchronize()
     gpu = helpers.to_np(img)
-    ref = osc.trace(W, H, np.array(pc.view_inverse[:], np.float32), np.array(pc.proj_inverse[:], np.float32),
+    ref = osc.trace(w, h, np.array(pc.view_inverse[:], np.float32), np.array(pc.proj_inverse[:], np.float32),
                     frame=frame, precision=32)
     frac = _compare_frame(gpu, ref, f"{tracer} frame {frame}")
     _assert_mirror_exact(frac)
@@ -173,12 +185,13 @@ def test_tracer_matches_fp32_mirror(cuda, cfg1, frame, tracer):
 
 @pytest.mark.parametrize("tracer", helpers.TRACERS)
 @pytest.mark.parametrize("mode", [capi.LIGHT_SAMPLE_LIGHT_STRENGTH, capi.LIGHT_SAMPLE_UNIFORM])
-def test_light_sampling_modes_match_fp32_mirror(cuda, cfg1, tracer, mode):
+@pytest.mark.parametrize("w,h", [(128, 128), LARGE])
+def test_light_sampling_modes_match_fp32_mirror(cuda, cfg1, tracer, mode, w, h):
     """The other two light samplers (lighting.glsl:98-168 by light strength, :170-227
     uniform; the host picks uniform above 800 lights) against the oracle run in the
-    same mode."""
+    same mode; the smaller frame runs the small-frame kernel for both megakernels, the
+    larger one the tracer named."""
     gen, scene, osc = cfg1
-    w = h = 128
     pc, _, _ = helpers.frame_push_constants(gen, w, h, 2)
     img = helpers.gbuffer(cuda, w, h)
     kind = helpers.tracer_kind(tracer)
@@ -197,13 +210,13 @@ def test_light_sampling_modes_match_fp32_mirror(cuda, cfg1, tracer, mode):
 
 
 @pytest.mark.parametrize("tracer", helpers.TRACERS)
-def test_final_image_output_matches_fp32_mirror(cuda, cfg1, tracer):
+@pytest.mark.parametrize("w,h", [(96, 96), LARGE])
+def test_final_image_output_matches_fp32_mirror(cuda, cfg1, tracer, w, h):
     """The tracer's own progressive output (PBRT_OUTPUT_FINAL_IMAGE, ptRaygen.rgen:84-103):
     sample 0 writes the gamma-encoded radiance; later samples jitter the camera ray
     and blend with the previous image in linear space.  Each sample is checked against
     the oracle given the same previous image."""
     gen, scene, osc = cfg1
-    w = h = 96
     kind = helpers.tracer_kind(tracer)
     img = helpers.gbuffer(cuda, w, h)
     prev = np.zeros((h, w, 4), np.float32)
@@ -221,18 +234,25 @@ def test_final_image_output_matches_fp32_mirror(cuda, cfg1, tracer):
         prev = gpu["illumination"].copy()
 
 
-def test_atrium_matches_fp32_mirror(cuda, pbrt_lib, oracle_lib):
+@pytest.mark.parametrize("w,h,builder", [(128, 72, capi.PBRT_BVH_SBVH_HOST), (*LARGE, capi.PBRT_BVH_SBVH_HOST),
+                                         (*LARGE, capi.PBRT_BVH_PLOC_GPU)])
+def test_atrium_matches_fp32_mirror(cuda, pbrt_lib, oracle_lib, w, h, builder):
     """The atrium (instanced geometry, 1024x1024 textures with alpha masks taken by the
-    any-hit test, three area lights and a sun, spatial-split tree) at 128x72, 4 bounces.
+    any-hit test, three area lights and a sun), 4 bounces: a frame of the small-frame kernel
+    and one past its limit, over a spatial-split tree of depth <= 32 (the megakernel's
+    32-entry stack) and over the device-built PLOC tree, deeper than that (its 40-entry one).
     Four bounces through 262k triangles make this frame sensitive to FP32 rounding (the
     oracle's own FP64 run agrees with its FP32 mirror on ~89 % of the pixels' radiance),
     but the tracer and the mirror evaluate the same FP32 operations -- the same
     ray/triangle test on the same triangle records, the same transcendental
     polynomials -- so the bar is the mirror's frame bit for bit."""
     gen = capi.GeneratedScene(2, 2)
+    gen.desc.bvh_builder = builder
     scene = capi.Scene(gen.desc)
+    assert (scene.info().bvh_depth > 32) == (builder == capi.PBRT_BVH_PLOC_GPU)
+    if (w, h) == LARGE:
+        assert_past_small_frames(cuda, w, h)
     osc = oracle_lib.OracleScene(gen.desc)
-    w, h = 128, 72
     pc, _, _ = helpers.frame_push_constants(gen, w, h, 7)
     iv, ip = np.array(pc.view_inverse[:], np.float32), np.array(pc.proj_inverse[:], np.float32)
     ref = osc.trace(w, h, iv, ip, frame=7, max_depth=4, precision=32)
@@ -291,21 +311,26 @@ def test_wavefront_counts_rays(cuda, cfg1):
     assert np.array_equal(counts[capi.TRACER_PERSISTENT], mk)
 
 
-@pytest.mark.parametrize("w,h", [(W, H), (61, 37), (1, 1), (200, 9)])
+@pytest.mark.parametrize("w,h", [(W, H), (61, 37), (1, 1), (200, 9), LARGE, (640, 480), (1021, 577)])
 def test_persistent_equals_megakernel(cuda, cfg1, w, h):
     """The persistent tracer draws pixels from a per-launch counter that its last wave
     clears: frames traced back to back (different sizes and frames in between) are
     byte-identical to the megakernel's, so every pixel is traced exactly once per
-    launch and the counter starts from zero each time."""
+    launch and the counter starts from zero each time.  That is from 523x257 on; smaller
+    frames run the small-frame kernel under either name, which leaves the counter alone."""
     gen, scene, _ = cfg1
+    ow, oh = (13, 11) if w * h <= W * H else (701, 397)
+    if w * h > W * H:
+        assert_past_small_frames(cuda, w, h)
+        assert_past_small_frames(cuda, ow, oh)
     for frame in (0, 3, 3):
         pc, _, _ = helpers.frame_push_constants(gen, w, h, frame)
         ref = helpers.gbuffer(cuda, w, h)
         helpers.trace(cuda, scene, pc, ref, w, h, max_depth=3, tracer=capi.TRACER_MEGAKERNEL)
         img = {k: cuda.full_like(v, 7) for k, v in helpers.gbuffer(cuda, w, h).items()}
         helpers.trace(cuda, scene, pc, img, w, h, max_depth=3, tracer=capi.TRACER_PERSISTENT)
-        other = helpers.gbuffer(cuda, 13, 11)  # another size between the launches
-        helpers.trace(cuda, scene, pc, other, 13, 11, tracer=capi.TRACER_PERSISTENT)
+        other = helpers.gbuffer(cuda, ow, oh)  # another size between the launches
+        helpers.trace(cuda, scene, pc, other, ow, oh, tracer=capi.TRACER_PERSISTENT)
         cuda.cuda.synchronize()
         for k in ref:
             a, b = ref[k].cpu().numpy(), img[k].cpu().numpy()
