@@ -46,7 +46,7 @@ __device__ __forceinline__ int mirror_coord(int x, int s) {
     return x;
 }
 
-__device__ __forceinline__ int wrap_coord(int i, int n) {
+PBRT_HD int wrap_coord(int i, int n) {
     int r = i % n;
     return r < 0 ? r + n : r;
 }
@@ -55,7 +55,7 @@ __device__ __forceinline__ int wrap_coord(int i, int n) {
 // addressing.  Within one image of the origin (reprojected positions are) they wrap by one
 // addition and one compare; the integer remainders of the general case are some twenty
 // instructions each, four to a fetch.
-__device__ __forceinline__ void wrap_pair(int i, int n, int& i0, int& i1) {
+PBRT_HD void wrap_pair(int i, int n, int& i0, int& i1) {
     if ((uint32_t)i + (uint32_t)n < 2u * (uint32_t)n) {  // -n <= i < n
         i0 = i < 0 ? i + n : i;
         i1 = i0 + 1 == n ? 0 : i0 + 1;
