@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(64 * kW) k_bfr(BfrGeom g, pbrt_bfr_images im) 
         if (kW > 1)
             __syncthreads();
         else
-            __builtin_amdgcn_wave_barrier();  // LDS operations of one wave complete in order
+            wave_lds_sync();
         float gj = 0.0f;
         if (lane < kBfrSums) {
             if constexpr (kParts == 4) {
@@ -247,7 +247,7 @@ __global__ void __launch_bounds__(64 * kW) k_bfr(BfrGeom g, pbrt_bfr_images im) 
                 gj = slot[lane];
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        if (kW == 1) wave_lds_sync();  // one slot: read before the next step's sums are written
         const float step = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(step_lane), it));
         m = b1_mix * m + (1.0f - kBeta1) * gj;
         v = b2_mix * v + (1.0f - kBeta2) * (gj * gj);

@@ -165,13 +165,6 @@ struct OpAdd {
     __device__ T operator()(T a, T b) const { return a + b; }
 };
 
-// LDS written by some lanes of a wave and then read by others of the same wave.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 struct PixelIn {
     float depth;
     vec3 normal;

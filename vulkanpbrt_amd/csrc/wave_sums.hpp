@@ -12,6 +12,15 @@
 
 namespace pbrt {
 
+// LDS written by some lanes of a wave and then read by others of the same wave, or read
+// and then written again: the hardware completes a wave's LDS operations in order, and the
+// fences keep the compiler from moving them past each other.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ float swap_add32(float a, float b) {
     // lanes 0..31: a[l] + a[l ^ 32]; lanes 32..63: b[l] + b[l ^ 32]
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
