@@ -75,3 +75,20 @@ def test_bmfr_noalloc_rejects_oversized_frames_without_gpu(pbrt_lib):
     im = capi.BmfrImages(*fake, None, 0)
     assert pbrt_lib.pbrt_bmfr_noalloc(C.byref(p), C.byref(im), None) == capi.PBRT_ERR_INVALID_ARG
     assert b"scratch" in pbrt_lib.pbrt_last_error()
+
+
+def test_cnn_training_workspace_holds_one_partial_per_workgroup(pbrt_lib):
+    """Training scratch: bf16 features, activations and two gradients per pixel, a partial sum
+    of each 256 pixels' loss, the gradient, and one weight-gradient partial (37 KB) for each
+    of the at most 512 workgroups that write one, however many 16x16 tiles the batch has."""
+    def size(w, h, count):
+        n = C.c_size_t()
+        capi.check(pbrt_lib.pbrt_cnn_workspace_size(w, h, count, 1, C.byref(n)))
+        return n.value
+
+    partial = 4 * (9 * 32 * 32 + 32)
+    for w, h, count in ((128, 128, 8), (512, 512, 8), (1920, 1080, 2)):
+        px, tiles = w * h * count, -(-w // 16) * -(-h // 16) * count
+        pixels = px * 2 * (16 + 6 * 32 + 2 * 32) + 4 * -(-px // 256)
+        gradient = 4 * (9 * 32 * (16 + 5 * 32) + 6 * 32)
+        assert 0 <= size(w, h, count) - (pixels + gradient + min(tiles, 512) * partial) < 16 * 256

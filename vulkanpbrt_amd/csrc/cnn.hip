@@ -1401,7 +1401,7 @@ struct CnnWork {
     uint16_t* feat;
     uint16_t* act[kMaxLayers + 1];  // act[0] = feat; act[1..L-1] hidden, act[L] logits
     uint16_t* grad_act[2];       // training: upstream gradients (ping-pong)
-    float* partial;              // training: per-tile weight-gradient partials
+    float* partial;              // training: a weight-gradient partial per workgroup
     float* loss_part;
     float* grad;                 // training: padded gradient
     size_t bytes;
@@ -1423,11 +1423,11 @@ CnnWork layout(uint32_t w, uint32_t h, uint32_t count, bool training, int layers
         k.grad_act[0] = (uint16_t*)take(px * kCh * 2);
         k.grad_act[1] = (uint16_t*)take(px * kCh * 2);
         const size_t tiles = (size_t)((w + kTile - 1) / kTile) * ((h + kTile - 1) / kTile) * count;
-        k.partial = (float*)take(tiles * (kTaps * kCh * kCh + kCh) * 4);
+        k.partial = (float*)take(std::min<size_t>(tiles, kWgradGrid) * (kTaps * kCh * kCh + kCh) * 4);
         k.loss_part = (float*)take(((px + 255) / 256) * 4);
         k.grad = (float*)take(master_size(layers) * 4);
     } else {
-        // ping-pong hidden activations; logits in the second buffer
+        // the layer-by-layer route: ping-pong hidden activations (the logits stay in LDS)
         uint16_t* a = (uint16_t*)take(px * kCh * 2);
         uint16_t* b = (uint16_t*)take(px * kCh * 2);
         for (int l = 1; l <= layers; ++l) k.act[l] = (l & 1) ? a : b;
