@@ -51,13 +51,79 @@ __device__ __forceinline__ vec3 nee_inline(const DeviceScene& sc, uint32_t mode,
     return nee_unshadowed(ls, o, s, throughput);
 }
 
+// The images a path writes.
+struct PathImages {
+    float* depth;
+    float* normal;
+    uint8_t* material;
+    uint8_t* albedo;
+    float4* illum;
+};
+
+// The primary hit's G-buffer (ptRaygen.rgen:44-66).
+__device__ __forceinline__ void write_gbuffer(const PathImages& img, size_t pix, float depth, const SurfaceInfo& s,
+                                              uint32_t category, vec3 albedo) {
+    img.depth[pix] = depth;
+    img.normal[2 * pix + 0] = acosf(s.normal.z);
+    img.normal[2 * pix + 1] = atan2f(s.normal.y, s.normal.x);
+    uint8_t* mat = img.material + 4 * pix;
+    mat[0] = unorm8((float)category / 255.0f);
+    mat[1] = 0;
+    mat[2] = 0;
+    mat[3] = 0;
+    uint8_t* alb = img.albedo + 4 * pix;
+    alb[0] = unorm8(albedo.x);
+    alb[1] = unorm8(albedo.y);
+    alb[2] = unorm8(albedo.z);
+    alb[3] = 255;
+}
+
+// indirectLighting (lighting.glsl:263-287) at bounce `i` of a path that came from `from` to
+// the surface at `pos`: the direction and throughput of the next ray, or false where the
+// path ends.
+__device__ __forceinline__ bool bounce_ray(const TraceConsts& c, const SurfaceInfo& s, vec3 from, vec3 pos, int i,
+                                           Rng& re, vec3& throughput, vec3& l) {
+    const vec3 v = normalize(from - pos);
+    float pdf;
+    const vec3 brdf = sample_brdf(s, re, v, l, pdf);
+    if (brdf == make_vec3(0.0f) || pdf < kEpsilon) return false;
+    float tc = dot(l, s.normal);
+    if (s.illumination_type == 7) tc = 1.0f;
+    vec3 path_tp = throughput * (brdf * tc) / pdf;
+    if ((uint32_t)i > c.min_depth) {
+        if (rng_float(re) < kMinTermination) return false;
+        path_tp /= 1.0f - kMinTermination;
+    }
+    throughput = path_tp;
+    return true;
+}
+
+// The finished path's pixel: clamp, then demodulated radiance or the progressive image.
+__device__ __forceinline__ void write_radiance(const TraceConsts& c, const PathImages& img, size_t pix, vec3 radiance,
+                                               vec3 albedo, bool at_infinity) {
+    const vec3 color = vclamp(radiance, 0.0f, kMaxRadiance);
+    if (c.output == PBRT_OUTPUT_DEMOD_ILLUMINATION_FLOAT) {
+        vec3 demod = color;
+        if (!at_infinity) demod = vmin(color / (albedo + make_vec3(kEpsilon)), 1e3f);
+        img.illum[pix] = make_float4(demod.x, demod.y, demod.z, 1.0f);
+    } else {
+        vec3 fc = color;
+        if (c.sample_number > 0) {
+            float4 prev = img.illum[pix];
+            float alpha = 1.0f / (float)(c.sample_number + 1);
+            vec3 pl = srgb_to_linear(make_vec3(prev.x, prev.y, prev.z));
+            fc = vmix(pl, fc, alpha);
+        }
+        fc = linear_to_srgb(fc);
+        fc = vclamp(fc, 0.0f, 1.0f);
+        img.illum[pix] = make_float4(fc.x, fc.y, fc.z, 1.0f);
+    }
+}
+
 // kStack: traversal stack entries per lane (kShortStackSize: five waves per SIMD)
 template <bool kCount, int kStack>
 __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(kStack <= kShortStackSize ? 5 : 4)))
-pt_megakernel(DeviceScene sc, TraceConsts c, float* depth_img,
-                                                              float* normal_img, uint8_t* material_img,
-                                                              uint8_t* albedo_img, float4* illum_img,
-                                                              unsigned long long* counters) {
+pt_megakernel(DeviceScene sc, TraceConsts c, PathImages img, unsigned long long* counters) {
     __shared__ int stack_mem[kStack * kTileThreads];
     const uint32_t lid = threadIdx.x;
     int* stack = stack_mem + lid;
@@ -83,21 +149,7 @@ pt_megakernel(DeviceScene sc, TraceConsts c, float* depth_img,
                                 shadow_rays);
     color += s.emissive_color;
     vec3 albedo = s.diffuse_color + s.specular_color;
-    if (c.write_gbuffer) {
-        depth_img[pix] = distance(hit_pos, cam_pos);
-        normal_img[2 * pix + 0] = acosf(s.normal.z);
-        normal_img[2 * pix + 1] = atan2f(s.normal.y, s.normal.x);
-        uint8_t* mat = material_img + 4 * pix;
-        mat[0] = unorm8((float)category / 255.0f);
-        mat[1] = 0;
-        mat[2] = 0;
-        mat[3] = 0;
-        uint8_t* alb = albedo_img + 4 * pix;
-        alb[0] = unorm8(albedo.x);
-        alb[1] = unorm8(albedo.y);
-        alb[2] = unorm8(albedo.z);
-        alb[3] = 255;
-    }
+    if (c.write_gbuffer) write_gbuffer(img, pix, distance(hit_pos, cam_pos), s, category, albedo);
     if (!is_miss(s)) {
         int trans_depth = 0;
         vec3 wpos = cam_pos;
@@ -106,9 +158,10 @@ pt_megakernel(DeviceScene sc, TraceConsts c, float* depth_img,
                 --i;
                 ++trans_depth;
             }
+            // as bounce_ray, whose single exit costs this kernel five more spilled registers
+            // (1920x1080 atrium frame 3646 -> 3674 us)
             vec3 v = normalize(wpos - hit_pos);
             wpos = hit_pos;
-            // indirectLighting (lighting.glsl:263-287)
             vec3 l;
             float pdf;
             vec3 brdf = sample_brdf(s, re, v, l, pdf);
@@ -129,23 +182,7 @@ pt_megakernel(DeviceScene sc, TraceConsts c, float* depth_img,
             if (is_miss(s)) break;
         }
     }
-    color = vclamp(color, 0.0f, kMaxRadiance);
-    if (c.output == PBRT_OUTPUT_DEMOD_ILLUMINATION_FLOAT) {
-        vec3 demod = color;
-        if (!isinf(hit_pos.x)) demod = vmin(color / (albedo + make_vec3(kEpsilon)), 1e3f);
-        illum_img[pix] = make_float4(demod.x, demod.y, demod.z, 1.0f);
-    } else {
-        vec3 fc = color;
-        if (c.sample_number > 0) {
-            float4 prev = illum_img[pix];
-            float alpha = 1.0f / (float)(c.sample_number + 1);
-            vec3 pl = srgb_to_linear(make_vec3(prev.x, prev.y, prev.z));
-            fc = vmix(pl, fc, alpha);
-        }
-        fc = linear_to_srgb(fc);
-        fc = vclamp(fc, 0.0f, 1.0f);
-        illum_img[pix] = make_float4(fc.x, fc.y, fc.z, 1.0f);
-    }
+    write_radiance(c, img, pix, color, albedo, isinf(hit_pos.x));
     if (kCount) {
         atomicAdd(&counters[0], (unsigned long long)rays);
         atomicAdd(&counters[1], (unsigned long long)shadow_rays);
@@ -155,15 +192,6 @@ pt_megakernel(DeviceScene sc, TraceConsts c, float* depth_img,
         atomicAdd(&counters[5], (unsigned long long)cnt_sh.tris);
     }
 }
-
-// The images a path writes.
-struct PathImages {
-    float* depth;
-    float* normal;
-    uint8_t* material;
-    uint8_t* albedo;
-    float4* illum;
-};
 
 // A path between two walks (pt_pairs): the ray to walk next, the shadow ray of its last
 // vertex and the radiance for either outcome of it.
@@ -230,21 +258,7 @@ __device__ __forceinline__ void path_vertex(const DeviceScene& sc, const TraceCo
     p.at_infinity = isinf(pos.x);
     if (p.primary) {
         p.albedo = s.diffuse_color + s.specular_color;
-        if (c.write_gbuffer) {
-            img.depth[pix] = distance(pos, p.o);
-            img.normal[2 * pix + 0] = acosf(s.normal.z);
-            img.normal[2 * pix + 1] = atan2f(s.normal.y, s.normal.x);
-            uint8_t* mat = img.material + 4 * pix;
-            mat[0] = unorm8((float)category / 255.0f);
-            mat[1] = 0;
-            mat[2] = 0;
-            mat[3] = 0;
-            uint8_t* alb = img.albedo + 4 * pix;
-            alb[0] = unorm8(p.albedo.x);
-            alb[1] = unorm8(p.albedo.y);
-            alb[2] = unorm8(p.albedo.z);
-            alb[3] = 255;
-        }
+        if (c.write_gbuffer) write_gbuffer(img, pix, distance(pos, p.o), s, category, p.albedo);
     } else {
         ++p.depth_i;
     }
@@ -255,50 +269,11 @@ __device__ __forceinline__ void path_vertex(const DeviceScene& sc, const TraceCo
             --p.depth_i;
             ++p.trans_depth;
         }
-        const vec3 v = normalize(p.o - pos);
         vec3 l;
-        float pdf;
-        const vec3 brdf = sample_brdf(s, p.re, v, l, pdf);
-        if (!(brdf == make_vec3(0.0f) || pdf < kEpsilon)) {
-            float tc = dot(l, s.normal);
-            if (s.illumination_type == 7) tc = 1.0f;
-            vec3 path_tp = p.throughput * (brdf * tc) / pdf;
-            p.next = true;
-            if ((uint32_t)p.depth_i > c.min_depth) {
-                if (rng_float(p.re) < kMinTermination)
-                    p.next = false;
-                else
-                    path_tp /= 1.0f - kMinTermination;
-            }
-            if (p.next) {
-                p.throughput = path_tp;
-                p.d = l;
-            }
-        }
+        p.next = bounce_ray(c, s, p.o, pos, p.depth_i, p.re, p.throughput, l);
+        if (p.next) p.d = l;
     }
     p.o = pos;
-}
-
-// The finished path's pixel: clamp, then demodulated radiance or the progressive image.
-__device__ __forceinline__ void path_write(const TraceConsts& c, const PathImages& img, size_t pix,
-                                           const PathState& p) {
-    const vec3 color = vclamp(p.lit, 0.0f, kMaxRadiance);
-    if (c.output == PBRT_OUTPUT_DEMOD_ILLUMINATION_FLOAT) {
-        vec3 demod = color;
-        if (!p.at_infinity) demod = vmin(color / (p.albedo + make_vec3(kEpsilon)), 1e3f);
-        img.illum[pix] = make_float4(demod.x, demod.y, demod.z, 1.0f);
-    } else {
-        vec3 fc = color;
-        if (c.sample_number > 0) {
-            float4 prev = img.illum[pix];
-            float alpha = 1.0f / (float)(c.sample_number + 1);
-            vec3 pl = srgb_to_linear(make_vec3(prev.x, prev.y, prev.z));
-            fc = vmix(pl, fc, alpha);
-        }
-        fc = linear_to_srgb(fc);
-        fc = vclamp(fc, 0.0f, 1.0f);
-        img.illum[pix] = make_float4(fc.x, fc.y, fc.z, 1.0f);
-    }
 }
 
 constexpr uint32_t kPairX = 8, kPairY = 4;  // pixels of a wave of pt_pairs
@@ -343,7 +318,7 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
             if (p.next) {
                 path_vertex(sc, c, img, pix, h, p);
             } else {
-                path_write(c, img, pix, p);
+                write_radiance(c, img, pix, p.lit, p.albedo, p.at_infinity);
                 p.shadow = false;
                 alive = false;
             }
@@ -376,10 +351,7 @@ __device__ __forceinline__ void persistent_pixel(uint32_t id, uint32_t w, uint32
 // the frame runs out instead of idling while the wave's longest path finishes.
 // The wave that finishes last sets work[0..1] back to zero for the next launch.
 template <bool kCount>
-__global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4))) pt_persistent(DeviceScene sc, TraceConsts c, float* depth_img,
-                                                              float* normal_img, uint8_t* material_img,
-                                                              uint8_t* albedo_img, float4* illum_img,
-                                                              unsigned long long* counters, uint32_t* work) {
+__global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4))) pt_persistent(DeviceScene sc, TraceConsts c, PathImages img, unsigned long long* counters, uint32_t* work) {
     __shared__ int stack_mem[kTraversalStackSize * kTileThreads];
     const uint32_t lane = threadIdx.x;
     int* stack = stack_mem + lane;
@@ -434,21 +406,7 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
             color += ne;
             color += s.emissive_color;
             albedo = s.diffuse_color + s.specular_color;
-            if (c.write_gbuffer) {
-                depth_img[pix] = distance(hit_pos, ro);
-                normal_img[2 * pix + 0] = acosf(s.normal.z);
-                normal_img[2 * pix + 1] = atan2f(s.normal.y, s.normal.x);
-                uint8_t* mat = material_img + 4 * (size_t)pix;
-                mat[0] = unorm8((float)category / 255.0f);
-                mat[1] = 0;
-                mat[2] = 0;
-                mat[3] = 0;
-                uint8_t* alb = albedo_img + 4 * (size_t)pix;
-                alb[0] = unorm8(albedo.x);
-                alb[1] = unorm8(albedo.y);
-                alb[2] = unorm8(albedo.z);
-                alb[3] = 255;
-            }
+            if (c.write_gbuffer) write_gbuffer(img, pix, distance(hit_pos, ro), s, category, albedo);
             primary = false;
             depth_i = 0;
             trans_depth = 0;
@@ -465,47 +423,15 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
                 --depth_i;
                 ++trans_depth;
             }
-            const vec3 v = normalize(ro - hit_pos);
             vec3 l;
-            float pdf;
-            const vec3 brdf = sample_brdf(s, re, v, l, pdf);
-            if (brdf == make_vec3(0.0f) || pdf < kEpsilon) {
-                finish = true;
-            } else {
-                float tc = dot(l, s.normal);
-                if (s.illumination_type == 7) tc = 1.0f;
-                vec3 path_tp = throughput * (brdf * tc) / pdf;
-                if ((uint32_t)depth_i > c.min_depth) {
-                    if (rng_float(re) < kMinTermination)
-                        finish = true;
-                    else
-                        path_tp /= 1.0f - kMinTermination;
-                }
-                if (!finish) {
-                    throughput = path_tp;
-                    ro = hit_pos;
-                    rd = l;
-                }
+            finish = !bounce_ray(c, s, ro, hit_pos, depth_i, re, throughput, l);
+            if (!finish) {
+                ro = hit_pos;
+                rd = l;
             }
         }
         if (finish) {
-            color = vclamp(color, 0.0f, kMaxRadiance);
-            if (c.output == PBRT_OUTPUT_DEMOD_ILLUMINATION_FLOAT) {
-                vec3 demod = color;
-                if (!isinf(hit_pos.x)) demod = vmin(color / (albedo + make_vec3(kEpsilon)), 1e3f);
-                illum_img[pix] = make_float4(demod.x, demod.y, demod.z, 1.0f);
-            } else {
-                vec3 fc = color;
-                if (c.sample_number > 0) {
-                    float4 prev = illum_img[pix];
-                    float alpha = 1.0f / (float)(c.sample_number + 1);
-                    vec3 pl = srgb_to_linear(make_vec3(prev.x, prev.y, prev.z));
-                    fc = vmix(pl, fc, alpha);
-                }
-                fc = linear_to_srgb(fc);
-                fc = vclamp(fc, 0.0f, 1.0f);
-                illum_img[pix] = make_float4(fc.x, fc.y, fc.z, 1.0f);
-            }
+            write_radiance(c, img, pix, color, albedo, isinf(hit_pos.x));
             alive = false;
         }
     }
@@ -638,7 +564,8 @@ extern "C" int32_t pbrt_trace(const pbrt_scene* scene, const pbrt_trace_params* 
         dim3 grid((p->width + kTileX - 1) / kTileX, (p->height + kTileY - 1) / kTileY);
         const dim3 pair_grid((p->width + kPairX - 1) / kPairX, (p->height + kPairY - 1) / kPairY);
         hipStream_t st = (hipStream_t)stream;
-        float4* illum = reinterpret_cast<float4*>(img->illumination);
+        const PathImages images{img->depth, img->normal, img->material, img->albedo,
+                                reinterpret_cast<float4*>(img->illumination)};
         TraceTiming* tm = scene_timing(scene);
         if (p->tracer == PBRT_TRACER_WAVEFRONT) {
             wavefront_trace(sc, scene_bvh_depth(scene), c, *img, counters, tm, p->block_threads, p->queue_paths, st);
@@ -647,12 +574,11 @@ extern "C" int32_t pbrt_trace(const pbrt_scene* scene, const pbrt_trace_params* 
             // time is its longest path's, which pt_pairs shortens, also when other streams
             // trace at the same time.  Larger frames gain alone while their waves are all
             // resident (atrium 480x270 545 -> 447 us), but on four streams at once the
-            // chip is full and the pairs' idle lanes cost more than they save.  us per
-            // frame with four streams, megakernel and pairs: atrium 200x150 0.74 of the
-            // megakernel's time, 320x180 0.93, 256x256 1.05, 320x240 1.11, 480x270 1.41;
-            // city 256x256 0.81, 480x270 1.24; Cornell box 256x256 0.95.  Counted traces
-            // keep the tracer they name, whose traversal counts they report.
-            const PathImages images{img->depth, img->normal, img->material, img->albedo, illum};
+            // chip is full and the pairs' idle lanes cost more than they save.  Of the
+            // megakernel's time with four streams: atrium 200x150 0.74, 320x180 0.93,
+            // 256x256 1.05, 320x240 1.11, 480x270 1.41; city 256x256 0.81, 480x270 1.24;
+            // Cornell box 256x256 0.95.  Counted traces keep the tracer they name, whose
+            // traversal counts they report.
             if (tm) tm->frame_begin(st);
             hipLaunchKernelGGL(pt_pairs, pair_grid, dim3(kTileThreads), 0, st, sc, c, images);
             if (tm) tm->mark(kTimeMegakernel, st);
@@ -664,11 +590,11 @@ extern "C" int32_t pbrt_trace(const pbrt_scene* scene, const pbrt_trace_params* 
             uint32_t* work = scene_work_counter(scene);
             if (tm) tm->frame_begin(st);
             if (counters)
-                hipLaunchKernelGGL(pt_persistent<true>, dim3(waves), dim3(kTileThreads), 0, st, sc, c, img->depth,
-                                   img->normal, img->material, img->albedo, illum, counters, work);
+                hipLaunchKernelGGL(pt_persistent<true>, dim3(waves), dim3(kTileThreads), 0, st, sc, c, images,
+                                   counters, work);
             else
-                hipLaunchKernelGGL(pt_persistent<false>, dim3(waves), dim3(kTileThreads), 0, st, sc, c, img->depth,
-                                   img->normal, img->material, img->albedo, illum, counters, work);
+                hipLaunchKernelGGL(pt_persistent<false>, dim3(waves), dim3(kTileThreads), 0, st, sc, c, images,
+                                   counters, work);
             if (tm) tm->mark(kTimeMegakernel, st);
         } else {
             if (tm) tm->frame_begin(st);
@@ -678,8 +604,7 @@ extern "C" int32_t pbrt_trace(const pbrt_scene* scene, const pbrt_trace_params* 
                                                   : pt_megakernel<true, kTraversalStackSize>)
                                    : (short_stack ? pt_megakernel<false, kShortStackSize>
                                                   : pt_megakernel<false, kTraversalStackSize>);
-            hipLaunchKernelGGL(kernel, grid, dim3(kTileThreads), 0, st, sc, c, img->depth, img->normal,
-                               img->material, img->albedo, illum, counters);
+            hipLaunchKernelGGL(kernel, grid, dim3(kTileThreads), 0, st, sc, c, images, counters);
             if (tm) tm->mark(kTimeMegakernel, st);
         }
         PBRT_HIP(hipGetLastError());
