@@ -396,8 +396,9 @@ enum pbrt_bmfr_fit {
      * sky blocks cond(A^T A) reaches 1e10 and the fit error grows to ~1e-1. */
     PBRT_BMFR_FIT_GRAM_F16 = 1,
     /* as PBRT_BMFR_FIT_GRAM_F16 but the Gram matrix is accumulated by FP64 MFMA
-     * (v_mfma_f64_4x4x4f64) from the fp32 projected columns; fitted values
-     * stay within ~1e-5 of the FP64 least-squares solution on every block. */
+     * (v_mfma_f64_4x4x4f64) from the raw fp32 columns, the projection following in FP64; fitted
+     * values stay within 1e-5 (32-pixel blocks), 4e-5 (16) and 2e-4 (8) of the FP64
+     * least-squares solution. */
     PBRT_BMFR_FIT_GRAM_F64 = 2
 };
 

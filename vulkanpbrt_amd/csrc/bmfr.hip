@@ -236,7 +236,7 @@ __global__ void __launch_bounds__(1024) k_bmfr_pre(BmfrGeom g, pbrt_bmfr_images 
 // (2 u v) / |u|^2 divides by one number per column, so it is a product with its
 // reciprocal and one correction by the exact residual (the correctly rounded quotient,
 // in three operations), except where the divisor's magnitude could make the residual
-// inexact.  The back-substitution runs in the first wave: lane i holds row i, and each
+// inexact.  (Numerators below 2^-110 may end one place of the subnormal range off.)  The back-substitution runs in the first wave: lane i holds row i, and each
 // solved weight is broadcast to the rows above it.  A 16-pixel block is one wave of four
 // rows per lane (no barrier; four waves of one row each took 226 us where this takes
 // 138).  Whole passes (pre, fit, post), 32-pixel blocks: 1279x719 246 -> 69 us, 1920x1080
@@ -715,7 +715,8 @@ __device__ __forceinline__ void bmfr_fit_raw_gram_block(const BmfrGeom& g, const
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // the block size follows from the rows, so a pixel's place in its block is a shift and
     // a mask (by the run-time size they were an integer division and a remainder per pixel;
-    // with the bilinear fetch's, 1920x1080 BMFR 57.5 -> 54.1 us)
+    // with the bilinear fetch's, 1920x1080 BMFR 57.5 -> 54.1 us, called again and again on
+    // one frame; some 5 us more with another frame every call)
     constexpr int bs = kRows == 1024 ? 32 : kRows == 256 ? 16 : 8;
     const int basex = bx * bs, basey = by * bs;
 
@@ -800,7 +801,7 @@ __device__ __forceinline__ void bmfr_fit_raw_gram_block(const BmfrGeom& g, const
     //    take the nine pairs R needs (the upper triangle without b's own) where a
     //    16x16 product forms all sixteen: 9 x 16 cycles per 16 rows against 4 x 64.
     //    Both operands hold the same values (lane l: row l / 4, column l % 4 of a group).
-    //    1920x1080, whole BMFR: 63.5 -> 57.5 us.
+    //    1920x1080, whole BMFR on one frame: 63.5 -> 57.5 us.
     {
         //    Four waves with one chunk of a 16-pixel block each exchange the staged rows and
         //    divide the nine pairs instead, so that each sum runs over the block's rows in

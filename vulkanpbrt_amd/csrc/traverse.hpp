@@ -52,8 +52,8 @@ __device__ __forceinline__ int wrap_repeat(int i, int n) {
 }
 
 // The texels x0 and x1 of a row; one load where they are neighbours (all but the wrap, and
-// rows of one texel): half the fetches of scattered lines.  1920x1080 megakernel, 4 bounces:
-// atrium 3613 -> 3573 us, city 1942 -> 1933.
+// rows of one texel): half the fetches of scattered lines.  1920x1080 megakernel alone, 4
+// bounces, both builds in turn: atrium 3613 -> 3575 us, city 1945 -> 1940 (runs differ by 0.3 %).
 __device__ __forceinline__ uint2 load_texels(const uint32_t* row, int x0, int x1) {
     uint2 t;
     if (x1 > x0) {
