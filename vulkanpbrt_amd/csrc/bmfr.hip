@@ -543,7 +543,7 @@ __device__ __forceinline__ void bmfr_fit_gram_f16_block(const BmfrGeom& g, const
                                z * z, a[s][10], a[s][11], a[s][12]};
 #pragma unroll
         for (int c = 0; c < kAlphaSize; ++c) {
-            float v = h2f(f2h(f[c]));
+            float v = h2f(f2h(as_float(f[c])));
             if (c < kFeatures) v = __fadd_rn(v, noise[c][s]);
             a[s][c] = v;
         }
@@ -1126,12 +1126,16 @@ static void launch_gram_rows(int bs, dim3 grid, hipStream_t st, const BmfrGeom& 
 template <bool kF64>
 static void launch_gram_threads(int bs, uint32_t threads, dim3 grid, hipStream_t st, const BmfrGeom& g,
                                 const pbrt_bmfr_images& im) {
-    if (kF64 && threads == 64) {
-        if (bs == 16)
-            hipLaunchKernelGGL((k_bmfr_fit_gram<256, kF64, 64>), grid, dim3(64), 0, st, g, im);
-        else
-            hipLaunchKernelGGL((k_bmfr_fit_gram<64, kF64, 64>), grid, dim3(64), 0, st, g, im);
-    } else if (threads == 1024)
+    if constexpr (kF64) {
+        if (threads == 64) {
+            if (bs == 16)
+                hipLaunchKernelGGL((k_bmfr_fit_gram<256, kF64, 64>), grid, dim3(64), 0, st, g, im);
+            else
+                hipLaunchKernelGGL((k_bmfr_fit_gram<64, kF64, 64>), grid, dim3(64), 0, st, g, im);
+            return;
+        }
+    }
+    if (threads == 1024)
         launch_gram_rows<kF64, 1024>(bs, grid, st, g, im);
     else if (threads == 512)
         launch_gram_rows<kF64, 512>(bs, grid, st, g, im);
